@@ -579,8 +579,8 @@ def md_step(integrator, U, P, step_size, driver):
 def md_trajectory(U, P, driver, *, diagnostics=True, fused=False):
     """One deterministic MD trajectory (no momentum refresh, no accept/reject).
 
-    Built-in integrators run in the library's native driver (one C call per trajectory;
-    ``fused=True`` merges adjacent half steps into single force + kick + exp kernels).
+    Built-in integrators run in the library's native driver (one C call per trajectory, adjacent
+    half steps merged into single force + kick + exp kernels; ``fused`` selects nothing any more).
     Custom integrators (callables) are stepped from here."""
     _check_same(U, P)
     integ = driver.integrator

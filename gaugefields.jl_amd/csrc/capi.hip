@@ -881,7 +881,6 @@ int gf_md_update(gf_ctx* c, double coeff, double eps_p, double eps_u) {
 int gf_md_trajectory(gf_ctx* c, double coeff, int integrator, double lambda, int steps, double tau, double* H) {
     CTXCHK(c);
     const int kind = integrator & 0xff;
-    const bool fused = (integrator & GF_FUSED) != 0;
     if (steps <= 0) return fail(c, GF_EINVAL, "steps must be positive; got %d", steps);
     if (!std::isfinite(tau)) return fail(c, GF_EINVAL, "trajectory_length must be finite; got %g", tau);
     if (tau == 0.0) return fail(c, GF_EINVAL, "trajectory_length must not be zero");
@@ -890,25 +889,13 @@ int gf_md_trajectory(gf_ctx* c, double coeff, int integrator, double lambda, int
     double h0 = 0.0;
     if (H) TRY(hamiltonian(c, coeff, &h0));
     const double e = tau / steps;
-    if (!fused) {
-        for (int k = 0; k < steps; k++) {
-            if (kind == GF_QPQ) {
-                TRY(expupd(c, e / 2));
-                TRY(kick(c, coeff, e));
-                TRY(expupd(c, e / 2));
-            } else if (kind == GF_PQP) {
-                TRY(kick(c, coeff, e / 2));
-                TRY(expupd(c, e));
-                TRY(kick(c, coeff, e / 2));
-            } else {
-                TRY(kick(c, coeff, lambda * e));
-                TRY(expupd(c, 0.5 * e));
-                TRY(kick(c, coeff, (1.0 - 2.0 * lambda) * e));
-                TRY(expupd(c, 0.5 * e));
-                TRY(kick(c, coeff, lambda * e));
-            }
-        }
-    } else if (kind == GF_QPQ) {  // Q(e/2) [P(e) Q(e)]^(n-1) P(e) Q(e/2)
+    // Neighbouring sub-steps of the same kind are one: the links do not change between the closing
+    // kick of one step and the opening kick of the next, so their forces are the same and one kick of
+    // the summed size does for both (2MN: two force evaluations a step instead of three, PQP: one
+    // instead of two), and the link updates exp(e/2 P) exp(e/2 P) of QPQ are exp(e P).  Every kick that
+    // a link update follows runs as one kernel with it (gf_md_update).  16^4 FP64, 15 2MN steps: 1.70 ->
+    // 1.00 ms; 24^4 with three stout levels, 10 2MN steps: 56 -> 40 ms.
+    if (kind == GF_QPQ) {  // Q(e/2) [P(e) Q(e)]^(n-1) P(e) Q(e/2)
         TRY(expupd(c, e / 2));
         for (int k = 0; k < steps - 1; k++) TRY(kick_exp(c, coeff, e, e));
         TRY(kick_exp(c, coeff, e, e / 2));

@@ -670,8 +670,8 @@ _integrator_code(::PQP) = (GF_PQP, OMELYAN_LAMBDA)
 _integrator_code(i::OmelyanPQP) = (GF_OMELYAN2MN, i.λ)
 
 """md_trajectory!(U, P, driver; diagnostics=true, fused=false) (molecular_dynamics.jl:712-730).
-QPQ, PQP and OmelyanPQP of a single action run as one library call per trajectory (`fused=true` merges adjacent
-half steps into single force + kick + exp kernels); other integrators step through md_step!."""
+QPQ, PQP and OmelyanPQP of a single action run as one library call per trajectory (adjacent half
+steps merged into single force + kick + exp kernels); other integrators step through md_step!."""
 function md_trajectory!(U::HIPLinks, P::HIPMomenta, driver::MDDriver; diagnostics::Bool=true,
                         fused::Bool=false)
     c = _same(U, P)

@@ -145,8 +145,9 @@ int gf_exp_update(gf_ctx *ctx, double eps);
  * (force + kick + exp; the new links go to a second buffer that becomes current) */
 int gf_md_update(gf_ctx *ctx, double coeff, double eps_p, double eps_u);
 /* md_trajectory! (molecular_dynamics.jl:712-730) with md_step! QPQ/PQP (:604-616) or the
- * Omelyan 2MN step of docs/src/howtoimplement.md:94-112 (integrator | GF_FUSED merges
- * adjacent half steps and uses gf_md_update).  Force: plain Wilson action, or the
+ * Omelyan 2MN step of docs/src/howtoimplement.md:94-112; adjacent half steps of the same kind are
+ * merged and kicks run with the link update that follows them (gf_md_update), with or without the
+ * GF_FUSED flag, which is accepted for callers that set it.  Force: plain Wilson action, or the
  * stout-smeared one when gf_stout_config set nlev > 0.  H[3] = {H0, H1, H1 - H0}. */
 int gf_md_trajectory(gf_ctx *ctx, double coeff, int integrator, double lambda, int steps, double tau,
                      double *H);
