@@ -361,13 +361,6 @@ int state64_step(gf_ctx* c, int mode, double eps_u) {
                                   c->stream));
     return GF_OK;
 }
-// the force of the links rounded to float, FP32 throughout, into F
-int force_f32(gf_ctx* c, double coeff) {
-    if (c->nlev > 0) return stout_force_impl(c, coeff, FORCE_STORE, 0.0);
-    HIPCHK(c, launch_force<float>(FORCE_STORE, c->geo, (const float*)c->U, (float*)c->F, nullptr, coeff, 0.0, 0.0,
-                                  c->stream));
-    return GF_OK;
-}
 int not_state64(gf_ctx* c, const char* what) {
     return fail(c, GF_ESTATE,
                 "%s is not available in the FP32-force form (FP64 links and momenta, forces in FP32); use a GF_F64 or "

@@ -16,8 +16,32 @@ template <typename T>
 inline constexpr bool kFloatBulk = std::is_same<T, float>::value;
 
 inline int grid_for(int V, int block = kBlock) { return (V + block - 1) / block; }
+// gridDim.y of the streaming link kernels: threads per site (4: one per link) on lattices of so few
+// workgroups of sites that CUs stay empty (4^4: 5.2 -> 3.5 us, 12^3x8: 7.6 -> 3.7; 16^4: 12.4 -> 12.9, hence
+// the limit between)
+inline int link_dirs(int V) { return grid_for(V) <= 128 ? 4 : 1; }
 // grid of the (site, direction) kernels: one 256-thread workgroup per 64 sites
 inline int grid_sites_mu(int V) { return (V + 63) / 64; }
+
+// f(std::true_type) where every 64-site group is whole x-rows (rows_whole), f(std::false_type) otherwise
+template <typename F>
+inline void by_rows(const Geo& g, F&& f) {
+    if (rows_whole(g))
+        f(std::true_type{});
+    else
+        f(std::false_type{});
+}
+// f(std::integral_constant<int, ST>) of the lattice's stencil form for fields of T
+template <typename T, typename F>
+inline void by_form(const Geo& g, F&& f) {
+    const int form = stencil_form<T>(g);
+    if (form == ST_WIDE)
+        f(std::integral_constant<int, ST_WIDE>{});
+    else if (form == ST_ROWS)
+        f(std::integral_constant<int, ST_ROWS>{});
+    else
+        f(std::integral_constant<int, ST_CUT>{});
+}
 
 // force kernel modes
 enum ForceMode { FORCE_STORE = 0, FORCE_KICK = 1, FORCE_KICK_EXP = 2, FORCE_KICK_S64 = 3, FORCE_KICK_EXP_S64 = 4 };

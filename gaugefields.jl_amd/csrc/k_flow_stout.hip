@@ -10,29 +10,15 @@ namespace gf {
 //   Wout_mu = exp(A_mu) W_mu               (exp_aF_U!, AbstractGaugefields.jl:2810-2841)
 // stages (alpha, beta) = (-eps/4, 0), (-8eps/9, -17/9), (-3eps/4, -1)
 // ---------------------------------------------------------------------------
-// ST: stencil form as in k_force (stencil_form).  At most 168 VGPRs: three waves per SIMD.
+// ST: form of the stencil (stencil_form).  At most 168 VGPRs: three waves per SIMD.
 template <typename T, int ST>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_flow_stage(Geo g, const T* __restrict__ W, T* __restrict__ Wout,
-                                                       T* __restrict__ A, double alpha, double beta) {
-    __shared__ T2<T> ol[ST ? 4 : 1][6][64];
-    __shared__ T2<T> tp[ST ? 7 : 1][4][64];
-    const SiteMu sm = site_mu_index(g);
-    const int mu = sm.mu;
-    int s;
-    if (!stencil_site<(ST > 0)>(g, sm, s)) return;
-    int x[4];
-    decode(g, s, x);
-    const unsigned V = g.V;
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_flow_stage(
+    Geo g, const T* __restrict__ W, T* __restrict__ Wout, T* __restrict__ A, double alpha, double beta) {
+    int s, mu;
     R6<T> own;
     T c[8];
-    if constexpr (ST == ST_XROW) {
-        ta_force_xrow(g, W, V, s, x, mu, own, ol, tp, c);
-    } else if constexpr (ST == ST_SHARED) {
-        ta_force_shared(g, W, V, s, x, mu, own, ol, tp, c);
-    } else {
-        const M3<T> sig = staple_sigma_own(g, W, V, s, x, mu, own);
-        ta_coeffs(mul(full_of(own), sig), c);
-    }
+    if (!ta_force<ST, T>(g, W, s, mu, own, c)) return;
+    const unsigned V = g.V;
     const M3<T> w = full_of(own);
     if (beta != T(0)) {
         T a[8];
@@ -53,19 +39,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
 //   C_mu = rho V_mu = rho Sigma_mu^dag,  Q_mu = TA(C_mu U_mu^dag),  Uout_mu = exp(Q_mu) U_mu
 // STORE keeps C_mu for the backward pass.
 // ---------------------------------------------------------------------------
-template <typename T, bool STORE, bool SHARED>
+template <typename T, bool STORE, bool ROWS>
 __global__ __launch_bounds__(kBlock) void k_stout_forward(Geo g, const T* __restrict__ Uin, T* __restrict__ Uout,
                                                           T* __restrict__ Cst, double rho) {
-    __shared__ T2<T> xs[SHARED ? 6 : 1][6][64];
+    __shared__ T2<T> xs[6][6][64];
     const SiteMu sm = site_mu_index(g);
     const int mu = sm.mu;
-    int s;
-    if (!stencil_site<SHARED>(g, sm, s)) return;
+    const int s = stencil_site<ROWS>(g, sm);
     int x[4];
     decode(g, s, x);
     const unsigned V = g.V;
     R6<T> own;
-    const M3<T> sig = staple_sum_own<T, SHARED>(g, Uin, V, s, x, mu, own, xs);
+    const M3<T> sig = staple_sigma_shared(g, Uin, V, s, x, mu, own, xs);
+    if (!in_lattice<ROWS>(g, sm)) return;
     const M3<T> u = full_of(own);
     if constexpr (std::is_same<T, float>::value) {
         // C = rho Sigma^dag rounded once (the backward pass reads this C), Q and exp(Q) U in double
@@ -115,11 +101,11 @@ __device__ __forceinline__ M3<T> staged_m3(MStage<T> st, int mu, int lane) {
     }
     return m;
 }
-template <typename T, bool STORED, bool SHARED>
+template <typename T, bool STORED, bool ROWS>
 __global__ __launch_bounds__(kBlock) void k_stout_back_local(Geo g, const T* __restrict__ Uin,
                                                              const T* __restrict__ Cst, const T* __restrict__ Dout,
                                                              T* __restrict__ Din, T* __restrict__ Lc, double rho) {
-    __shared__ T2<T> xs[SHARED ? 6 : 1][6][64];
+    __shared__ T2<T> xs[STORED ? 1 : 6][6][64];
     // Dout_mu and a stored C_mu are used before and after exp_dexp: kept in LDS in between (the
     // second read from memory missed L2 for a third of the kernel's HBM reads)
     __shared__ T2<T> dst[4][9][64];
@@ -127,8 +113,7 @@ __global__ __launch_bounds__(kBlock) void k_stout_back_local(Geo g, const T* __r
     const SiteMu sm = site_mu_index(g);
     const int mu = sm.mu;
     const int lane = (int)(threadIdx.x & 63u);
-    int s;
-    if (!stencil_site<SHARED>(g, sm, s)) return;
+    const int s = stencil_site<ROWS>(g, sm);
     const unsigned V = g.V;
     M3<T> C;  // recomputed C; a stored C is staged in LDS instead of kept live
     R6<T> own;
@@ -137,8 +122,9 @@ __global__ __launch_bounds__(kBlock) void k_stout_back_local(Geo g, const T* __r
     } else {  // the same staple evaluation (and rounding) as the forward kernel
         int x[4];
         decode(g, s, x);
-        C = round_link<T>(scal(rho, dag(to_f64(staple_sum_own<T, SHARED>(g, Uin, V, s, x, mu, own, xs)))));
+        C = round_link<T>(scal(rho, dag(to_f64(staple_sigma_shared(g, Uin, V, s, x, mu, own, xs)))));
     }
+    if (!in_lattice<ROWS>(g, sm)) return;
     M3<T> E, L;
     {
         const M3<T> u = full_of(own);
@@ -228,14 +214,7 @@ __device__ __forceinline__ void acc_hd(M3<T>& c, const Herm<T>& h, const M3<T>& 
 }
 
 template <typename T>
-__device__ __forceinline__ R6<T> lds_r6(XShare<T> ul, int d, int l) {
-    R6<T> r;
-#pragma unroll
-    for (int e = 0; e < 6; e++) r.v[e] = ul[d][e][l];
-    return r;
-}
-template <typename T>
-__device__ __forceinline__ void lds_c8(PairShare<T> hl, int d, int l, T c[8]) {
+__device__ __forceinline__ void lds_c8(XCoefs<T> hl, int d, int l, T c[8]) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const T2<T> v = hl[d][e][l];
@@ -243,34 +222,32 @@ __device__ __forceinline__ void lds_c8(PairShare<T> hl, int d, int l, T c[8]) {
         c[2 * e + 1] = v.y;
     }
 }
-// Plane b of K6b added into acc.  SH: U_b(y) and Lam_b(y) from the workgroup's LDS copies
-// (ul, hl) instead of memory; A0 (a = 0) and B0 (b = 0): the x-neighbour links and Lam at
-// y + 1 (lane lxp) and y - 1 (lane lxm) from LDS as well (workgroups of whole x-rows).
-template <typename T, bool SH, bool A0, bool B0>
+// Plane b of K6b added into acc.  U_b(y) and Lam_b(y) come from the workgroup's LDS copies (ul, hl);
+// A0 (a = 0) and B0 (b = 0): the x-neighbour links and Lam at y + 1 and y - 1 (xr) as well.
+template <typename T, bool A0, bool B0>
 __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U, const T* __restrict__ Lc, unsigned V,
-                                           int y, const int x[4], int a, int b, int ypa, M3<T>& acc, XShare<T> ul,
-                                           PairShare<T> hl, int lane, int lxm, int lxp) {
+                                           int y, const int x[4], int a, int b, int ypa, M3<T>& acc, XLinks<T> ul,
+                                           XCoefs<T> hl, int lane, const XRow& xr) {
     const int ypb0 = y + dlt(g, x, b, 1);
     const int dmb = dlt(g, x, b, -1);
     const int ymb0 = y + dmb, ypamb0 = ypa + dmb;
     // each group loads its links through its own opaque index copies, so the compiler
     // issues them group by group instead of hoisting all of them
     {  // upper: i X H_a(y+b) U_b(y)^dag + i [S H_b(y) - H_b(y+a) S],  S = X U_b(y)^dag
-        int y0 = y, y1 = ypa, ypb = ypb0;
-        asm volatile("" : "+v"(y0), "+v"(y1), "+v"(ypb));
-        const R6<T> uby = A0 ? lds_r6<T>(ul, b, lxp) : ldr(U, V, b, y1);                // U_b(y+a)
-        const M3<T> X = su3_mul_nd(uby, full_of(B0 ? lds_r6<T>(ul, a, lxp) : ldr(U, V, a, ypb)));  // U_a(y+b)
+        int y1 = ypa, ypb = ypb0;
+        asm volatile("" : "+v"(y1), "+v"(ypb));
+        const R6<T> uby = A0 ? shared_link<T>(ul, b, xr.p) : ldr(U, V, b, y1);                // U_b(y+a)
+        const M3<T> X = su3_mul_nd(uby, full_of(B0 ? shared_link<T>(ul, a, xr.p) : ldr(U, V, a, ypb)));  // U_a(y+b)
         T c[8];
-        if (B0) lds_c8<T>(hl, a, lxp, c);  // Lam_a(y+b)
+        if (B0) lds_c8<T>(hl, a, xr.p, c);  // Lam_a(y+b)
         else ldp(Lc, V, a, ypb, c);
         const M3<T> XH = times_i(mul_mh(X, herm_of_coeffs(c)));
-        const M3<T> ub = full_of(SH ? lds_r6<T>(ul, b, lane) : ldr(U, V, b, y0));        // U_b(y)
+        const M3<T> ub = full_of(shared_link<T>(ul, b, lane));        // U_b(y)
         acc_mul_nd(acc, XH, ub);
         const M3<T> S = su3_mul_nd(rows_of(X), ub);
-        if (SH) lds_c8<T>(hl, b, lane, c);  // Lam_b(y)
-        else ldp(Lc, V, b, y0, c);
+        lds_c8<T>(hl, b, lane, c);  // Lam_b(y)
         acc_i_mh<T, 1>(acc, S, herm_of_coeffs(c));
-        if (A0) lds_c8<T>(hl, b, lxp, c);  // Lam_b(y+a)
+        if (A0) lds_c8<T>(hl, b, xr.p, c);  // Lam_b(y+a)
         else ldp(Lc, V, b, y1, c);
         acc_i_hm<T, -1>(acc, herm_of_coeffs(c), S);
     }
@@ -278,11 +255,11 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
        // H_d = H_a(y-b) - H_b(y-b)
         int ymb = ymb0, ypamb = ypamb0;
         asm volatile("" : "+v"(ymb), "+v"(ypamb));
-        const M3<T> ua = full_of(B0 ? lds_r6<T>(ul, a, lxm) : ldr(U, V, a, ymb));  // U_a(y-b)
+        const M3<T> ua = full_of(B0 ? shared_link<T>(ul, a, xr.m) : ldr(U, V, a, ymb));  // U_a(y-b)
         T ca[8], cb[8];
         if (B0) {
-            lds_c8<T>(hl, a, lxm, ca);
-            lds_c8<T>(hl, 0, lxm, cb);
+            lds_c8<T>(hl, a, xr.m, ca);
+            lds_c8<T>(hl, 0, xr.m, cb);
         } else {
             ldp(Lc, V, a, ymb, ca);
             ldp(Lc, V, b, ymb, cb);
@@ -291,56 +268,52 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
         for (int k = 0; k < 8; k++) ca[k] -= cb[k];
         M3<T> A = mul_dh(ua, herm_of_coeffs(ca));
         acc_hd(A, herm_at(Lc, V, b, ypamb), ua);
-        const M3<T> ubm = full_of(B0 ? lds_r6<T>(ul, 0, lxm) : ldr(U, V, b, ymb));  // U_b(y-b)
+        const M3<T> ubm = full_of(B0 ? shared_link<T>(ul, 0, xr.m) : ldr(U, V, b, ymb));  // U_b(y-b)
         acc_mul_dn(acc, ldu(U, V, b, ypamb), times_i(mul(A, ubm)));
     }
 }
 
-// The staple part of K6b for output direction a at site y (all planes b != a), with the
-// stencil form ST: ST_OWN every link and Lam from memory; ST_SHARED U(y) and Lam(y) of the
-// workgroup's sites through LDS (per wave 6 link and 3 Lam loads fewer); ST_XROW also the
-// x-neighbours (6 + 3 more).  The LDS forms fill ul/hl and pass one workgroup barrier.
-template <typename T, int ST>
+// The staple part of K6b for output direction a at site y (all planes b != a).  U(y) and Lam(y) of
+// the workgroup's sites and of their x-neighbours go through LDS (per wave 12 link and 6 Lam loads
+// fewer than from memory); one workgroup barrier after filling ul/hl.
+template <bool ROWS, typename T>
 __device__ __forceinline__ M3<T> back_stencil_acc(const Geo& g, const T* __restrict__ U, const T* __restrict__ Lc,
-                                                  int y, const int x[4], int a, int lane, XShare<T> ul,
-                                                  PairShare<T> hl) {
+                                                  int y, const int x[4], int a, int lane, XLinks<T> ul,
+                                                  XCoefs<T> hl) {
     const unsigned V = g.V;
-    if constexpr (ST > 0) {
-        const R6<T> u = ldr(U, V, a, (unsigned)y);
+    const XRow xr = xrow_of<ROWS>(g, y, x[0], lane);
+    {
         T c[8];
+        const R6<T> u = ldr(U, V, a, (unsigned)y);
         ldp(Lc, V, a, (unsigned)y, c);
+        share_links<ROWS, T>(ul, U, V, a, lane, xr, u);
+        auto put = [&](int l) {
 #pragma unroll
-        for (int e = 0; e < 6; e++) ul[a][e][lane] = u.v[e];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            T2<T> v;
-            v.x = c[2 * e];
-            v.y = c[2 * e + 1];
-            hl[a][e][lane] = v;
+            for (int e = 0; e < 4; e++) {
+                T2<T> v;
+                v.x = c[2 * e];
+                v.y = c[2 * e + 1];
+                hl[a][e][l] = v;
+            }
+        };
+        put(lane);
+        if (xr.halo >= 0) {
+            ldp(Lc, V, a, (unsigned)xr.halo, c);
+            put(64 + lane);
         }
         __syncthreads();
     }
-    const int nxm1 = g.n[0] - 1;
-    const int lxm = xlane(lane, nxm1, -1), lxp = xlane(lane, nxm1, 1);
     M3<T> acc = zero3<T>();
     const int ypa = y + dlt(g, x, a, 1);
-    if constexpr (ST == ST_XROW) {
-        if (a == 0) {
+    if (a == 0) {
 #pragma unroll 1
-            for (int b = 1; b < 4; b++) back_plane<T, true, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, lxm, lxp);
-        } else {
-            back_plane<T, true, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, lxm, lxp);
-#pragma unroll 1
-            for (int b = 1; b < 4; b++) {
-                if (b == a) continue;
-                back_plane<T, true, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, lxm, lxp);
-            }
-        }
+        for (int b = 1; b < 4; b++) back_plane<T, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
     } else {
+        back_plane<T, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, xr);
 #pragma unroll 1
-        for (int b = 0; b < 4; b++) {
+        for (int b = 1; b < 4; b++) {
             if (b == a) continue;
-            back_plane<T, ST == ST_SHARED, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, lxm, lxp);
+            back_plane<T, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
         }
     }
     return acc;
@@ -366,31 +339,27 @@ __device__ __forceinline__ M3<T> back_stencil_din(const T* __restrict__ Din, uns
 // to a buffer other than U, which the other threads still read.  OUT = FORCE_KICK_S64 /
 // FORCE_KICK_EXP_S64 (FP32 only): FP is the FP64 momenta, kicked by the force as rounded to float;
 // U64 the FP64 links, U64_a(y) <- exp(eps_u FP) U64_a(y) in place, and Unew its float rounding.
-template <typename T, int ST, int OUT>
+template <typename T, int OUT, bool ROWS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil(
     Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho,
     T* __restrict__ FP, double eps, T* __restrict__ Unew, double eps_u, double* __restrict__ U64) {
-    __shared__ T2<T> ul[ST ? 4 : 1][6][64];
-    __shared__ T2<T> hl[ST ? 4 : 1][4][64];
+    __shared__ T2<T> ul[4][6][kXW];
+    __shared__ T2<T> hl[4][4][kXW];
     const SiteMu sm = site_mu_index(g);
     const int a = sm.mu;
-    int y;
-    if (!stencil_site<(ST > 0)>(g, sm, y)) return;
+    const int y = stencil_site<ROWS>(g, sm);
     int x[4];
     decode(g, y, x);
     const unsigned V = g.V;
     const int lane = (int)(threadIdx.x & 63u);
-    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, back_stencil_acc<T, ST>(g, U, Lc, y, x, a, lane, ul, hl));
+    const M3<T> acc = back_stencil_acc<ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl);
+    if (!in_lattice<ROWS>(g, sm)) return;
+    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, acc);
     if constexpr (OUT < 0) {
         stm<T, GF_ST_NT>(Din, V, a, y, dn);
     } else {  // the force from the thin-link derivative
         constexpr double fac = -1.0 / 3.0;
-        R6<T> ur;
-        if constexpr (ST > 0)
-            ur = lds_r6<T>(ul, a, lane);
-        else
-            ur = ldr(U, V, a, (unsigned)y);
-        const M3<T> ua = full_of(ur);
+        const M3<T> ua = full_of(shared_link<T>(ul, a, lane));
         T c[8];
         ta_coeffs(mul(ua, dn), c);
         if constexpr (OUT == FORCE_STORE) {
@@ -452,33 +421,32 @@ __device__ __forceinline__ void back_local_stored(const T* __restrict__ Uin, con
 template <typename T>
 constexpr int kChainLds = (int)(2 * 4 * 9 * 64 * sizeof(T2<T>));  // dst + cst; >= ul + hl
 // FP32: three waves per SIMD (at most 168 VGPRs); FP64 holds two (its LDS allows two workgroups per CU)
-template <typename T, int ST>
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 1))) void k_stout_back_chain(Geo g, const T* __restrict__ U, const T* __restrict__ Lc,
                                                              T* __restrict__ Din, double rho,
                                                              const T* __restrict__ Uprev, const T* __restrict__ Cprev,
                                                              T* __restrict__ Lout) {
     __shared__ __align__(16) unsigned char smem[kChainLds<T>];
-    static_assert(4 * 10 * 64 * sizeof(T2<T>) <= kChainLds<T>, "ul + hl fit the staging space");
-    XShare<T> ul = reinterpret_cast<XShare<T>>(smem);
-    PairShare<T> hl = reinterpret_cast<PairShare<T>>(smem + 4 * 6 * 64 * sizeof(T2<T>));
+    static_assert(4 * 10 * kXW * sizeof(T2<T>) <= kChainLds<T>, "ul + hl fit the staging space");
+    XLinks<T> ul = reinterpret_cast<XLinks<T>>(smem);
+    XCoefs<T> hl = reinterpret_cast<XCoefs<T>>(smem + 4 * 6 * kXW * sizeof(T2<T>));
     MStage<T> dst = reinterpret_cast<MStage<T>>(smem);
     MStage<T> cst = reinterpret_cast<MStage<T>>(smem + 4 * 9 * 64 * sizeof(T2<T>));
     const SiteMu sm = site_mu_index(g);
     const int a = sm.mu;
-    int y;
-    if (!stencil_site<(ST > 0)>(g, sm, y)) return;
+    const int y = stencil_site<ROWS>(g, sm);
     int x[4];
     decode(g, y, x);
     const unsigned V = g.V;
     const int lane = (int)(threadIdx.x & 63u);
-    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, back_stencil_acc<T, ST>(g, U, Lc, y, x, a, lane, ul, hl));
-    if constexpr (ST > 0) __syncthreads();  // every wave is done with ul/hl before the staging reuses them
-    back_local_stored<T>(Uprev, Cprev, dn, Din, Lout, V, a, y, lane, dst, cst);
+    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, back_stencil_acc<ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl));
+    __syncthreads();  // every wave is done with ul/hl before the staging reuses them
+    if (in_lattice<ROWS>(g, sm)) back_local_stored<T>(Uprev, Cprev, dn, Din, Lout, V, a, y, lane, dst, cst);
 }
 
 // K2 chained into the K6a of the top level (stored C): dS/dU of the top smeared level, coeff
 // Sigma_mu(y), is Dout of the top level's site-local step at the same (y, mu)
-template <typename T, bool SHARED>
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(kBlock) void k_dsdu_chain(Geo g, const T* __restrict__ Utop, double coeff,
                                                        const T* __restrict__ Uin, const T* __restrict__ Cst,
                                                        T* __restrict__ Din, T* __restrict__ Lout) {
@@ -488,82 +456,47 @@ __global__ __launch_bounds__(kBlock) void k_dsdu_chain(Geo g, const T* __restric
     MStage<T> dst = reinterpret_cast<MStage<T>>(smem);
     MStage<T> cst = reinterpret_cast<MStage<T>>(smem + 4 * 9 * 64 * sizeof(T2<T>));
     const SiteMu sm = site_mu_index(g);
-    int s;
-    if (!stencil_site<SHARED>(g, sm, s)) return;
+    const int s = stencil_site<ROWS>(g, sm);
     int x[4];
     decode(g, s, x);
-    M3<T> sig;
-    if constexpr (SHARED) {
-        R6<T> own;
-        sig = staple_sigma_shared(g, Utop, (unsigned)g.V, s, x, sm.mu, own, xs);
-    } else {
-        sig = staple_sigma(g, Utop, (unsigned)g.V, s, x, sm.mu);
-    }
+    R6<T> own;
+    M3<T> sig = staple_sigma_shared(g, Utop, (unsigned)g.V, s, x, sm.mu, own, xs);
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         sig.m[k].r = scale1(coeff, sig.m[k].r);
         sig.m[k].i = scale1(coeff, sig.m[k].i);
     }
-    if constexpr (SHARED) __syncthreads();  // every wave is done with xs before the staging reuses it
-    back_local_stored<T>(Uin, Cst, sig, Din, Lout, (unsigned)g.V, sm.mu, s, (int)(threadIdx.x & 63u), dst, cst);
+    __syncthreads();  // every wave is done with xs before the staging reuses it
+    if (in_lattice<ROWS>(g, sm)) back_local_stored<T>(Uin, Cst, sig, Din, Lout, (unsigned)g.V, sm.mu, s, (int)(threadIdx.x & 63u), dst, cst);
 }
 
 // ---------------------------------------------------------------------------
 template <typename T>
 hipError_t launch_flow_stage(const Geo& g, const T* W, T* Wout, T* A, double alpha, double beta, hipStream_t st) {
-    const int form = stencil_form(g), nb = grid_sites_mu(g.V);
-    if (form == ST_XROW)
-        k_flow_stage<T, ST_XROW><<<nb, kBlock, 0, st>>>(g, W, Wout, A, alpha, beta);
-    else if (form == ST_SHARED)
-        k_flow_stage<T, ST_SHARED><<<nb, kBlock, 0, st>>>(g, W, Wout, A, alpha, beta);
-    else
-        k_flow_stage<T, ST_OWN><<<nb, kBlock, 0, st>>>(g, W, Wout, A, alpha, beta);
+    by_form<T>(g, [&](auto f) {
+        k_flow_stage<T, decltype(f)::value><<<stencil_groups(f, grid_sites_mu(g.V)), stencil_threads(f), 0, st>>>(g, W, Wout, A, alpha, beta);
+    });
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_stout_forward(const Geo& g, const T* Uin, T* Uout, T* Cst, double rho, hipStream_t st) {
     const int nb = grid_sites_mu(g.V);
-    const bool sh = g.V % 64 == 0;
-    if (Cst && sh)
-        k_stout_forward<T, true, true><<<nb, kBlock, 0, st>>>(g, Uin, Uout, Cst, rho);
-    else if (Cst)
-        k_stout_forward<T, true, false><<<nb, kBlock, 0, st>>>(g, Uin, Uout, Cst, rho);
-    else if (sh)
-        k_stout_forward<T, false, true><<<nb, kBlock, 0, st>>>(g, Uin, Uout, nullptr, rho);
+    if (Cst)
+        by_rows(g, [&](auto rows) { k_stout_forward<T, true, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Uout, Cst, rho); });
     else
-        k_stout_forward<T, false, false><<<nb, kBlock, 0, st>>>(g, Uin, Uout, nullptr, rho);
+        by_rows(g, [&](auto rows) { k_stout_forward<T, false, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Uout, nullptr, rho); });
     return hipGetLastError();
-}
-template <typename T, int OUT>
-void launch_back_stencil(int form, int nb, hipStream_t st, const Geo& g, const T* Uin, const T* Lc, T* Din,
-                         double rho, T* FP, double eps, T* Unew, double eps_u, double* U64) {
-    if (form == ST_XROW)
-        k_stout_back_stencil<T, ST_XROW, OUT><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
-    else if (form == ST_SHARED)
-        k_stout_back_stencil<T, ST_SHARED, OUT><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
-    else
-        k_stout_back_stencil<T, ST_OWN, OUT><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
 }
 template <typename T>
 hipError_t launch_stout_back_chain(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, const T* Uprev,
                                    const T* Cprev, T* Lout, hipStream_t st) {
-    const int nb = grid_sites_mu(g.V), form = stencil_form(g);
-    if (form == ST_XROW)
-        k_stout_back_chain<T, ST_XROW><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, Uprev, Cprev, Lout);
-    else if (form == ST_SHARED)
-        k_stout_back_chain<T, ST_SHARED><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, Uprev, Cprev, Lout);
-    else
-        k_stout_back_chain<T, ST_OWN><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, Uprev, Cprev, Lout);
+    by_rows(g, [&](auto rows) { k_stout_back_chain<T, decltype(rows)::value><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, Uin, Lc, Din, rho, Uprev, Cprev, Lout); });
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_dsdu_chain(const Geo& g, const T* Utop, double coeff, const T* Uin, const T* Cst, T* Din, T* Lout,
                              hipStream_t st) {
-    const int nb = grid_sites_mu(g.V);
-    if (g.V % 64 == 0)
-        k_dsdu_chain<T, true><<<nb, kBlock, 0, st>>>(g, Utop, coeff, Uin, Cst, Din, Lout);
-    else
-        k_dsdu_chain<T, false><<<nb, kBlock, 0, st>>>(g, Utop, coeff, Uin, Cst, Din, Lout);
+    by_rows(g, [&](auto rows) { k_dsdu_chain<T, decltype(rows)::value><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, Utop, coeff, Uin, Cst, Din, Lout); });
     return hipGetLastError();
 }
 // K6a alone (the top level of a backward pass that starts from a given dS/dU)
@@ -572,37 +505,34 @@ hipError_t launch_stout_back_local(const Geo& g, const T* Uin, const T* Cst, con
                                    hipStream_t st) {
     const int nb = grid_sites_mu(g.V);
     if (Cst)
-        k_stout_back_local<T, true, false><<<nb, kBlock, 0, st>>>(g, Uin, Cst, Dout, Din, Lc, rho);
-    else if (g.V % 64 == 0)  // recompute C exactly as k_stout_forward<T, *, true> formed it
-        k_stout_back_local<T, false, true><<<nb, kBlock, 0, st>>>(g, Uin, nullptr, Dout, Din, Lc, rho);
-    else
-        k_stout_back_local<T, false, false><<<nb, kBlock, 0, st>>>(g, Uin, nullptr, Dout, Din, Lc, rho);
+        by_rows(g, [&](auto rows) { k_stout_back_local<T, true, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Cst, Dout, Din, Lc, rho); });
+    else  // recompute C exactly as k_stout_forward formed it
+        by_rows(g, [&](auto rows) { k_stout_back_local<T, false, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, nullptr, Dout, Din, Lc, rho); });
     return hipGetLastError();
 }
 // K6b alone (the thin-link level, or any level whose lower neighbour is not chained)
 template <typename T>
 hipError_t launch_stout_back_stencil(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, hipStream_t st,
                                      int fmode, T* FP, double eps, T* Unew, double eps_u, double* U64) {
-    const int nb = grid_sites_mu(g.V), form = stencil_form(g);
+    const int nb = grid_sites_mu(g.V);
     if (fmode == FORCE_STORE)
-        launch_back_stencil<T, FORCE_STORE>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
+        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_STORE, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
     else if (fmode == FORCE_KICK)
-        launch_back_stencil<T, FORCE_KICK>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
+        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
     else if (fmode == FORCE_KICK_EXP)
-        launch_back_stencil<T, FORCE_KICK_EXP>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
+        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_EXP, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
     else if (fmode == FORCE_KICK_S64 || fmode == FORCE_KICK_EXP_S64) {
         if constexpr (sizeof(T) == 4) {  // FP32 force kernels only
             if (!U64 && fmode == FORCE_KICK_EXP_S64) return hipErrorInvalidValue;
             if (fmode == FORCE_KICK_S64)
-                launch_back_stencil<T, FORCE_KICK_S64>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
+                by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_S64, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
             else
-                launch_back_stencil<T, FORCE_KICK_EXP_S64>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u,
-                                                           U64);
+                by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_EXP_S64, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
         } else {
             return hipErrorInvalidValue;
         }
     } else
-        launch_back_stencil<T, -1>(form, nb, st, g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64);
+        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, -1, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
     return hipGetLastError();
 }
 template <typename T>

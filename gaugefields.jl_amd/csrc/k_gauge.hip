@@ -40,33 +40,24 @@ __global__ __launch_bounds__(kBlock) void k_plaquette(Geo g, const T* __restrict
     block_sum_store<kBlock>(v, partial);
 }
 
-// K1 for workgroups of whole x-rows (NX divides 64, V a multiple of 64): each wave stores its
-// U_w(x) in LDS, so the 13 distinct links the six planes of a site need are loaded once per
-// workgroup (4 own links, U_0(x+nu) of the planes (0, nu); the links at x+0 from the x-row)
-// instead of 4 per plane (24).  Waves 0..2 take the planes (0, w+1) and (1,2) / (1,3) / (2,3):
+// K1 for workgroups of whole x-rows (rows_whole): each wave stores its U_w(x) in LDS, so the 13
+// distinct links the six planes of a site need are loaded once per workgroup (4 own links, U_0(x+nu)
+// of the planes (0, nu); the links at x+0 from the x-row) instead of 4 per plane (24).  Waves 0..2 take the planes (0, w+1) and (1,2) / (1,3) / (2,3):
 // three loaded links each; wave 3 loads only its own link.  Same products in FP64 as k_plaquette.
 // 32^4 FP64: 0.190 -> 0.177 ms per plaquette with the host readback.
 template <typename T>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_plaquette_xrow(
     Geo g, const T* __restrict__ U, double* __restrict__ partial) {
-    __shared__ T2<T> ol[4][6][64];
+    __shared__ T2<T> ol[4][6][kXW];
     const SiteMu sm = site_mu_index(g);
     const int s = sm.s, w = sm.mu;  // V % 64 == 0: every lane is a site
     const int lane = (int)(threadIdx.x & 63u);
     int x[4];
     decode(g, s, x);
     const unsigned V = g.V;
-    auto lds_link = [&](int d, int l) {
-        R6<T> r;
-#pragma unroll
-        for (int e = 0; e < 6; e++) r.v[e] = ol[d][e][l];
-        return full_of(r6_f64(r));
-    };
-    {
-        const R6<T> o = ldr(U, V, w, (unsigned)s);
-#pragma unroll
-        for (int e = 0; e < 6; e++) ol[w][e][lane] = o.v[e];
-    }
+    auto lds_link = [&](int d, int l) { return full_of(r6_f64(shared_link<T>(ol, d, l))); };
+    const XRow xr = xrow_of<true>(g, s, x[0], lane);
+    share_links<true, T>(ol, U, V, w, lane, xr, ldr(U, V, w, (unsigned)s));
     // the wave's memory links, issued before the barrier: plane (0, n1) needs U_0(x+n1); plane
     // (m2, n2) needs U_n2(x+m2) and U_m2(x+n2)
     const int n1 = w + 1;
@@ -76,12 +67,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     __syncthreads();  // every wave's U(x) is in LDS
     double v = 0.0;
     if (w < 3) {
-        const int lxp = xlane(lane, g.n[0] - 1, 1);
         // the second plane's links, in flight during the first plane's products
         const R6<T> l2 = ldr(U, V, n2, (unsigned)(s + dlt(g, x, m2, 1)));
         const R6<T> l3 = ldr(U, V, m2, (unsigned)(s + dlt(g, x, n2, 1)));
         // Re tr U_mu(x) U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag = Re tr (a b^dag)
-        v += retr_nd(mul(lds_link(0, lane), lds_link(n1, lxp)), mul(lds_link(n1, lane), full_of(r6_f64(l1))));
+        v += retr_nd(mul(lds_link(0, lane), lds_link(n1, xr.p)), mul(lds_link(n1, lane), full_of(r6_f64(l1))));
         asm volatile("" : "+v"(v));  // the first plane before the second one's LDS reads
         v += retr_nd(mul(lds_link(m2, lane), full_of(r6_f64(l2))), mul(lds_link(n2, lane), full_of(r6_f64(l3))));
     }
@@ -158,22 +148,17 @@ __global__ __launch_bounds__(1024) void k_sum_partials(const double* __restrict_
 }
 
 // K2: dSdU_mu = coeff * Sigma_mu
-// SHARED: upper-staple products shared between directions through LDS (V % 64 == 0)
-template <typename T, bool SHARED>
+// (upper-staple products shared between directions through LDS)
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(kBlock) void k_dsdu(Geo g, const T* __restrict__ U, double coeff, T* __restrict__ D) {
-    __shared__ T2<T> xs[SHARED ? 6 : 1][6][64];
+    __shared__ T2<T> xs[6][6][64];
     const SiteMu sm = site_mu_index(g);
-    int s;
-    if (!stencil_site<SHARED>(g, sm, s)) return;
+    const int s = stencil_site<ROWS>(g, sm);
     int x[4];
     decode(g, s, x);
-    M3<T> sig;
-    if constexpr (SHARED) {
-        R6<T> own;
-        sig = staple_sigma_shared(g, U, (unsigned)g.V, s, x, sm.mu, own, xs);
-    } else {
-        sig = staple_sigma(g, U, (unsigned)g.V, s, x, sm.mu);
-    }
+    R6<T> own;
+    M3<T> sig = staple_sigma_shared(g, U, (unsigned)g.V, s, x, sm.mu, own, xs);
+    if (!in_lattice<ROWS>(g, sm)) return;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         sig.m[k].r = scale1(coeff, sig.m[k].r);
@@ -190,32 +175,16 @@ __global__ __launch_bounds__(kBlock) void k_dsdu(Geo g, const T* __restrict__ U,
 //     on the FP64 momenta (FP points to them) and FP64 links U64 (updated in place: a thread reads
 //     only its own U64 link); the float force enters as F = float(fac c), as if stored, and Unew
 //     receives the updated links rounded to float
-// ST (stencil_form): ST_OWN per-thread staples; ST_SHARED upper-staple plaquettes shared between
-// directions through LDS (ta_force_shared, V % 64 == 0); ST_XROW the same with the x-neighbour
-// links from LDS as well (ta_force_xrow, NX divides 64).  At most 168 VGPRs: three waves per SIMD.
+// ST: form of the stencil (stencil_form).  At most 168 VGPRs: three waves per SIMD.
 template <typename T, int MODE, int ST>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_force(Geo g, const T* __restrict__ U, T* __restrict__ FP,
-                                                  T* __restrict__ Unew, double fac, double eps_u,
-                                                  double eps_p, double* __restrict__ U64) {
-    __shared__ T2<T> ol[ST ? 4 : 1][6][64];
-    __shared__ T2<T> tp[ST ? 7 : 1][4][64];
-    const SiteMu sm = site_mu_index(g);
-    const int mu = sm.mu;
-    int s;
-    if (!stencil_site<(ST > 0)>(g, sm, s)) return;
-    int x[4];
-    decode(g, s, x);
-    const unsigned V = g.V;
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_force(
+    Geo g, const T* __restrict__ U, T* __restrict__ FP, T* __restrict__ Unew, double fac, double eps_u, double eps_p,
+    double* __restrict__ U64) {
+    int s, mu;
     R6<T> own;
     T c[8];
-    if constexpr (ST == ST_XROW) {
-        ta_force_xrow(g, U, V, s, x, mu, own, ol, tp, c);
-    } else if constexpr (ST == ST_SHARED) {
-        ta_force_shared(g, U, V, s, x, mu, own, ol, tp, c);
-    } else {
-        const M3<T> sig = staple_sigma_own(g, U, V, s, x, mu, own);
-        ta_coeffs(mul(full_of(own), sig), c);
-    }
+    if (!ta_force<ST, T>(g, U, s, mu, own, c)) return;
+    const unsigned V = g.V;
     const M3<T> umu = full_of(own);
     if constexpr (MODE == FORCE_KICK_S64 || MODE == FORCE_KICK_EXP_S64) {
         double* P64 = reinterpret_cast<double*>(FP);
@@ -250,12 +219,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_exp_update(Geo g, const T* __restrict__ Uin, T* __restrict__ Uout,
                                                        const T* __restrict__ P, double eps) {
-    // purely streaming: one thread per site walking its four links keeps more loads in flight
+    // purely streaming: one thread per site walking its four links keeps more loads in flight; on
+    // lattices that leave CUs empty so (link_dirs) a thread takes one link, gridDim.y = 4
     const int s = site_index();
     if (s >= g.V) return;
     const unsigned V = g.V;
 #pragma unroll 1
-    for (int mu = 0; mu < 4; mu++) {
+    for (int mu = (int)blockIdx.y; mu < 4; mu += (int)gridDim.y) {
         T p[8];
         ldp<T, GF_LD_NT>(P, V, mu, s, p);
         const M3<T> un = exp_coeffs_times(p, eps, ldu<T, GF_LD_NT>(Uin, V, mu, s));
@@ -287,7 +257,7 @@ __global__ __launch_bounds__(kBlock) void k_links_widen(const float* __restrict_
 // the force kernels read U32, the links rounded to float (their FP64-state epilogues kick P64 and
 // update U64 in the same launch).  The lone steps: MODE 1: U64 <- exp(eps_u P64) U64 (in place:
 // only the thread's own link is read) and U32 <- round(U64).  MODE 3: U32 <- round(U64).
-// One thread per site walking its four links: a streaming kernel.
+// One thread per site walking its four links (gridDim.y = 1) or per link (4): a streaming kernel.
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_state64_step(Geo g, const double* __restrict__ P64,
                                                          double* __restrict__ U64, float* __restrict__ U32,
@@ -296,7 +266,7 @@ __global__ __launch_bounds__(kBlock) void k_state64_step(Geo g, const double* __
     if (s >= g.V) return;
     const unsigned V = g.V;
 #pragma unroll 1
-    for (int mu = 0; mu < 4; mu++) {
+    for (int mu = (int)blockIdx.y; mu < 4; mu += (int)gridDim.y) {
         if (MODE == 3) {
             stu<float, GF_ST_NT>(U32, V, mu, s, round_link<float>(ldu<double, GF_LD_NT>(U64, V, mu, s)));
             continue;
@@ -311,7 +281,7 @@ __global__ __launch_bounds__(kBlock) void k_state64_step(Geo g, const double* __
 
 hipError_t launch_state64_step(int mode, const Geo& g, const double* P64, double* U64, float* U32, double eps_u,
                                hipStream_t st) {
-    const int nb = grid_for(g.V);
+    const dim3 nb(grid_for(g.V), link_dirs(g.V));
     if (mode == 1)
         k_state64_step<1><<<nb, kBlock, 0, st>>>(g, P64, U64, U32, eps_u);
     else if (mode == 3)
@@ -478,7 +448,9 @@ hipError_t launch_sum_partials(const double* partial, int n, double* out, hipStr
 template <typename T>
 hipError_t launch_plaquette(const Geo& g, const T* U, double* partial, double* out, hipStream_t st) {
     const int nb = grid_sites_mu(g.V);
-    if (sizeof(T) == 8 && stencil_form(g) == ST_XROW)  // FP32: 16 B spilled at 168 VGPRs, slower
+    // the shared form for whole rows in FP64 only: with rows cut by the groups it was slower (24^4: 57 -> 60
+    // us), and in FP32 it spilled 16 B at 168 VGPRs (32^4: 0.156 -> 0.171 ms)
+    if (sizeof(T) == 8 && rows_whole(g))
         k_plaquette_xrow<T><<<nb, kBlock, 0, st>>>(g, U, partial);
     else
         k_plaquette<T><<<nb, kBlock, 0, st>>>(g, U, partial);
@@ -499,45 +471,31 @@ hipError_t launch_momenta_dot(const Geo& g, const T* P, double* partial, double*
 }
 template <typename T>
 hipError_t launch_dsdu(const Geo& g, const T* U, double coeff, T* D, hipStream_t st) {
-    if (g.V % 64 == 0)
-        k_dsdu<T, true><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, U, coeff, D);
-    else
-        k_dsdu<T, false><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, U, coeff, D);
+    by_rows(g, [&](auto rows) { k_dsdu<T, decltype(rows)::value><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, U, coeff, D); });
     return hipGetLastError();
-}
-template <typename T, int MODE>
-void launch_force_st(int form, int nb, hipStream_t st, const Geo& g, const T* U, T* FP, T* Unew, double fac,
-                     double eps_u, double eps_p = 0.0, double* U64 = nullptr) {
-    if (form == ST_XROW)
-        k_force<T, MODE, ST_XROW><<<nb, kBlock, 0, st>>>(g, U, FP, Unew, fac, eps_u, eps_p, U64);
-    else if (form == ST_SHARED)
-        k_force<T, MODE, ST_SHARED><<<nb, kBlock, 0, st>>>(g, U, FP, Unew, fac, eps_u, eps_p, U64);
-    else
-        k_force<T, MODE, ST_OWN><<<nb, kBlock, 0, st>>>(g, U, FP, Unew, fac, eps_u, eps_p, U64);
 }
 template <typename T>
 hipError_t launch_force(int mode, const Geo& g, const T* U, T* FP, T* Unew, double coeff, double eps_p,
                         double eps_u, hipStream_t st, double* U64) {
     const int nb = grid_sites_mu(g.V);
     const double fac = -coeff / 3.0;
-    const int form = stencil_form(g);
     switch (mode) {
         case FORCE_STORE:
-            launch_force_st<T, FORCE_STORE>(form, nb, st, g, U, FP, Unew, fac, eps_u);
+            by_form<T>(g, [&](auto f) { k_force<T, FORCE_STORE, decltype(f)::value><<<stencil_groups(f, nb), stencil_threads(f), 0, st>>>(g, U, FP, Unew, fac, eps_u, 0.0, nullptr); });
             break;
         case FORCE_KICK:
-            launch_force_st<T, FORCE_KICK>(form, nb, st, g, U, FP, Unew, fac * eps_p, eps_u);
+            by_form<T>(g, [&](auto f) { k_force<T, FORCE_KICK, decltype(f)::value><<<stencil_groups(f, nb), stencil_threads(f), 0, st>>>(g, U, FP, Unew, fac * eps_p, eps_u, 0.0, nullptr); });
             break;
         case FORCE_KICK_EXP:
-            launch_force_st<T, FORCE_KICK_EXP>(form, nb, st, g, U, FP, Unew, fac * eps_p, eps_u);
+            by_form<T>(g, [&](auto f) { k_force<T, FORCE_KICK_EXP, decltype(f)::value><<<stencil_groups(f, nb), stencil_threads(f), 0, st>>>(g, U, FP, Unew, fac * eps_p, eps_u, 0.0, nullptr); });
             break;
         case FORCE_KICK_S64:
         case FORCE_KICK_EXP_S64:
             if constexpr (sizeof(T) == 4) {
                 if (mode == FORCE_KICK_S64)
-                    launch_force_st<T, FORCE_KICK_S64>(form, nb, st, g, U, FP, Unew, fac, 0.0, eps_p, U64);
+                    by_form<T>(g, [&](auto f) { k_force<T, FORCE_KICK_S64, decltype(f)::value><<<stencil_groups(f, nb), stencil_threads(f), 0, st>>>(g, U, FP, Unew, fac, 0.0, eps_p, U64); });
                 else
-                    launch_force_st<T, FORCE_KICK_EXP_S64>(form, nb, st, g, U, FP, Unew, fac, eps_u, eps_p, U64);
+                    by_form<T>(g, [&](auto f) { k_force<T, FORCE_KICK_EXP_S64, decltype(f)::value><<<stencil_groups(f, nb), stencil_threads(f), 0, st>>>(g, U, FP, Unew, fac, eps_u, eps_p, U64); });
                 break;
             } else {
                 return hipErrorInvalidValue;
@@ -549,7 +507,7 @@ hipError_t launch_force(int mode, const Geo& g, const T* U, T* FP, T* Unew, doub
 }
 template <typename T>
 hipError_t launch_exp_update(const Geo& g, const T* Uin, T* Uout, const T* P, double eps, hipStream_t st) {
-    k_exp_update<T><<<grid_for(g.V), kBlock, 0, st>>>(g, Uin, Uout, P, eps);
+    k_exp_update<T><<<dim3(grid_for(g.V), link_dirs(g.V)), kBlock, 0, st>>>(g, Uin, Uout, P, eps);
     return hipGetLastError();
 }
 hipError_t launch_links_widen(const float* Uf, double* Ud, int V, hipStream_t st) {

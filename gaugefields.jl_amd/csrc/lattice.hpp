@@ -78,12 +78,11 @@ __device__ __forceinline__ int dlt(const Geo& g, const int x[4], int mu, int d) 
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b -> XCD b % 8).  xcd_block()
-// renumbers them so that XCD k runs the contiguous k-th eighth of the block sequence.
+// renumbers them so that XCD k runs the k-th of eight contiguous parts of the block sequence (the
+// first nb % 8 parts are one block longer), which keeps neighbouring groups in one XCD's L2.
 __device__ __forceinline__ unsigned xcd_block() {
-    unsigned b = blockIdx.x;
-    const unsigned nb = gridDim.x;
-    if ((nb & 7u) == 0u) b = (b & 7u) * (nb >> 3) + (b >> 3);
-    return b;
+    const unsigned b = blockIdx.x, k = b & 7u, q = gridDim.x >> 3, r = gridDim.x & 7u;
+    return k * q + min(k, r) + (b >> 3);
 }
 
 // one thread per site (legacy site-parallel kernels: reductions, layout conversion)
@@ -518,7 +517,7 @@ __device__ __forceinline__ M3<T> staple_sigma_pipe(const Geo& g, const T* __rest
     }
     return sig;
 }
-// the staple sum and U_mu(x) (own, as loaded): force, flow and stout-forward kernels
+// the staple sum and U_mu(x) (own, as loaded): the heatbath kernel
 template <typename T, int DEPTH = 1>
 __device__ __forceinline__ M3<T> staple_sigma_own(const Geo& g, const T* __restrict__ U, unsigned V, int s,
                                                   const int x[4], int mu, R6<T>& own) {
@@ -533,8 +532,7 @@ __device__ __forceinline__ M3<T> staple_sigma_own(const Geo& g, const T* __restr
 // barrier every wave reads the three it needs: per site 12 of 76 link loads and 6 of 24 staple
 // products fewer than staple_sigma_own.  Pair (a, b), a < b, is formed by wave
 // w0: (0,1), (0,3)  w1: (1,2), (1,3)  w2: (0,2)  w3: (2,3), in a loop of its own ahead of the
-// pipelined lower staples.  Requires every lane of the workgroup to reach the barrier: the
-// kernels use it only when V is a multiple of 64 (no idle lanes).
+// pipelined lower staples.  Every lane of the workgroup has to reach the barrier.
 // LDS: xs[6][6][64] complex (37 KB FP64, 18 KB FP32).
 __device__ __forceinline__ int pair_index(int a, int b) {  // a < b
     return a == 0 ? b - 1 : (a == 1 ? b + 1 : 5);
@@ -604,116 +602,94 @@ __device__ __forceinline__ M3<T> staple_sigma_shared(const Geo& g, const T* __re
             }
         acc_mul_nd(sig, Mt, full_of(cur));
     }
+    // pin the sum: otherwise the staple arithmetic is sunk past the callers' in_lattice branch and
+    // every loaded link stays live (400 registers)
+#pragma unroll
+    for (int e = 0; e < 9; e++) asm volatile("" : "+v"(sig.m[e].r), "+v"(sig.m[e].i));
     return sig;
+}
+
+// ---------------------------------------------------------------------------
+// x-neighbours inside a workgroup.  The 64 sites of a group are consecutive, so x +- 1 of a site is
+// a site of the same group except where the group cuts a row: then at most four sites outside it are
+// needed (the one before its first and the one after its last, and, round the periodic boundary, the
+// first site of the row it starts in and the last of the row it ends in).  An array of kXW entries
+// per plane holds the 64 sites and these four, so the neighbours come from LDS on any extents.
+constexpr int kXW = 68;
+template <typename T>
+using XLinks = T2<T> (*)[6][kXW];
+template <typename T>
+using XCoefs = T2<T> (*)[4][kXW];
+// The ROWS kernels are those of lattices whose groups are all whole rows (rows_whole: NX divides 64 and
+// V is a multiple of 64): no outside sites, no idle lanes (1-2 % faster at 32^4 than the general form).
+inline bool rows_whole(const Geo& g) { return 64 % g.n[0] == 0 && g.V % 64 == 0; }
+struct XRow {
+    int m, p;  // entries of x - 1 and x + 1
+    int halo;  // lanes 0..3: the outside site of entry 64 + lane; others: -1 (none)
+};
+template <bool ROWS>
+__device__ __forceinline__ XRow xrow_of(const Geo& g, int s, int x0, int lane) {
+    const int nx = g.n[0];
+    if constexpr (ROWS) return XRow{(lane & ~(nx - 1)) | ((lane - 1) & (nx - 1)), (lane & ~(nx - 1)) | ((lane + 1) & (nx - 1)), -1};
+    const int s0 = __builtin_amdgcn_readfirstlane(s - lane);  // first site of the group (lane 0 is a site)
+    XRow r;
+    const int p = (x0 == nx - 1 ? s - x0 : s + 1) - s0, m = (x0 == 0 ? s + nx - 1 : s - 1) - s0;
+    r.p = p > 63 ? 64 : (p < 0 ? 65 : p);
+    r.m = m < 0 ? 66 : (m > 63 ? 67 : m);
+    r.halo = -1;
+    if (64 % nx != 0 && lane < 4) {
+        const int first = s0 - (int)((unsigned)s0 - divq(g, 0, (unsigned)s0) * (unsigned)nx);
+        const int last = (int)(divq(g, 0, (unsigned)(s0 + 63)) * (unsigned)nx) + nx - 1;
+        const int h = lane == 0 ? s0 + 64 : (lane == 1 ? first : (lane == 2 ? s0 - 1 : last));
+        r.halo = min(max(h, 0), g.V - 1);
+    }
+    return r;
+}
+// U_mu of the workgroup's sites (own, already loaded) and of its outside x-neighbours into LDS
+template <bool ROWS, typename T>
+__device__ __forceinline__ void share_links(XLinks<T> ol, const T* __restrict__ U, unsigned V, int mu, int lane,
+                                            const XRow& xr, const R6<T>& own) {
+#pragma unroll
+    for (int e = 0; e < 6; e++) ol[mu][e][lane] = own.v[e];
+    if (!ROWS && xr.halo >= 0) {
+        const R6<T> h = ldr(U, V, mu, (unsigned)xr.halo);
+#pragma unroll
+        for (int e = 0; e < 6; e++) ol[mu][e][64 + lane] = h.v[e];
+    }
+}
+template <typename T>
+__device__ __forceinline__ R6<T> shared_link(XLinks<T> ol, int d, int l) {
+    R6<T> r;
+#pragma unroll
+    for (int e = 0; e < 6; e++) r.v[e] = ol[d][e][l];
+    return r;
 }
 
 // ---------------------------------------------------------------------------
 // TA(U_mu(x) Sigma_mu(x)) (8 su(3) coefficients, ta_coeffs) with the upper staples taken as
 // whole plaquettes shared between directions.  U_mu(x) X_mu,nu U_nu(x)^dag is the plaquette
 // P_mu,nu(x), and P_nu,mu = P_mu,nu^dag, so TA(P_nu,mu) = -TA(P_mu,nu).  Each unordered pair's
-// plaquette is formed once (by the waves and in the slots of staple_sigma_shared), only its 8
-// TA coefficients go to LDS, and the links U_nu(x) reach the other waves through LDS as well:
-// per wave 14 link loads (88 vector-memory loads with the momenta) instead of 17 (106).
-// Order: lower staples, U_mu(x) (-> LDS, TA of U_mu times the lower staples), the pairs.
-// TA is linear, so the result is TA(U_mu Sigma_mu) up to rounding.  Two workgroup barriers
-// (every lane must reach them: V a multiple of 64).
-// LDS: ol[4][6][64] links and tp[7][4][64] coefficient pairs (52 KB FP64, 26 KB FP32).
+// plaquette is formed once and only its 8 TA coefficients go to LDS; the links U_nu(x) and the links
+// at x +- 1 reach the other waves through LDS as well: U_mu(x-1), U_0(x-1) of the nu = 0 lower staple
+// and U_b(x+1) of the pairs (0, b).  Pairs: w0 (0,3); w1 (1,2), (0,1); w2 (2,3), (0,2); w3 (1,3)
+// (link loads per wave 12, 11, 11, 10; 17 with neither sharing).
+// Order: lower staples, TA of U_mu times them, the pairs.  TA is linear, so the result is
+// TA(U_mu Sigma_mu) up to rounding.  Two workgroup barriers (every lane must reach them: lanes past
+// the last site work on a clamped one, and the kernels store nothing for them).
+// LDS: ol[4][6][kXW] links and tp[6][4][64] coefficient pairs (50 KB FP64: three workgroups per CU).
 template <typename T>
 using PairShare = T2<T> (*)[4][64];
-template <typename T>
-__device__ __forceinline__ void ta_force_shared(const Geo& g, const T* __restrict__ U, unsigned V, int s,
-                                                const int x[4], int mu, R6<T>& own, XShare<T> ol,
-                                                PairShare<T> tp, T c[8]) {
-    const int lane = (int)(threadIdx.x & 63u);
-    int fw[4];
-#pragma unroll
-    for (int d = 0; d < 4; d++) fw[d] = dlt(g, x, d, 1);
-    // pairs formed by this wave: w0 (0,1),(0,3); w1 (1,2),(1,3); w2 (0,2); w3 (2,3); waves 2 and 3
-    // form (2,3) a second time into the unused slot 6 (same branch-free sequence for all)
-    const int pa1 = mu == 2 ? 0 : (mu == 3 ? 2 : mu);
-    const int pb1 = mu == 0 ? 1 : (mu == 1 ? 2 : (mu == 2 ? 2 : 3));
-    const int pa2 = mu < 2 ? mu : 2;
-    const int pb2 = 3;
-    const int p1 = pair_index(pa1, pb1), p2 = mu < 2 ? pair_index(pa2, pb2) : 6;
-    // TA coefficients of P_a,b = U_a(x) X U_b(x)^dag into slot p
-    auto plaq = [&](int a, int b, const M3<T>& X, int p) {
-        R6<T> ra, rb;
-#pragma unroll
-        for (int e = 0; e < 6; e++) {
-            ra.v[e] = ol[a][e][lane];
-            rb.v[e] = ol[b][e][lane];
-        }
-        T q[8];
-        ta_coeffs(su3_mul_nd(rows_of(su3_mul(ra, X)), full_of(rb)), q);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            T2<T> v;
-            v.x = q[2 * e];
-            v.y = q[2 * e + 1];
-            tp[p][e][lane] = v;
-        }
-    };
-    const M3<T> sig = staple_sigma_pipe<T, true, true>(g, U, V, s, x, mu, &own);
-#pragma unroll
-    for (int e = 0; e < 6; e++) ol[mu][e][lane] = own.v[e];
-    ta_coeffs(mul(full_of(own), sig), c);
-    // pin c here: otherwise the staple arithmetic is sunk past the pairs to its use, keeping
-    // every loaded staple link live across them
-    asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]),
-                 "+v"(c[7]));
-    // the pairs: a loop of its own, so that its loads are not hoisted into the staples above
-#pragma unroll 1
-    for (int q = 0; q < 2; q++) {
-        const int a = q == 0 ? pa1 : pa2, b = q == 0 ? pb1 : pb2;
-        const int fa = sel4(a, fw[0], fw[1], fw[2], fw[3]), fb = sel4(b, fw[0], fw[1], fw[2], fw[3]);
-        const M3<T> Xp = su3_mul_nd(ldr(U, V, b, (unsigned)(s + fa)), ldu(U, V, a, (unsigned)(s + fb)));
-        if (q == 0) __syncthreads();  // every wave's U(x) is in LDS
-        plaq(a, b, Xp, q == 0 ? p1 : p2);
-    }
-    __syncthreads();  // every pair's coefficients are in LDS
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int nu = j + (j >= mu ? 1 : 0);
-        const int p = pair_index(mu < nu ? mu : nu, mu < nu ? nu : mu);
-        const T sg = mu < nu ? T(1) : T(-1);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const T2<T> v = tp[p][e][lane];
-            c[2 * e] = fma(sg, v.x, c[2 * e]);
-            c[2 * e + 1] = fma(sg, v.y, c[2 * e + 1]);
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// ta_force_shared for workgroups of whole x-rows (NX divides 64, V a multiple of 64): the
-// x-neighbours x +- 1 of every site are sites of the same workgroup, so the links at them come
-// from the U(x) copies in LDS instead of memory: U_mu(x-1), U_0(x-1) of the nu = 0 lower staple
-// and U_b(x+1) of the pairs (0, b).  Pairs: w0 (0,3); w1 (1,2), (0,1); w2 (2,3), (0,2); w3 (1,3)
-// (link loads per wave 12, 11, 11, 10 instead of 14).
-// LDS: ol[4][6][64] links and tp[6][4][64] coefficient pairs.
-__device__ __forceinline__ int xlane(int lane, int nxm1, int d) { return (lane & ~nxm1) | ((lane + d) & nxm1); }
-template <typename T>
+template <bool ROWS, typename T>
 __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict__ U, unsigned V, int s,
-                                              const int x[4], int mu, R6<T>& own, XShare<T> ol,
+                                              const int x[4], int mu, R6<T>& own, XLinks<T> ol,
                                               PairShare<T> tp, T c[8]) {
     const int lane = (int)(threadIdx.x & 63u);
-    const int nxm1 = g.n[0] - 1;
-    const int lxm = xlane(lane, nxm1, -1), lxp = xlane(lane, nxm1, 1);
+    const XRow xr = xrow_of<ROWS>(g, s, x[0], lane);
     int fw[4];
 #pragma unroll
     for (int d = 0; d < 4; d++) fw[d] = dlt(g, x, d, 1);
-    auto lds_link = [&](int d, int l) {
-        R6<T> r;
-#pragma unroll
-        for (int e = 0; e < 6; e++) r.v[e] = ol[d][e][l];
-        return r;
-    };
-    {
-        const R6<T> o = ldr(U, V, mu, (unsigned)s);
-#pragma unroll
-        for (int e = 0; e < 6; e++) ol[mu][e][lane] = o.v[e];
-    }
+    auto lds_link = [&](int d, int l) { return shared_link<T>(ol, d, l); };
+    share_links<ROWS, T>(ol, U, V, mu, lane, xr, ldr(U, V, mu, (unsigned)s));
     __syncthreads();  // every wave's U(x) is in LDS
     M3<T> sig;
     if (mu == 0) {
@@ -721,8 +697,8 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
     } else {
         sig = staple_sigma_pipe<T, false, true, 1>(g, U, V, s, x, mu, nullptr);
         // nu = 0: (U_mu(x-1) U_0(x+mu-1))^dag U_0(x-1)
-        const M3<T> X = su3_mul(lds_link(mu, lxm), ldu(U, V, 0, (unsigned)(s + fw[mu] + dlt(g, x, 0, -1))));
-        acc_mul_dn(sig, X, full_of(lds_link(0, lxm)));
+        const M3<T> X = su3_mul(lds_link(mu, xr.m), ldu(U, V, 0, (unsigned)(s + fw[mu] + dlt(g, x, 0, -1))));
+        acc_mul_dn(sig, X, full_of(lds_link(0, xr.m)));
     }
     own = lds_link(mu, lane);  // read back rather than held through the staples
     ta_coeffs(mul(full_of(own), sig), c);
@@ -736,7 +712,7 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
         const int a = q == 1 ? 0 : (mu == 2 ? 2 : (mu == 3 ? 1 : mu));
         const int b = q == 1 ? mu : (mu == 0 ? 3 : (mu == 1 ? 2 : 3));
         // X_ab = U_b(x+a) U_a(x+b)^dag
-        const R6<T> ub = a == 0 ? lds_link(b, lxp) : ldr(U, V, b, (unsigned)(s + sel4(a, fw[0], fw[1], fw[2], fw[3])));
+        const R6<T> ub = a == 0 ? lds_link(b, xr.p) : ldr(U, V, b, (unsigned)(s + sel4(a, fw[0], fw[1], fw[2], fw[3])));
         const M3<T> X = su3_mul_nd(ub, ldu(U, V, a, (unsigned)(s + sel4(b, fw[0], fw[1], fw[2], fw[3]))));
         T q8[8];
         ta_coeffs(su3_mul_nd(rows_of(su3_mul(lds_link(a, lane), X)), full_of(lds_link(b, lane))), q8);
@@ -764,64 +740,123 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
     }
 }
 
-// staple_sigma_own or, when SHARED, staple_sigma_shared (xs: the kernel's LDS array)
-template <typename T, bool SHARED>
-__device__ __forceinline__ M3<T> staple_sum_own(const Geo& g, const T* __restrict__ U, unsigned V, int s,
-                                                const int x[4], int mu, R6<T>& own, XShare<T> xs) {
-    if constexpr (SHARED)
-        return staple_sigma_shared(g, U, V, s, x, mu, own, xs);
-    else
-        return staple_sigma_own(g, U, V, s, x, mu, own);
+// Site of a stencil thread.  The stencil kernels have workgroup barriers, so no lane leaves early:
+// lanes past the last site (only where V is not a multiple of 64) work on a clamped one, and their
+// kernels store nothing for them (in_lattice).
+template <bool ROWS>
+__device__ __forceinline__ int stencil_site(const Geo& g, const SiteMu& sm) {
+    return ROWS ? sm.s : min(sm.s, g.V - 1);
 }
-// Stencil form of the force-type kernels (k_force, k_flow_stage): per-thread staples; upper-
-// staple plaquettes shared through LDS (every lane a site: V % 64 == 0); and the same with the
-// x-neighbour links from LDS (workgroups of whole x-rows: NX divides 64).
-enum { ST_OWN = 0, ST_SHARED = 1, ST_XROW = 2 };
-inline int stencil_form(const Geo& g) {
-    if (g.V % 64 != 0) return ST_OWN;
-    return 64 % g.n[0] == 0 ? ST_XROW : ST_SHARED;
-}
-// Site of a stencil thread.  The SHARED kernels have a workgroup barrier, so no lane may
-// leave early: they run only for V % 64 == 0, where every lane is a site; the clamp keeps
-// their indices in range regardless.
-template <bool SHARED>
-__device__ __forceinline__ bool stencil_site(const Geo& g, const SiteMu& sm, int& s) {
-    s = sm.s;
-    if constexpr (SHARED) {
-        s = min(s, g.V - 1);
-        return true;
-    } else {
-        return s < g.V;
-    }
+template <bool ROWS>
+__device__ __forceinline__ bool in_lattice(const Geo& g, const SiteMu& sm) {
+    return ROWS || sm.s < g.V;
 }
 
-// Unpipelined form for kernels with large register state of their own (the stout backward's
-// recomputation, dS/dU off the 64-site grid), where the prefetch buffer would cost occupancy: links
-// are loaded at their use, through opaque copies of the site indices so that the compiler
-// neither merges them with the loads of other (mu, nu) iterations nor hoists them all.
+// ---------------------------------------------------------------------------
+// ta_force_xrow for small lattices, where a kernel's time is the length of one wave's chain: a workgroup of
+// three waves over 64 sites and one direction mu, wave j forming the two staples of U_mu in the j-th
+// plane and TA(U_mu times them), the three added in LDS.  A wave waits for two batches of loads instead
+// of a dozen links one after another and multiplies a third of the matrices, and the work is spread over
+// four times as many CUs; no product is shared between directions, so the whole lattice costs 1.3 times
+// the operations, which one that leaves CUs empty does not notice.  Wave 0 returns true and goes on with
+// c and own.
 template <typename T>
-__device__ __forceinline__ M3<T> staple_sigma(const Geo& g, const T* __restrict__ U, unsigned V, int s,
-                                              const int x[4], int mu) {
-    M3<T> sig = zero3<T>();
-    const int spm = s + dlt(g, x, mu, 1);
+__device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict__ U, unsigned V, int s, const int x[4],
+                                              int mu, R6<T>& own, T2<T> (*tp)[4][64], T c[8]) {
+    const int lane = (int)(threadIdx.x & 63u);
+    const int j = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nu = j + (j >= mu ? 1 : 0);
+    int fw[4], bw[4];
 #pragma unroll
-    for (int nu = 0; nu < 4; nu++) {
-        if (nu == mu) continue;
-        {  // upper: (U_nu(x+mu) U_mu(x+nu)^dag) U_nu(x)^dag
-            int s0 = s, s1 = spm, spn = s + dlt(g, x, nu, 1);
-            asm volatile("" : "+v"(s0), "+v"(s1), "+v"(spn));
-            const M3<T> a = mul_nd(ldu(U, V, nu, s1), ldu(U, V, mu, spn));
-            acc_mul_nd(sig, a, ldu(U, V, nu, s0));
-        }
-        {  // lower: (U_mu(x-nu) U_nu(x+mu-nu))^dag U_nu(x-nu)
-            const int dmn = dlt(g, x, nu, -1);
-            int smn = s + dmn, spmmn = spm + dmn;
-            asm volatile("" : "+v"(smn), "+v"(spmmn));
-            const M3<T> b = mul(ldu(U, V, mu, smn), ldu(U, V, nu, spmmn));
-            acc_mul_dn(sig, b, ldu(U, V, nu, smn));
+    for (int d = 0; d < 4; d++) {
+        fw[d] = dlt(g, x, d, 1);
+        bw[d] = dlt(g, x, d, -1);
+    }
+    const int fmu = sel4(mu, fw[0], fw[1], fw[2], fw[3]), fnu = sel4(nu, fw[0], fw[1], fw[2], fw[3]);
+    const int bnu = sel4(nu, bw[0], bw[1], bw[2], bw[3]);
+    M3<T> sig = zero3<T>();
+    {
+        const R6<T> a = ldr(U, V, nu, (unsigned)(s + fmu)), b = ldr(U, V, mu, (unsigned)(s + fnu)),
+                    d = ldr(U, V, nu, (unsigned)s);
+        __builtin_amdgcn_sched_barrier(0);
+        const M3<T> X = su3_mul_nd(a, full_of(b));
+        const R6<T> e = ldr(U, V, mu, (unsigned)(s + bnu)), f = ldr(U, V, nu, (unsigned)(s + fmu + bnu));
+        __builtin_amdgcn_sched_barrier(0);
+        acc_mul_nd(sig, X, full_of(d));
+        const R6<T> h = ldr(U, V, nu, (unsigned)(s + bnu));
+        own = ldr(U, V, mu, (unsigned)s);
+        __builtin_amdgcn_sched_barrier(0);
+        acc_mul_dn(sig, su3_mul(e, full_of(f)), full_of(h));
+    }
+    ta_coeffs(mul(full_of(own), sig), c);
+    if (j > 0) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            T2<T> v;
+            v.x = c[2 * e];
+            v.y = c[2 * e + 1];
+            tp[j - 1][e][lane] = v;
         }
     }
-    return sig;
+    __syncthreads();
+    if (j > 0) return false;
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const T2<T> v = tp[k][e][lane];
+            c[2 * e] += v.x;
+            c[2 * e + 1] += v.y;
+        }
+    return true;
+}
+
+// Forms of the force-type kernels (k_force, k_flow_stage), chosen by stencil_form:
+//   ST_WIDE  lattices of few 64-site groups: ta_force_wide, four workgroups of three waves a group
+//   ST_ROWS  groups of whole x-rows (rows_whole): ta_force_xrow, a workgroup of four waves a group
+//   ST_CUT   any other extents: the same with outside x-neighbours and idle lanes
+// MD update / force + kick, the other forms -> ST_WIDE (us): FP64 4^4 7.9 / 6.7 -> 4.7 / 3.8, 8^4 9.3 / 7.3 ->
+// 5.8 / 4.0, 10x6x14x9 (119 groups) 9.9 / 6.3 -> 8.4 / 6.0, 12^3x8 (216 groups) 11.3 / 7.9 -> 11.2 / 8.3; FP32
+// 8^4 8.5 / 6.6 -> 5.1 / 3.6, 12^3x8 9.3 / 6.5 -> 8.9 / 5.4.  Hence the limits.
+enum { ST_CUT = 0, ST_ROWS = 1, ST_WIDE = 2 };
+template <typename T>
+inline int stencil_form(const Geo& g) {
+    if ((g.V + 63) / 64 <= (sizeof(T) == 8 ? 160 : 256)) return ST_WIDE;
+    return rows_whole(g) ? ST_ROWS : ST_CUT;
+}
+constexpr int stencil_threads(int form) { return form == ST_WIDE ? 192 : 256; }
+constexpr int stencil_groups(int form, int groups) { return form == ST_WIDE ? 4 * groups : groups; }
+// links and coefficient pairs a workgroup shares
+template <typename T, int ST>
+struct ForceShare {
+    T2<T> ol[4][6][kXW];
+    T2<T> tp[6][4][64];
+};
+template <typename T>
+struct ForceShare<T, ST_WIDE> {
+    T2<T> tp[2][4][64];
+};
+// The workgroup's waves, with the site and U_mu(x) they work on, and TA(U_mu Sigma_mu) in c; false for the
+// waves and lanes that have nothing to store.
+template <int ST, typename T>
+__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, T c[8]) {
+    __shared__ ForceShare<T, ST> sh;
+    int x[4];
+    if constexpr (ST == ST_WIDE) {
+        const unsigned b = xcd_block();
+        const int site = (int)((b >> 2) * 64u + (threadIdx.x & 63u));
+        mu = (int)(b & 3u);
+        s = min(site, g.V - 1);
+        decode(g, s, x);
+        return ta_force_wide<T>(g, U, (unsigned)g.V, s, x, mu, own, sh.tp, c) && site < g.V;
+    } else {
+        const SiteMu sm = site_mu_index(g);
+        mu = sm.mu;
+        s = stencil_site<ST == ST_ROWS>(g, sm);
+        decode(g, s, x);
+        ta_force_xrow<ST == ST_ROWS>(g, U, (unsigned)g.V, s, x, mu, own, sh.ol, sh.tp, c);
+        return in_lattice<ST == ST_ROWS>(g, sm);
+    }
 }
 
 // block sum of a double into partial[blockIdx.x] (fixed order: deterministic)
