@@ -41,11 +41,12 @@ struct gf_ctx {
     double rho = 0.0;
     int smode = GF_STOUT_STORE;
     void* lev[GF_MAX_LEV] = {};  // smeared levels 1..nlev
-    void* Cst[GF_MAX_LEV] = {};  // stored C per level (input level index)
-    void* D = nullptr;
+    void* Qst[GF_MAX_LEV] = {};  // Q coefficients per level (input level index; recompute mode: [0] only)
+    void* G = nullptr;           // Lam of the level being pulled back
+    void* Fl = nullptr;          // its derivative without the far plaquette contributions
+    void* far = nullptr;         // those (3 momentum fields)
+    void* D = nullptr;           // explicit derivative, explicit backward pass (general matrices)
     void* D2 = nullptr;
-    void* G = nullptr;
-    void* G2 = nullptr;  // second Lam buffer (stored-C mode: levels chained across kernels)
     // FP32 bulk: FP64 copies of the links (and smeared levels, ping-pong) for the Hamiltonian
     void* W64[2] = {nullptr, nullptr};
     // FP32 forces over an FP64 state: the links and momenta as held and updated (U holds the links
@@ -278,63 +279,38 @@ double topo_of(int method, const double o[4]) {
 int stout_alloc(gf_ctx* c) {
     for (int l = 0; l < c->nlev; l++) {
         TRY(alloc(c, &c->lev[l], link_bytes(c)));
-        if (c->smode == GF_STOUT_STORE) TRY(alloc(c, &c->Cst[l], mat_bytes(c)));
+        if (l == 0 || c->smode == GF_STOUT_STORE) TRY(alloc(c, &c->Qst[l], mom_bytes(c)));
     }
-    TRY(alloc(c, &c->D, mat_bytes(c)));
-    TRY(alloc(c, &c->D2, mat_bytes(c)));
-    TRY(alloc(c, &c->G, mom_bytes(c)));  // Lam coefficients of the stout backward
-    if (c->smode == GF_STOUT_STORE) TRY(alloc(c, &c->G2, mom_bytes(c)));
+    TRY(alloc(c, &c->G, mom_bytes(c)));
+    TRY(alloc(c, &c->Fl, mom_bytes(c)));
+    TRY(alloc(c, &c->far, 3 * mom_bytes(c)));
     return GF_OK;
 }
 const void* level_in(gf_ctx* c, int l) { return l == 0 ? c->U : c->lev[l - 1]; }
+const void* top_links(gf_ctx* c) { return c->nlev > 0 ? c->lev[c->nlev - 1] : c->U; }
 
-int stout_forward_all(gf_ctx* c) {
+// the smeared levels and, with_q, Q: every level's (stored) or the top one's (recomputed for the others)
+int stout_forward_all(gf_ctx* c, bool with_q = false) {
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
+        const bool stored = c->smode == GF_STOUT_STORE;
         for (int l = 0; l < c->nlev; l++)
             HIPCHK(c, launch_stout_forward<T>(c->geo, (const T*)level_in(c, l), (T*)c->lev[l],
-                                              c->smode == GF_STOUT_STORE ? (T*)c->Cst[l] : nullptr, c->rho,
-                                              c->stream));
+                                              with_q && (stored || l == c->nlev - 1) ? (T*)c->Qst[stored ? l : 0]
+                                                                                     : nullptr,
+                                              c->rho, c->stream));
         return GF_OK;
     });
 }
 
-// D (dS/dU of the top level) -> D holds dS/dU_bare afterwards; or, with fmode FORCE_STORE /
-// FORCE_KICK, the last (thin-link) level forms the force from dS/dU_bare instead of storing it:
-// F = -(1/3) TA(U dS/dU_bare) into FP, or FP += eps F.  from_dsdu: D is not given, dS/dU of the top
-// level for the plaquette action with coefficient coeff is formed first.  With stored C every level
-// boundary is one kernel (the stencil half of level l chained with the site-local half of level
-// l - 1), and dS/dU is chained into the top level's site-local half.
-const void* top_links(gf_ctx* c) { return c->nlev > 0 ? c->lev[c->nlev - 1] : c->U; }
-
-int stout_backward_all(gf_ctx* c, int fmode = -1, void* FP = nullptr, double eps = 0.0, double eps_u = 0.0,
-                       bool from_dsdu = false, double coeff = 0.0) {
+// explicit backward pass: D (dS/dU of the top level) -> D holds dS/dU_bare
+int stout_backward_all(gf_ctx* c) {
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        const int top = c->nlev - 1;
-        if (c->smode != GF_STOUT_STORE) {
-            if (from_dsdu) HIPCHK(c, launch_dsdu<T>(c->geo, (const T*)top_links(c), coeff, (T*)c->D, c->stream));
-            for (int l = top; l >= 0; l--) {
-                HIPCHK(c, launch_stout_backward<T>(c->geo, (const T*)level_in(c, l), nullptr, (const T*)c->D, (T*)c->D2,
-                                                   (T*)c->G, c->rho, c->stream, l == 0 ? fmode : -1, (T*)FP, eps,
-                                                   (T*)c->Ualt, eps_u, (double*)c->U64));
-                std::swap(c->D, c->D2);
-            }
-            return GF_OK;
-        }
-        T* const lam[2] = {(T*)c->G, (T*)c->G2};
-        if (from_dsdu)
-            HIPCHK(c, launch_dsdu_chain<T>(c->geo, (const T*)top_links(c), coeff, (const T*)level_in(c, top),
-                                           (const T*)c->Cst[top], (T*)c->D2, lam[top & 1], c->stream));
-        else
-            HIPCHK(c, launch_stout_back_local<T>(c->geo, (const T*)level_in(c, top), (const T*)c->Cst[top],
-                                                 (const T*)c->D, (T*)c->D2, lam[top & 1], c->rho, c->stream));
-        for (int l = top; l >= 1; l--)
-            HIPCHK(c, launch_stout_back_chain<T>(c->geo, (const T*)level_in(c, l), lam[l & 1], (T*)c->D2, c->rho,
-                                                 (const T*)level_in(c, l - 1), (const T*)c->Cst[l - 1],
-                                                 lam[(l - 1) & 1], c->stream));
-        HIPCHK(c, launch_stout_back_stencil<T>(c->geo, (const T*)level_in(c, 0), lam[0], (T*)c->D2, c->rho, c->stream,
-                                               fmode, (T*)FP, eps, (T*)c->Ualt, eps_u, (double*)c->U64));
+        const T* in[GF_MAX_LEV];
+        for (int l = 0; l < c->nlev; l++) in[l] = (const T*)level_in(c, l);
+        HIPCHK(c, launch_stout_backward<T>(c->geo, in, c->nlev, (T*)c->D, (T*)c->D2, (T*)c->G, (T*)c->Fl, c->rho,
+                                           c->stream));
         std::swap(c->D, c->D2);
         return GF_OK;
     });
@@ -345,12 +321,39 @@ int stout_backward_all(gf_ctx* c, int fmode = -1, void* FP = nullptr, double eps
 // momenta and links of an FP64 state (Ualt: the updated links rounded to float)
 // into_force: FORCE_KICK into the force field F instead of the momenta (F += eps force)
 int stout_force_impl(gf_ctx* c, double coeff, int mode, double eps, double eps_u = 0.0, bool into_force = false) {
-    TRY(stout_forward_all(c));
-    // the thin-link level's stencil kernel forms the force from dS/dU_bare
+    TRY(stout_forward_all(c, true));
     void* target = (mode == FORCE_STORE || into_force) ? (void*)c->F
                    : (mode == FORCE_KICK_S64 || mode == FORCE_KICK_EXP_S64) ? c->P64
                                                                           : (void*)c->P;
-    return stout_backward_all(c, mode, target, eps, eps_u, true, coeff);
+    return dispatch(c, [&](auto* tag) -> int {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        // Q of level l: kept by the forward pass, or formed again from the level's links
+        const int top = c->nlev - 1;
+        auto q_of = [&](int l, const T** q) -> int {
+            const bool stored = c->smode == GF_STOUT_STORE;
+            *q = (const T*)c->Qst[stored ? l : 0];
+            if (!stored && l != top)
+                HIPCHK(c, launch_stout_forward<T>(c->geo, (const T*)level_in(c, l), nullptr, (T*)c->Qst[0], c->rho,
+                                                  c->stream));
+            return GF_OK;
+        };
+        const T* q = nullptr;
+        TRY(q_of(top, &q));
+        HIPCHK(c, launch_stout_top<T>(c->geo, (const T*)top_links(c), coeff, q, (T*)c->G, (T*)c->Fl, c->stream));
+        for (int l = top; l >= 0; l--) {
+            HIPCHK(c, launch_stout_pair<T>(c->geo, (const T*)level_in(c, l), (const T*)c->G, (T*)c->Fl, (T*)c->far,
+                                           c->rho, c->stream));
+            if (l > 0) {
+                TRY(q_of(l - 1, &q));
+                HIPCHK(c, launch_stout_gather<T>(c->geo, (const T*)c->far, (T*)c->Fl, c->rho, q, (T*)c->G, c->stream));
+            } else {
+                HIPCHK(c, launch_stout_gather<T>(c->geo, (const T*)c->far, (T*)c->Fl, c->rho, nullptr, nullptr, c->stream,
+                                                 mode, (const T*)c->U, (T*)target, eps, (T*)c->Ualt, eps_u,
+                                                 (double*)c->U64));
+            }
+        }
+        return GF_OK;
+    });
 }
 
 // ---- FP32 forces over an FP64 MD state ---------------------------------------------------
@@ -560,12 +563,12 @@ int gf_destroy(gf_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void** bufs[] = {&c->U,   &c->Ualt, &c->Ubak, &c->P,      &c->F,      &c->A,   &c->D,   &c->D2,
-                     &c->G,   &c->G2,   &c->W64[0], &c->W64[1], &c->U64, &c->P64, &c->U64bak};
+                     &c->G,   &c->Fl,   &c->far, &c->W64[0], &c->W64[1], &c->U64, &c->P64, &c->U64bak};
     for (void** b : bufs)
         if (*b) (void)hipFree(*b);
     for (int l = 0; l < GF_MAX_LEV; l++) {
         if (c->lev[l]) (void)hipFree(c->lev[l]);
-        if (c->Cst[l]) (void)hipFree(c->Cst[l]);
+        if (c->Qst[l]) (void)hipFree(c->Qst[l]);
     }
     if (c->staging) (void)hipFree(c->staging);
     if (c->partial) (void)hipFree(c->partial);
@@ -1070,21 +1073,20 @@ int gf_stout_config(gf_ctx* c, int nlev, double rho, int mode) {
     if (mode != GF_STOUT_STORE && mode != GF_STOUT_RECOMPUTE && mode != GF_STOUT_AUTO)
         return fail(c, GF_EINVAL, "unknown stout mode %d", mode);
     if (mode == GF_STOUT_AUTO) {
-        // bytes still to allocate for levels, derivatives and (if stored) C per level
+        // bytes still to allocate for levels, backward buffers and (if stored) Q per level
         size_t free_b = 0, total_b = 0;
         HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
-        size_t need_levels = 0, need_c = 0;
+        size_t need_levels = 0, need_q = 0;
         for (int l = 0; l < nlev; l++) {
             if (!c->lev[l]) need_levels += link_bytes(c);
-            if (!c->Cst[l]) need_c += mat_bytes(c);
+            if (!c->Qst[l]) need_q += mom_bytes(c);
         }
-        need_c += c->G2 ? 0 : mom_bytes(c);
-        need_levels += (c->D ? 0 : mat_bytes(c)) + (c->D2 ? 0 : mat_bytes(c)) + (c->G ? 0 : mom_bytes(c));
-        mode = (double)(need_levels + need_c) * 1.1 <= (double)free_b ? GF_STOUT_STORE : GF_STOUT_RECOMPUTE;
+        need_levels += (c->G ? 0 : mom_bytes(c)) + (c->Fl ? 0 : mom_bytes(c)) + (c->far ? 0 : 3 * mom_bytes(c));
+        mode = (double)(need_levels + need_q) * 1.1 <= (double)free_b ? GF_STOUT_STORE : GF_STOUT_RECOMPUTE;
     }
-    // release stored C of a previous store-mode configuration if no longer needed
+    // release the levels' Q of a previous store-mode configuration if no longer needed
     for (int l = 0; l < GF_MAX_LEV; l++)
-        if (l >= nlev || mode != GF_STOUT_STORE) release(c, &c->Cst[l], mat_bytes(c));
+        if (l >= nlev || (l > 0 && mode != GF_STOUT_STORE)) release(c, &c->Qst[l], mom_bytes(c));
     for (int l = nlev; l < GF_MAX_LEV; l++) release(c, &c->lev[l], link_bytes(c));
     c->nlev = nlev;
     c->rho = rho;
@@ -1113,6 +1115,8 @@ int gf_stout_backward(gf_ctx* c, const double* dout_ref, double* din_ref) {
     NOT_S64(c, "back_prop");
     if (c->nlev == 0) return fail(c, GF_ESTATE, "no stout levels configured");
     if (!dout_ref || !din_ref) return fail(c, GF_EINVAL, "null derivative buffer");
+    TRY(alloc(c, &c->D, mat_bytes(c)));
+    TRY(alloc(c, &c->D2, mat_bytes(c)));
     TRY(upload_linkfield(c, c->D, dout_ref, true));
     TRY(stout_backward_all(c));
     return download_linkfield(c, c->D, din_ref, true);

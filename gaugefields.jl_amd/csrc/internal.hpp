@@ -48,6 +48,39 @@ enum ForceMode { FORCE_STORE = 0, FORCE_KICK = 1, FORCE_KICK_EXP = 2, FORCE_KICK
 // FORCE_KICK_S64 / FORCE_KICK_EXP_S64 (FP32 kernels over an FP64 MD state): the FP32 force kicks the
 // FP64 momenta, and the FP64 links are updated in place, their float rounding written to Unew
 
+// What a force kernel does with fac * c, c = TA coefficients of a link (MODE: ForceMode; link() is U_mu(s),
+// read only by the modes that update it)
+template <typename T, int MODE, typename L>
+__device__ __forceinline__ void force_out(T c[8], L&& link, unsigned V, int mu, int s, T* __restrict__ FP,
+                                          T* __restrict__ Unew, double fac, double eps_u, double eps_p,
+                                          double* __restrict__ U64) {
+    if constexpr (MODE == FORCE_KICK_S64 || MODE == FORCE_KICK_EXP_S64) {
+        double* P64 = reinterpret_cast<double*>(FP);
+        double p[8];
+        ldp<double, GF_LD_NT>(P64, V, mu, s, p);
+#pragma unroll
+        for (int a = 0; a < 8; a++) p[a] = fma(eps_p, (double)scale1(fac, c[a]), p[a]);
+        stp<double, GF_ST_NT>(P64, V, mu, s, p);
+        if constexpr (MODE == FORCE_KICK_EXP_S64) {
+            const M3<double> un = exp_coeffs_times(p, eps_u, ldu<double, GF_LD_NT>(U64, V, mu, s));
+            stu<double, GF_ST_NT>(U64, V, mu, s, un);
+            stu<T, GF_ST_NT>(Unew, V, mu, s, round_link<T>(un));
+        }
+    } else if constexpr (MODE == FORCE_STORE) {
+#pragma unroll
+        for (int a = 0; a < 8; a++) c[a] = scale1(fac, c[a]);
+        stp<T, GF_ST_NT>(FP, V, mu, s, c);
+    } else {
+        const M3<T> u = MODE == FORCE_KICK_EXP ? link() : M3<T>{};
+        T p[8];
+        ldp<T, GF_LD_NT>(FP, V, mu, s, p);
+#pragma unroll
+        for (int a = 0; a < 8; a++) p[a] = fma1(fac, c[a], p[a]);
+        stp<T, GF_ST_NT>(FP, V, mu, s, p);
+        if constexpr (MODE == FORCE_KICK_EXP) stu<T, GF_ST_NT>(Unew, V, mu, s, exp_coeffs_times(p, eps_u, u));
+    }
+}
+
 // ---- k_gauge.hip ----
 // dst = src, bytes a multiple of 16 (streaming copy: the measured HBM ceiling)
 hipError_t launch_stream_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
@@ -116,40 +149,32 @@ template <typename T>
 hipError_t launch_heatbath(const Geo& g, T* U, int mode, double beta, unsigned long long seed,
                            unsigned long long sweep, int itmax, double* partial, double* failures, hipStream_t st);
 
-// ---- k_flow.hip ----
+// ---- k_flow_stout.hip ----
 // A = alpha * TA(W V^dag) + beta * A ; Wout = exp(A) W
 template <typename T>
 hipError_t launch_flow_stage(const Geo& g, const T* W, T* Wout, T* A, double alpha, double beta,
                              hipStream_t st);
 
-// ---- k_stout.hip ----
+// one smearing level: the smeared links (Uout) and / or the coefficients of Q (Qst); null: not wanted
 template <typename T>
-hipError_t launch_stout_forward(const Geo& g, const T* Uin, T* Uout, T* Cst, double rho, hipStream_t st);
+hipError_t launch_stout_forward(const Geo& g, const T* Uin, T* Uout, T* Qst, double rho, hipStream_t st);
+// the backward pass of a stout force in the algebra (k_flow_stout.hip): F' of the top links and the top
+// level's site-local step: Lam into Lc, Floc into Fl
 template <typename T>
-// Lc: scratch momentum-layout field (the 8 su(3) coefficients of Lam per link).
-// fmode < 0: Din = dS/dU_in.  fmode = FORCE_STORE / FORCE_KICK / FORCE_KICK_EXP (the thin-link
-// level of a stout force, test/HMCstout_test_nowing.jl:99-118): Din is not stored; FP = -(1/3)
-// TA(U_in Din), or FP += eps of that, and with FORCE_KICK_EXP also Unew = exp(eps_u FP) U_in.
-hipError_t launch_stout_backward(const Geo& g, const T* Uin, const T* Cst, const T* Dout, T* Din, T* Lc,
-                                 double rho, hipStream_t st, int fmode = -1, T* FP = nullptr, double eps = 0.0,
-                                 T* Unew = nullptr, double eps_u = 0.0, double* U64 = nullptr);
-// the site-local half of the stout backward alone (Cst null: C recomputed)
+hipError_t launch_stout_top(const Geo& g, const T* Utop, double coeff, const T* Qst, T* Lc, T* Fl, hipStream_t st);
+// the plaquettes of a level (U its input links): near contributions added to Fl, far ones (3 momentum fields)
 template <typename T>
-hipError_t launch_stout_back_local(const Geo& g, const T* Uin, const T* Cst, const T* Dout, T* Din, T* Lc, double rho,
-                                   hipStream_t st);
-// the stencil half of the stout backward alone (fmode as above)
+hipError_t launch_stout_pair(const Geo& g, const T* U, const T* Lc, T* Fl, T* far, double rho, hipStream_t st);
+// F of the level's input links; fmode < 0: the site-local step of the level below (Qst its Q) into Lc
+// and Fl; otherwise the force -(1/3) F as launch_force's modes, U the thin links
 template <typename T>
-hipError_t launch_stout_back_stencil(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, hipStream_t st,
-                                     int fmode, T* FP, double eps, T* Unew, double eps_u, double* U64 = nullptr);
-// stored-C mode: the stencil half of level l (Uin, Lc; Din in: its site-local part) chained with
-// the site-local half of level l-1 (Uprev, Cprev): Din out = level l-1's site-local part, Lout =
-// Lam_{l-1} (a buffer other than Lc)
+hipError_t launch_stout_gather(const Geo& g, const T* far, T* Fl, double rho, const T* Qst, T* Lc, hipStream_t st,
+                               int fmode = -1, const T* U = nullptr, T* FP = nullptr, double eps_p = 0.0,
+                               T* Unew = nullptr, double eps_u = 0.0, double* U64 = nullptr);
+// explicit backward pass of nlev levels (Uin[l] the input links of level l): D2 = dS/dU_bare from D = dS/dU
+// of the top level (general matrix fields); Lc, Lc2: scratch momentum fields
 template <typename T>
-hipError_t launch_stout_back_chain(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, const T* Uprev,
-                                   const T* Cprev, T* Lout, hipStream_t st);
-// dS/dU of the top level (Utop, coeff) chained with the top level's site-local half (Uin, Cst)
-template <typename T>
-hipError_t launch_dsdu_chain(const Geo& g, const T* Utop, double coeff, const T* Uin, const T* Cst, T* Din, T* Lout,
-                             hipStream_t st);
+hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, int nlev, T* D, T* D2, T* Lc, T* Lc2, double rho,
+                                 hipStream_t st);
 
 }  // namespace gf

@@ -1,7 +1,30 @@
 // k_flow_stout.hip -- Luscher RK3 Wilson-flow stage, stout smearing forward and backward.
+#include <utility>
+
 #include "internal.hpp"
 
 namespace gf {
+
+// the 8 coefficients of a link in a workgroup's LDS (an array [..][4][..] of pairs)
+template <typename T, typename A>
+__device__ __forceinline__ void put_c8(A* a, int k, int l, const T c[8]) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        T2<T> v;
+        v.x = c[2 * e];
+        v.y = c[2 * e + 1];
+        a[k][e][l] = v;
+    }
+}
+template <typename T, typename A>
+__device__ __forceinline__ void get_c8(const A* a, int k, int l, T c[8]) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const T2<T> v = a[k][e][l];
+        c[2 * e] = v.x;
+        c[2 * e + 1] = v.y;
+    }
+}
 
 // ---------------------------------------------------------------------------
 // K7: one RK3 stage (flow!, gradientflow.jl:171-238, in the low-storage form):
@@ -36,32 +59,225 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
 
 // ---------------------------------------------------------------------------
 // K5: stout forward level (forward!, stout_fast.jl:250-274; calc_C! :603-624)
-//   C_mu = rho V_mu = rho Sigma_mu^dag,  Q_mu = TA(C_mu U_mu^dag),  Uout_mu = exp(Q_mu) U_mu
-// STORE keeps C_mu for the backward pass.
+//   C_mu = rho V_mu = rho Sigma_mu^dag,  Q_mu = TA(C_mu U_mu^dag) = -rho TA(U_mu Sigma_mu),
+//   Uout_mu = exp(Q_mu) U_mu
+// so the level is the force kernel's stencil with a link update on top (32^4 FP64: 0.50 ms when it formed
+// the whole staple sum and stored C).  WHAT: STOUT_LINKS the smeared links, STOUT_Q the 8 coefficients of
+// Q_mu, which are all the backward pass of a force needs of the level besides its links.
 // ---------------------------------------------------------------------------
-template <typename T, bool STORE, bool ROWS>
-__global__ __launch_bounds__(kBlock) void k_stout_forward(Geo g, const T* __restrict__ Uin, T* __restrict__ Uout,
-                                                          T* __restrict__ Cst, double rho) {
-    __shared__ T2<T> xs[6][6][64];
+enum { STOUT_LINKS = 1, STOUT_Q = 2 };
+template <typename T, int WHAT, int ST>
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_forward(
+    Geo g, const T* __restrict__ Uin, T* __restrict__ Uout, T* __restrict__ Qst, double rho) {
+    int s, mu;
+    R6<T> own;
+    T c[8];
+    if (!ta_force<ST, T>(g, Uin, s, mu, own, c)) return;
+    const unsigned V = g.V;
+    if constexpr (WHAT & STOUT_LINKS) stu<T, GF_ST_NT>(Uout, V, mu, s, exp_coeffs_times(c, -rho, full_of(own)));
+    if constexpr (WHAT & STOUT_Q) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] = scale1(-rho, c[k]);
+        stp<T, GF_ST_NT>(Qst, V, mu, s, c);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Backward pass of a stout force.  The action depends on a level's links only through the group, so
+// what a level hands down is not dS/dU (18 reals) but F = TA(U dS/dU) (8), and what it keeps is Q (8)
+// instead of C (18).  Per level, from F' of its output links:
+//   site-local (stout_local): Lam = derivative with respect to Q, Floc = derivative at fixed Q
+//   staples: dQ_mu(x) = -rho dTA(U_mu Sigma_mu); summed over links, sum Re tr(Lam dQ) is -rho d of
+//     sum over plaquettes of Re tr(Z P),  P = U_a(z) U_b(z+a) U_a(z+b)^dag U_b(z)^dag  (a < b),
+//     Z = Lam_a + G - G' - Lam_b,  G = U_a Lam_b(z+a) U_a^dag,  G' = U_b Lam_a(z+b) U_b^dag,
+//   so each plaquette gives its four links
+//     U_a(z):    TA(P Z + G P - P G)          U_b(z+a): U_a^dag TA(P Z) U_a
+//     U_b(z):   -TA(Z P + G' P - P G')        U_a(z+b): -U_b^dag TA(Z P) U_b
+//   times -rho.
+// k_stout_pair evaluates every plaquette once: the sums at the near links (z) are added to Floc, the two
+// far ones are stored at z (3 momentum-shaped fields: field j of direction mu holds the contribution
+// to U_mu(z + b), b = j + (j >= mu)); k_stout_gather reads those back at z = y - b and goes on to the
+// next level's site-local step or to the force.  The start of the chain, F' of the top level (coeff
+// TA(U Sigma)) and its site-local step, is k_stout_top.
+// (Replaces a gather that evaluated every plaquette once per link, 3258 instead of 1390 x 6/4 FMAs per
+// link and four times the loads, and carried dS/dU and C.)
+// ---------------------------------------------------------------------------
+template <typename T, int ST>
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_top(
+    Geo g, const T* __restrict__ Utop, double coeff, const T* __restrict__ Qst, T* __restrict__ Lc,
+    T* __restrict__ Fl) {
+    int s, mu;
+    R6<T> own;
+    T c[8];
+    if (!ta_force<ST, T>(g, Utop, s, mu, own, c)) return;
+    const unsigned V = g.V;
+    T q[8], lam[8], fl[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) c[k] = scale1(coeff, c[k]);
+    ldp<T, GF_LD_NT>(Qst, V, mu, s, q);
+    stout_local(q, c, lam, fl);
+    stp(Lc, V, mu, s, lam);
+    stp(Fl, V, mu, s, fl);
+}
+
+// One workgroup = 64 sites, NW wavefronts for the six pairs (a, b).  NW = 4: two waves take two, another
+// two in every other workgroup; three workgroups fit a CU.  (With six waves a CU holds one workgroup: its
+// first two SIMDs get two waves of 168 VGPRs and have no room for the next one's two.  32^4 FP64: 0.79
+// against 0.64 ms.)  NW = 6 on small lattices, one pair each.  The waves work by themselves (what three
+// pairs of a site share comes from L1) up to one exchange in LDS of the near contributions.  Three waves
+// per SIMD are too few to hide memory behind each other, so a wave asks for a pair's inputs at once: the
+// four links and the site's two Lam into registers, the neighbours' Lam straight into LDS, where the near
+// contributions will go.  ROWS: the far contribution to U_b(z + x) of the pairs (0, b) goes to a site of
+// the workgroup and is added to the near ones there, a quarter of the far fields less.
+template <typename T, bool ROWS, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_pair(
+    Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Fl, T* __restrict__ far, double rho) {
+    __shared__ C8Lds<T> near_[12];
     const SiteMu sm = site_mu_index(g);
-    const int mu = sm.mu;
-    const int s = stencil_site<ROWS>(g, sm);
+    const int w = sm.mu, s = stencil_site<ROWS>(g, sm);
+    const int lane = (int)(threadIdx.x & 63u);
+    const unsigned V = g.V;
+    int x[4], fw[4];
+    decode(g, s, x);
+#pragma unroll
+    for (int d = 0; d < 4; d++) fw[d] = s + dlt(g, x, d, 1);
+    const int first = NW == 4 ? w ^ (int)((blockIdx.x >> 2) & 2u) : w;
+#pragma unroll 1
+    for (int p = first; p < 6; p += NW) {
+        const int a = p < 3 ? 0 : (p < 5 ? 1 : 2), b = p < 3 ? p + 1 : (p < 5 ? p - 1 : 3);
+        const int sa = sel4(a, fw[0], fw[1], fw[2], fw[3]), sb = sel4(b, fw[0], fw[1], fw[2], fw[3]);
+        M3<T> P;
+        Herm<T> G, Gp, Z;
+        {
+            const R6<T> nb = ldr(U, V, b, (unsigned)sa), na = ldr(U, V, a, (unsigned)sb);
+            const R6<T> ra = ldr(U, V, a, (unsigned)s), rb = ldr(U, V, b, (unsigned)s);
+            T ca[8], cb[8];
+            ldp(Lc, V, a, (unsigned)s, ca);
+            ldp(Lc, V, b, (unsigned)s, cb);
+            ldp_lds(Lc, V, a, (unsigned)sb, &near_[2 * p]);
+            ldp_lds(Lc, V, b, (unsigned)sa, &near_[2 * p + 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            P = su3_mul(ra, su3_mul_nd(nb, full_of(na)));
+#pragma unroll
+            for (int k = 0; k < 8; k++) ca[k] -= cb[k];
+            Z = herm_of_coeffs(ca);
+            const M3<T> ub = full_of(rb);
+            P = su3_mul_nd(rows_of(P), ub);
+            wait_lds_loads();
+            T h[8];
+            get_c8(&near_[2 * p], lane, h);
+            Gp = herm_conj(ub, herm_of_coeffs(h));
+            get_c8(&near_[2 * p + 1], lane, h);
+            G = herm_conj(full_of(ra), herm_of_coeffs(h));
+        }
+        T fa[8], fb[8];  // TA(i Z P), TA(i P Z)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            Z.d[k] += G.d[k] - Gp.d[k];
+            Z.u[k].r += G.u[k].r - Gp.u[k].r;
+            Z.u[k].i += G.u[k].i - Gp.u[k].i;
+        }
+        ta_coeffs_i(mul_mh(P, Z), fb);
+        ta_coeffs_i(mul_hm(Z, P), fa);
+        T c[8];
+        ta_coeffs_i(herm_comm(G, P), c);
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] += fb[k];
+        put_c8(&near_[2 * p], lane, c);
+        ta_coeffs_i(herm_comm(Gp, P), c);  // TA(i (P G' - G' P)) is minus this
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] = -(c[k] + fa[k]);
+        // the far links; U_a and U_b again from L1 rather than held
+        int s1 = s;
+        asm volatile("" : "+v"(s1));
+        const R6<T> ra = ldr(U, V, a, (unsigned)s1), rb = ldr(U, V, b, (unsigned)s1);
+        T t[8];
+        coeffs_of_herm(herm_conj_dag(full_of(ra), herm_of_coeffs(fb)), t);
+        if (ROWS && a == 0) {
+            // the contribution to lane x + 1, through this wave's place in LDS (its lanes in step)
+            put_c8(&near_[2 * p + 1], lane, t);
+            __builtin_amdgcn_wave_barrier();
+            get_c8(&near_[2 * p + 1], xrow_of<true>(g, s, x[0], lane).m, t);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < 8; k++) c[k] += t[k];
+        } else if (in_lattice<ROWS>(g, sm)) {
+            stp<T, GF_ST_NT>(far + (size_t)a * 32 * V, V, b, (unsigned)s, t);
+        }
+        put_c8(&near_[2 * p + 1], lane, c);
+#pragma unroll
+        for (int k = 0; k < 8; k++) fa[k] = -fa[k];
+        coeffs_of_herm(herm_conj_dag(full_of(rb), herm_of_coeffs(fa)), t);
+        if (in_lattice<ROWS>(g, sm)) stp<T, GF_ST_NT>(far + (size_t)(b - 1) * 32 * V, V, a, (unsigned)s, t);
+    }
+    T f[8];
+    if (w < 4) ldp<T, GF_LD_NT>(Fl, V, w, (unsigned)s, f);
+    __syncthreads();  // every pair's near contributions are in LDS
+    if (w < 4 && in_lattice<ROWS>(g, sm)) {
+        T c[8], t[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] = T(0);
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int nu = j + (j >= w ? 1 : 0);
+            get_c8(&near_[2 * pair_index(w < nu ? w : nu, w < nu ? nu : w) + (w < nu ? 0 : 1)], lane, t);
+#pragma unroll
+            for (int k = 0; k < 8; k++) c[k] += t[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) f[k] = fma1(-rho, c[k], f[k]);
+        stp<T, GF_ST_NT>(Fl, V, w, (unsigned)s, f);
+    }
+}
+
+// F of a level's input links: Floc and near contributions (Fl, as k_stout_pair left it) plus the far
+// contributions of the three plaquettes below.  OUT < 0: the site-local step of the next level down (Qst its
+// Q), Lam and Floc in place.  Otherwise the thin-link level of a force, -(1/3) F, as k_force's modes
+// (test/HMCstout_test_nowing.jl:99-118).  Streaming: a thread per link; workgroups of one wave on small
+// lattices, to reach more CUs.
+template <typename T, int OUT, bool ROWS>
+__global__ __launch_bounds__(kBlock) void k_stout_gather(Geo g, const T* __restrict__ far, T* __restrict__ Fl,
+                                                         double rho, const T* __restrict__ Qst, T* __restrict__ Lc,
+                                                         const T* __restrict__ U, T* __restrict__ FP,
+                                                         T* __restrict__ Unew, double fac, double eps_u, double eps_p,
+                                                         double* __restrict__ U64) {
+    int s, mu;
+    if (blockDim.x == 64u) {
+        const unsigned b = xcd_block();
+        s = (int)((b >> 2) * 64u + threadIdx.x);
+        mu = (int)(b & 3u);
+    } else {
+        const SiteMu sm = site_mu_index(g);
+        s = sm.s;
+        mu = sm.mu;
+    }
+    if (s >= g.V) return;
+    const unsigned V = g.V;
     int x[4];
     decode(g, s, x);
-    const unsigned V = g.V;
-    R6<T> own;
-    const M3<T> sig = staple_sigma_shared(g, Uin, V, s, x, mu, own, xs);
-    if (!in_lattice<ROWS>(g, sm)) return;
-    const M3<T> u = full_of(own);
-    if constexpr (std::is_same<T, float>::value) {
-        // C = rho Sigma^dag rounded once (the backward pass reads this C), Q and exp(Q) U in double
-        const M3<T> C = round_link<T>(scal(rho, dag(to_f64(sig))));
-        stu<T, GF_ST_NT>(Uout, V, mu, s, exp_antiherm_times(ta_mat(mul_nd(to_f64(C), to_f64(u))), u));
-        if (STORE) stm<T, GF_ST_NT>(Cst, V, mu, s, C);
+    T f[8], c[8], t[3][8];
+    ldp<T, GF_LD_NT>(Fl, V, mu, (unsigned)s, f);
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        if (ROWS && j == 0 && mu > 0) continue;  // the x-neighbour's is in Fl
+        const int nu = j + (j >= mu ? 1 : 0);
+        ldp(far + (size_t)j * 32 * V, V, mu, (unsigned)(s + dlt(g, x, nu, -1)), t[j]);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        c[k] = t[1][k] + t[2][k];
+        if (!ROWS || mu == 0) c[k] += t[0][k];
+        c[k] = fma1(-rho, c[k], f[k]);
+    }
+    if constexpr (OUT < 0) {
+        T q[8], lam[8], fl[8];
+        ldp<T, GF_LD_NT>(Qst, V, mu, (unsigned)s, q);
+        stout_local(q, c, lam, fl);
+        stp(Lc, V, mu, (unsigned)s, lam);
+        stp(Fl, V, mu, (unsigned)s, fl);
     } else {
-        const M3<T> C = scal(rho, dag(sig));
-        stu<T, GF_ST_NT>(Uout, V, mu, s, exp_antiherm_times(ta_mat(mul_nd(C, u)), u));
-        if (STORE) stm<T, GF_ST_NT>(Cst, V, mu, s, C);
+        force_out<T, OUT>(c, [&] { return ldu<T, GF_LD_NT>(U, V, mu, (unsigned)s); }, V, mu, s, FP, Unew, fac, eps_u,
+                          eps_p, U64);
     }
 }
 
@@ -70,66 +286,48 @@ __global__ __launch_bounds__(kBlock) void k_stout_forward(Geo g, const T* __rest
 //   Din_mu = Dout_mu e^{Q_mu} + (Lam_mu C_mu)^dag,   Lam_mu = TA(CdexpQdQ(U_mu Dout_mu, Q_mu))
 // Lam_mu (traceless anti-Hermitian) is stored as its 8 su(3) coefficients; the staple part
 // uses G_mu = U_mu^dag Lam_mu (= dS/dC_mu) without storing it.
-// STORED reads C_mu from the forward pass, otherwise it is recomputed from the staples.
+// C_mu is formed from the staples again.  (Used by the explicit backward pass, whose dS/dU_in is wanted
+// as a matrix; the forces take the algebra form above.)
 // ---------------------------------------------------------------------------
 // A 3x3 field element kept in the wave's own LDS slice between two uses (each lane reads back what
 // it wrote: no barrier), instead of being held in registers or read from memory twice.
 template <typename T>
-using MStage = T2<T> (*)[9][64];
+using MStage = T2<T> (*)[64];
 template <typename T>
-__device__ __forceinline__ M3<T> stage_m3(MStage<T> st, int mu, int lane, const M3<T>& m) {
+__device__ __forceinline__ M3<T> stage_m3(MStage<T> st, int lane, const M3<T>& m) {
 #pragma unroll
     for (int e = 0; e < 9; e++) {
         T2<T> v;
         v.x = m.m[e].r;
         v.y = m.m[e].i;
-        st[mu][e][lane] = v;
+        st[e][lane] = v;
     }
     return m;
 }
 template <typename T>
-__device__ __forceinline__ M3<T> staged_m3(MStage<T> st, int mu, int lane) {
+__device__ __forceinline__ M3<T> staged_m3(MStage<T> st, int lane) {
     // an opaque copy of the index, so that the compiler reads LDS rather than forwarding the
     // stored value (which would keep it live in registers)
     asm volatile("" : "+v"(lane));
     M3<T> m;
 #pragma unroll
     for (int e = 0; e < 9; e++) {
-        const T2<T> v = st[mu][e][lane];
+        const T2<T> v = st[e][lane];
         m.m[e].r = v.x;
         m.m[e].i = v.y;
     }
     return m;
 }
-template <typename T, bool STORED, bool ROWS>
-__global__ __launch_bounds__(kBlock) void k_stout_back_local(Geo g, const T* __restrict__ Uin,
-                                                             const T* __restrict__ Cst, const T* __restrict__ Dout,
-                                                             T* __restrict__ Din, T* __restrict__ Lc, double rho) {
-    __shared__ T2<T> xs[STORED ? 1 : 6][6][64];
-    // Dout_mu and a stored C_mu are used before and after exp_dexp: kept in LDS in between (the
-    // second read from memory missed L2 for a third of the kernel's HBM reads)
-    __shared__ T2<T> dst[4][9][64];
-    __shared__ T2<T> cst[STORED ? 4 : 1][9][64];
-    const SiteMu sm = site_mu_index(g);
-    const int mu = sm.mu;
-    const int lane = (int)(threadIdx.x & 63u);
-    const int s = stencil_site<ROWS>(g, sm);
-    const unsigned V = g.V;
-    M3<T> C;  // recomputed C; a stored C is staged in LDS instead of kept live
-    R6<T> own;
-    if (STORED) {
-        own = ldr<T, GF_LD_NT>(Uin, V, mu, s);
-    } else {  // the same staple evaluation (and rounding) as the forward kernel
-        int x[4];
-        decode(g, s, x);
-        C = round_link<T>(scal(rho, dag(to_f64(staple_sigma_shared(g, Uin, V, s, x, mu, own, xs)))));
-    }
-    if (!in_lattice<ROWS>(g, sm)) return;
+// from the staple sum and the link: Din and Lam of the level (dout() is Dout_mu(s); dst the lane's staging)
+template <typename T, typename D>
+__device__ __forceinline__ void back_local(const M3<T>& sig, const R6<T>& own, D&& dout, T* __restrict__ Din,
+                                           T* __restrict__ Lc, double rho, unsigned V, int mu, int s, int lane,
+                                           MStage<T> dst) {
+    const M3<T> C = round_link<T>(scal(rho, dag(to_f64(sig))));
     M3<T> E, L;
     {
         const M3<T> u = full_of(own);
-        const M3<T> Cq = STORED ? stage_m3<T>(cst, mu, lane, ldm<T, GF_LD_NT>(Cst, V, mu, s)) : C;
-        exp_dexp(ta_mat(mul_nd(Cq, u)), mul(u, stage_m3<T>(dst, mu, lane, ldm<T, GF_LD_NT>(Dout, V, mu, s))), E, L);
+        exp_dexp(ta_mat(mul_nd(C, u)), mul(u, stage_m3<T>(dst, lane, dout())), E, L);
     }
     const M3<T> Lam = ta_mat(L);
     {
@@ -137,9 +335,41 @@ __global__ __launch_bounds__(kBlock) void k_stout_back_local(Geo g, const T* __r
         ta_coeffs(Lam, c);
         stp<T, GF_ST_NT>(Lc, V, mu, s, c);
     }
-    M3<T> D = mul(staged_m3<T>(dst, mu, lane), E);
-    acc_dag(D, mul(Lam, STORED ? staged_m3<T>(cst, mu, lane) : C));
-    stm<T, GF_ST_NT>(Din, V, mu, s, D);
+    M3<T> D2 = mul(staged_m3<T>(dst, lane), E);
+    acc_dag(D2, mul(Lam, C));
+    stm<T, GF_ST_NT>(Din, V, mu, s, D2);
+}
+template <typename T, int ST>
+__global__ __launch_bounds__(stencil_threads(ST)) void k_stout_back_local(Geo g, const T* __restrict__ Uin,
+                                                                          const T* Dout, T* Din, T* __restrict__ Lc,
+                                                                          double rho) {
+    // the staples' exchange, then Dout_mu, which is used before and after exp_dexp: kept in LDS in between
+    __shared__ T2<T> xs[ST == ST_WIDE ? 1 : 6][6][64];
+    __shared__ T2<T> dst[ST == ST_WIDE ? 2 : 4][9][64];
+    const int lane = (int)(threadIdx.x & 63u);
+    const unsigned V = g.V;
+    int s, mu, x[4];
+    R6<T> own;
+    M3<T> sig;
+    bool valid;
+    if constexpr (ST == ST_WIDE) {
+        const WideIndex wi = wide_index(g);
+        s = wi.s;
+        mu = wi.mu;
+        decode(g, s, x);
+        sig = staples_of_plane(g, Uin, V, s, x, mu, wi.j + (wi.j >= mu ? 1 : 0), own);
+        valid = wide_sum(sig, wi.j, dst) && wi.site < g.V;
+    } else {
+        const SiteMu sm = site_mu_index(g);
+        s = stencil_site<ST == ST_ROWS>(g, sm);
+        mu = sm.mu;
+        decode(g, s, x);
+        sig = staple_sigma_shared(g, Uin, V, s, x, mu, own, xs);
+        valid = in_lattice<ST == ST_ROWS>(g, sm);
+    }
+    if (!valid) return;
+    back_local<T>(sig, own, [&] { return ldm<T, GF_LD_NT>(Dout, V, mu, s); }, Din, Lc, rho, V, mu, s, lane,
+                  dst[ST == ST_WIDE ? 0 : mu]);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,18 +443,9 @@ __device__ __forceinline__ void acc_hd(M3<T>& c, const Herm<T>& h, const M3<T>& 
         }
 }
 
-template <typename T>
-__device__ __forceinline__ void lds_c8(XCoefs<T> hl, int d, int l, T c[8]) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const T2<T> v = hl[d][e][l];
-        c[2 * e] = v.x;
-        c[2 * e + 1] = v.y;
-    }
-}
-// Plane b of K6b added into acc.  U_b(y) and Lam_b(y) come from the workgroup's LDS copies (ul, hl);
+// Plane b of K6b added into acc.  SH: U_b(y) and Lam_b(y) come from the workgroup's LDS copies (ul, hl);
 // A0 (a = 0) and B0 (b = 0): the x-neighbour links and Lam at y + 1 and y - 1 (xr) as well.
-template <typename T, bool A0, bool B0>
+template <typename T, bool SH, bool A0, bool B0>
 __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U, const T* __restrict__ Lc, unsigned V,
                                            int y, const int x[4], int a, int b, int ypa, M3<T>& acc, XLinks<T> ul,
                                            XCoefs<T> hl, int lane, const XRow& xr) {
@@ -239,15 +460,16 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
         const R6<T> uby = A0 ? shared_link<T>(ul, b, xr.p) : ldr(U, V, b, y1);                // U_b(y+a)
         const M3<T> X = su3_mul_nd(uby, full_of(B0 ? shared_link<T>(ul, a, xr.p) : ldr(U, V, a, ypb)));  // U_a(y+b)
         T c[8];
-        if (B0) lds_c8<T>(hl, a, xr.p, c);  // Lam_a(y+b)
+        if (B0) get_c8(hl, a, xr.p, c);  // Lam_a(y+b)
         else ldp(Lc, V, a, ypb, c);
         const M3<T> XH = times_i(mul_mh(X, herm_of_coeffs(c)));
-        const M3<T> ub = full_of(shared_link<T>(ul, b, lane));        // U_b(y)
+        const M3<T> ub = full_of(SH ? shared_link<T>(ul, b, lane) : ldr(U, V, b, (unsigned)y));        // U_b(y)
         acc_mul_nd(acc, XH, ub);
         const M3<T> S = su3_mul_nd(rows_of(X), ub);
-        lds_c8<T>(hl, b, lane, c);  // Lam_b(y)
+        if (SH) get_c8(hl, b, lane, c);  // Lam_b(y)
+        else ldp(Lc, V, b, (unsigned)y, c);
         acc_i_mh<T, 1>(acc, S, herm_of_coeffs(c));
-        if (A0) lds_c8<T>(hl, b, xr.p, c);  // Lam_b(y+a)
+        if (A0) get_c8(hl, b, xr.p, c);  // Lam_b(y+a)
         else ldp(Lc, V, b, y1, c);
         acc_i_hm<T, -1>(acc, herm_of_coeffs(c), S);
     }
@@ -258,8 +480,8 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
         const M3<T> ua = full_of(B0 ? shared_link<T>(ul, a, xr.m) : ldr(U, V, a, ymb));  // U_a(y-b)
         T ca[8], cb[8];
         if (B0) {
-            lds_c8<T>(hl, a, xr.m, ca);
-            lds_c8<T>(hl, 0, xr.m, cb);
+            get_c8(hl, a, xr.m, ca);
+            get_c8(hl, 0, xr.m, cb);
         } else {
             ldp(Lc, V, a, ymb, ca);
             ldp(Lc, V, b, ymb, cb);
@@ -287,19 +509,10 @@ __device__ __forceinline__ M3<T> back_stencil_acc(const Geo& g, const T* __restr
         const R6<T> u = ldr(U, V, a, (unsigned)y);
         ldp(Lc, V, a, (unsigned)y, c);
         share_links<ROWS, T>(ul, U, V, a, lane, xr, u);
-        auto put = [&](int l) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                T2<T> v;
-                v.x = c[2 * e];
-                v.y = c[2 * e + 1];
-                hl[a][e][l] = v;
-            }
-        };
-        put(lane);
-        if (xr.halo >= 0) {
+        put_c8(hl, a, lane, c);
+        if (!ROWS && xr.halo >= 0) {
             ldp(Lc, V, a, (unsigned)xr.halo, c);
-            put(64 + lane);
+            put_c8(hl, a, 64 + lane, c);
         }
         __syncthreads();
     }
@@ -307,21 +520,21 @@ __device__ __forceinline__ M3<T> back_stencil_acc(const Geo& g, const T* __restr
     const int ypa = y + dlt(g, x, a, 1);
     if (a == 0) {
 #pragma unroll 1
-        for (int b = 1; b < 4; b++) back_plane<T, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
+        for (int b = 1; b < 4; b++) back_plane<T, true, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
     } else {
-        back_plane<T, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, xr);
+        back_plane<T, true, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, xr);
 #pragma unroll 1
         for (int b = 1; b < 4; b++) {
             if (b == a) continue;
-            back_plane<T, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
+            back_plane<T, true, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
         }
     }
     return acc;
 }
-// Din_a(y) + rho * (staple part): the derivative with respect to the level's input links
+// Din_a(y) + rho * (staple part)
 template <typename T>
-__device__ __forceinline__ M3<T> back_stencil_din(const T* __restrict__ Din, unsigned V, int a, int y, double rho,
-                                                  const M3<T>& acc) {
+__device__ __forceinline__ M3<T> back_din(const T* __restrict__ Din, unsigned V, int a, int y, double rho,
+                                          const M3<T>& acc) {
     M3<T> dn = ldm<T, GF_LD_NT>(Din, V, a, y);
 #pragma unroll
     for (int k = 0; k < 9; k++) {
@@ -330,144 +543,65 @@ __device__ __forceinline__ M3<T> back_stencil_din(const T* __restrict__ Din, uns
     }
     return dn;
 }
+// K6b: Din += rho (staple part).  At most 168 VGPRs (FP64), so that three waves fit per SIMD.
+template <typename T, int ST>
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil(
+    Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho) {
+    const unsigned V = g.V;
+    const int lane = (int)(threadIdx.x & 63u);
+    int y, a, x[4];
+    M3<T> acc;
+    bool valid;
+    if constexpr (ST == ST_WIDE) {
+        __shared__ T2<T> red[2][9][64];
+        const WideIndex wi = wide_index(g);
+        y = wi.s;
+        a = wi.mu;
+        decode(g, y, x);
+        acc = zero3<T>();
+        back_plane<T, false, false, false>(g, U, Lc, V, y, x, a, wi.j + (wi.j >= a ? 1 : 0), y + dlt(g, x, a, 1), acc,
+                                           nullptr, nullptr, lane, XRow{});
+        valid = wide_sum(acc, wi.j, red) && wi.site < g.V;
+    } else {
+        __shared__ T2<T> ul[4][6][kXW];
+        __shared__ T2<T> hl[4][4][kXW];
+        const SiteMu sm = site_mu_index(g);
+        a = sm.mu;
+        y = stencil_site<ST == ST_ROWS>(g, sm);
+        decode(g, y, x);
+        acc = back_stencil_acc<ST == ST_ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl);
+        valid = in_lattice<ST == ST_ROWS>(g, sm);
+    }
+    if (!valid) return;
+    stm<T, GF_ST_NT>(Din, V, a, y, back_din(Din, V, a, y, rho, acc));
+}
 
-// K6b.  At most 168 VGPRs (FP64), so that three waves fit per SIMD.
-// OUT < 0: Din += rho (staple part).  OUT = FORCE_STORE / FORCE_KICK / FORCE_KICK_EXP: the thin-link
-// level of a stout force (test/HMCstout_test_nowing.jl:99-118): Din is not stored but turned into
-// the force FP = -(1/3) TA(U_a(y) Din), or FP += eps of that, in the same kernel; FORCE_KICK_EXP
-// then also writes Unew = exp(eps_u FP) U_a(y) (update_gaugefields!, molecular_dynamics.jl:513-531)
-// to a buffer other than U, which the other threads still read.  OUT = FORCE_KICK_S64 /
-// FORCE_KICK_EXP_S64 (FP32 only): FP is the FP64 momenta, kicked by the force as rounded to float;
-// U64 the FP64 links, U64_a(y) <- exp(eps_u FP) U64_a(y) in place, and Unew its float rounding.
-template <typename T, int OUT, bool ROWS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil(
+// K6b of a level and K6a of the one below (Uprev its input links) in one launch, on small lattices: the
+// three waves form their planes' parts of both stencils.  Lout is another buffer than Lc, whose entries
+// at neighbour sites other workgroups still read.
+template <typename T>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(1))) void k_stout_back_chain_wide(
     Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho,
-    T* __restrict__ FP, double eps, T* __restrict__ Unew, double eps_u, double* __restrict__ U64) {
-    __shared__ T2<T> ul[4][6][kXW];
-    __shared__ T2<T> hl[4][4][kXW];
-    const SiteMu sm = site_mu_index(g);
-    const int a = sm.mu;
-    const int y = stencil_site<ROWS>(g, sm);
-    int x[4];
-    decode(g, y, x);
+    const T* __restrict__ Uprev, T* __restrict__ Lout) {
+    __shared__ T2<T> red[2][2][9][64];
     const unsigned V = g.V;
     const int lane = (int)(threadIdx.x & 63u);
-    const M3<T> acc = back_stencil_acc<ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl);
-    if (!in_lattice<ROWS>(g, sm)) return;
-    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, acc);
-    if constexpr (OUT < 0) {
-        stm<T, GF_ST_NT>(Din, V, a, y, dn);
-    } else {  // the force from the thin-link derivative
-        constexpr double fac = -1.0 / 3.0;
-        const M3<T> ua = full_of(shared_link<T>(ul, a, lane));
-        T c[8];
-        ta_coeffs(mul(ua, dn), c);
-        if constexpr (OUT == FORCE_STORE) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) c[k] = scale1(fac, c[k]);
-            stp<T, GF_ST_NT>(FP, V, a, y, c);
-        } else if constexpr (OUT == FORCE_KICK_S64 || OUT == FORCE_KICK_EXP_S64) {
-            double* P64 = reinterpret_cast<double*>(FP);
-            double p[8];
-            ldp<double, GF_LD_NT>(P64, V, a, y, p);
-#pragma unroll
-            for (int k = 0; k < 8; k++) p[k] = fma(eps, (double)scale1(fac, c[k]), p[k]);
-            stp<double, GF_ST_NT>(P64, V, a, y, p);
-            if constexpr (OUT == FORCE_KICK_EXP_S64) {
-                const M3<double> un = exp_coeffs_times(p, eps_u, ldu<double, GF_LD_NT>(U64, V, a, y));
-                stu<double, GF_ST_NT>(U64, V, a, y, un);
-                stu<T, GF_ST_NT>(Unew, V, a, y, round_link<T>(un));
-            }
-        } else {
-            T p[8];
-            ldp<T, GF_LD_NT>(FP, V, a, y, p);
-            const double f = eps * fac;
-#pragma unroll
-            for (int k = 0; k < 8; k++) p[k] = fma1(f, c[k], p[k]);
-            stp<T, GF_ST_NT>(FP, V, a, y, p);
-            if constexpr (OUT == FORCE_KICK_EXP) stu<T, GF_ST_NT>(Unew, V, a, y, exp_coeffs_times(p, eps_u, ua));
-        }
-    }
-}
-
-// K6a of level l-1 chained after the K6b of level l (stored C): the derivative with respect to
-// level l's input links, Dout_{l-1}(y), is formed in registers by the K6b part and is exactly what
-// the site-local step of level l-1 needs at the same (y, a), so it is neither stored nor read
-// back (1152 B per site fewer per level boundary).  Same arithmetic as k_stout_back_local<T,
-// true, false>: Din_{l-1} = Dout e^Q + (Lam C)^dag into Din (each thread reads then writes only its
-// own element), Lam_{l-1} into Lout (another buffer than Lc, whose entries at neighbour sites the
-// K6b part reads).  Dout and C are staged in the lane's LDS slice between their two uses, in LDS
-// that the K6b part's copies occupied before (one workgroup barrier in between).
-template <typename T>
-__device__ __forceinline__ void back_local_stored(const T* __restrict__ Uin, const T* __restrict__ Cst,
-                                                  const M3<T>& dout, T* __restrict__ Din, T* __restrict__ Lout,
-                                                  unsigned V, int mu, int s, int lane, MStage<T> dst, MStage<T> cst) {
-    M3<T> E, L;
-    {
-        const M3<T> u = full_of(ldr<T, GF_LD_NT>(Uin, V, mu, s));
-        const M3<T> Cq = stage_m3<T>(cst, mu, lane, ldm<T, GF_LD_NT>(Cst, V, mu, s));
-        exp_dexp(ta_mat(mul_nd(Cq, u)), mul(u, stage_m3<T>(dst, mu, lane, dout)), E, L);
-    }
-    const M3<T> Lam = ta_mat(L);
-    {
-        T c[8];
-        ta_coeffs(Lam, c);
-        stp<T, GF_ST_NT>(Lout, V, mu, s, c);
-    }
-    M3<T> D = mul(staged_m3<T>(dst, mu, lane), E);
-    acc_dag(D, mul(Lam, staged_m3<T>(cst, mu, lane)));
-    stm<T, GF_ST_NT>(Din, V, mu, s, D);
-}
-template <typename T>
-constexpr int kChainLds = (int)(2 * 4 * 9 * 64 * sizeof(T2<T>));  // dst + cst; >= ul + hl
-// FP32: three waves per SIMD (at most 168 VGPRs); FP64 holds two (its LDS allows two workgroups per CU)
-template <typename T, bool ROWS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 1))) void k_stout_back_chain(Geo g, const T* __restrict__ U, const T* __restrict__ Lc,
-                                                             T* __restrict__ Din, double rho,
-                                                             const T* __restrict__ Uprev, const T* __restrict__ Cprev,
-                                                             T* __restrict__ Lout) {
-    __shared__ __align__(16) unsigned char smem[kChainLds<T>];
-    static_assert(4 * 10 * kXW * sizeof(T2<T>) <= kChainLds<T>, "ul + hl fit the staging space");
-    XLinks<T> ul = reinterpret_cast<XLinks<T>>(smem);
-    XCoefs<T> hl = reinterpret_cast<XCoefs<T>>(smem + 4 * 6 * kXW * sizeof(T2<T>));
-    MStage<T> dst = reinterpret_cast<MStage<T>>(smem);
-    MStage<T> cst = reinterpret_cast<MStage<T>>(smem + 4 * 9 * 64 * sizeof(T2<T>));
-    const SiteMu sm = site_mu_index(g);
-    const int a = sm.mu;
-    const int y = stencil_site<ROWS>(g, sm);
+    const WideIndex wi = wide_index(g);
+    const int a = wi.mu, b = wi.j + (wi.j >= a ? 1 : 0);
     int x[4];
-    decode(g, y, x);
-    const unsigned V = g.V;
-    const int lane = (int)(threadIdx.x & 63u);
-    const M3<T> dn = back_stencil_din(Din, V, a, y, rho, back_stencil_acc<ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl));
-    __syncthreads();  // every wave is done with ul/hl before the staging reuses them
-    if (in_lattice<ROWS>(g, sm)) back_local_stored<T>(Uprev, Cprev, dn, Din, Lout, V, a, y, lane, dst, cst);
-}
-
-// K2 chained into the K6a of the top level (stored C): dS/dU of the top smeared level, coeff
-// Sigma_mu(y), is Dout of the top level's site-local step at the same (y, mu)
-template <typename T, bool ROWS>
-__global__ __launch_bounds__(kBlock) void k_dsdu_chain(Geo g, const T* __restrict__ Utop, double coeff,
-                                                       const T* __restrict__ Uin, const T* __restrict__ Cst,
-                                                       T* __restrict__ Din, T* __restrict__ Lout) {
-    __shared__ __align__(16) unsigned char smem[kChainLds<T>];
-    static_assert(6 * 6 * 64 * sizeof(T2<T>) <= kChainLds<T>, "xs fits the staging space");
-    XShare<T> xs = reinterpret_cast<XShare<T>>(smem);
-    MStage<T> dst = reinterpret_cast<MStage<T>>(smem);
-    MStage<T> cst = reinterpret_cast<MStage<T>>(smem + 4 * 9 * 64 * sizeof(T2<T>));
-    const SiteMu sm = site_mu_index(g);
-    const int s = stencil_site<ROWS>(g, sm);
-    int x[4];
-    decode(g, s, x);
+    decode(g, wi.s, x);
     R6<T> own;
-    M3<T> sig = staple_sigma_shared(g, Utop, (unsigned)g.V, s, x, sm.mu, own, xs);
+    M3<T> sig = staples_of_plane(g, Uprev, V, wi.s, x, a, b, own);
 #pragma unroll
-    for (int k = 0; k < 9; k++) {
-        sig.m[k].r = scale1(coeff, sig.m[k].r);
-        sig.m[k].i = scale1(coeff, sig.m[k].i);
-    }
-    __syncthreads();  // every wave is done with xs before the staging reuses it
-    if (in_lattice<ROWS>(g, sm)) back_local_stored<T>(Uin, Cst, sig, Din, Lout, (unsigned)g.V, sm.mu, s, (int)(threadIdx.x & 63u), dst, cst);
+    for (int e = 0; e < 9; e++) asm volatile("" : "+v"(sig.m[e].r), "+v"(sig.m[e].i));  // one stencil after the other
+    M3<T> acc = zero3<T>();
+    back_plane<T, false, false, false>(g, U, Lc, V, wi.s, x, a, b, wi.s + dlt(g, x, a, 1), acc, nullptr, nullptr, lane,
+                                       XRow{});
+    const bool first = wide_sum(sig, wi.j, red[0]);
+    wide_sum(acc, wi.j, red[1]);
+    if (!first || wi.site >= g.V) return;
+    back_local<T>(sig, own, [&] { return back_din(Din, V, a, wi.s, rho, acc); }, Din, Lout, rho, V, a, wi.s, lane,
+                  red[0][0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -478,83 +612,106 @@ hipError_t launch_flow_stage(const Geo& g, const T* W, T* Wout, T* A, double alp
     });
     return hipGetLastError();
 }
+// Uout / Qst null: not written (one of them is wanted)
 template <typename T>
-hipError_t launch_stout_forward(const Geo& g, const T* Uin, T* Uout, T* Cst, double rho, hipStream_t st) {
-    const int nb = grid_sites_mu(g.V);
-    if (Cst)
-        by_rows(g, [&](auto rows) { k_stout_forward<T, true, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Uout, Cst, rho); });
-    else
-        by_rows(g, [&](auto rows) { k_stout_forward<T, false, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Uout, nullptr, rho); });
+hipError_t launch_stout_forward(const Geo& g, const T* Uin, T* Uout, T* Qst, double rho, hipStream_t st) {
+    by_form<T>(g, [&](auto f) {
+        const int nb = stencil_groups(f, grid_sites_mu(g.V)), nt = stencil_threads(f);
+        if (Uout && Qst)
+            k_stout_forward<T, STOUT_LINKS | STOUT_Q, decltype(f)::value><<<nb, nt, 0, st>>>(g, Uin, Uout, Qst, rho);
+        else if (Uout)
+            k_stout_forward<T, STOUT_LINKS, decltype(f)::value><<<nb, nt, 0, st>>>(g, Uin, Uout, Qst, rho);
+        else
+            k_stout_forward<T, STOUT_Q, decltype(f)::value><<<nb, nt, 0, st>>>(g, Uin, Uout, Qst, rho);
+    });
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_stout_back_chain(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, const T* Uprev,
-                                   const T* Cprev, T* Lout, hipStream_t st) {
-    by_rows(g, [&](auto rows) { k_stout_back_chain<T, decltype(rows)::value><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, Uin, Lc, Din, rho, Uprev, Cprev, Lout); });
+hipError_t launch_stout_top(const Geo& g, const T* Utop, double coeff, const T* Qst, T* Lc, T* Fl, hipStream_t st) {
+    by_form<T>(g, [&](auto f) {
+        k_stout_top<T, decltype(f)::value><<<stencil_groups(f, grid_sites_mu(g.V)), stencil_threads(f), 0, st>>>(
+            g, Utop, coeff, Qst, Lc, Fl);
+    });
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_dsdu_chain(const Geo& g, const T* Utop, double coeff, const T* Uin, const T* Cst, T* Din, T* Lout,
-                             hipStream_t st) {
-    by_rows(g, [&](auto rows) { k_dsdu_chain<T, decltype(rows)::value><<<grid_sites_mu(g.V), kBlock, 0, st>>>(g, Utop, coeff, Uin, Cst, Din, Lout); });
+hipError_t launch_stout_pair(const Geo& g, const T* U, const T* Lc, T* Fl, T* far, double rho, hipStream_t st) {
+    const int groups = grid_sites_mu(g.V);
+    by_rows(g, [&](auto rows) {
+        if (groups <= 256)
+            k_stout_pair<T, decltype(rows)::value, 6><<<groups, 384, 0, st>>>(g, U, Lc, Fl, far, rho);
+        else
+            k_stout_pair<T, decltype(rows)::value, 4><<<groups, 256, 0, st>>>(g, U, Lc, Fl, far, rho);
+    });
     return hipGetLastError();
 }
-// K6a alone (the top level of a backward pass that starts from a given dS/dU)
 template <typename T>
-hipError_t launch_stout_back_local(const Geo& g, const T* Uin, const T* Cst, const T* Dout, T* Din, T* Lc, double rho,
-                                   hipStream_t st) {
-    const int nb = grid_sites_mu(g.V);
-    if (Cst)
-        by_rows(g, [&](auto rows) { k_stout_back_local<T, true, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Cst, Dout, Din, Lc, rho); });
-    else  // recompute C exactly as k_stout_forward formed it
-        by_rows(g, [&](auto rows) { k_stout_back_local<T, false, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, nullptr, Dout, Din, Lc, rho); });
+hipError_t launch_stout_gather(const Geo& g, const T* far, T* Fl, double rho, const T* Qst, T* Lc, hipStream_t st,
+                               int fmode, const T* U, T* FP, double eps_p, T* Unew, double eps_u, double* U64) {
+    const int groups = grid_sites_mu(g.V);
+    const bool small = groups <= 512;
+    const int nb = small ? 4 * groups : groups, nt = small ? 64 : kBlock;
+    const double fac = -1.0 / 3.0;
+    auto go = [&](auto out) {
+        constexpr int OUT = decltype(out)::value;
+        const bool s64 = OUT == FORCE_KICK_S64 || OUT == FORCE_KICK_EXP_S64;
+        by_rows(g, [&](auto rows) {
+            k_stout_gather<T, OUT, decltype(rows)::value><<<nb, nt, 0, st>>>(
+                g, far, Fl, rho, Qst, Lc, U, FP, Unew, OUT == FORCE_KICK || OUT == FORCE_KICK_EXP ? fac * eps_p : fac,
+                eps_u, s64 ? eps_p : 0.0, U64);
+        });
+    };
+    switch (fmode) {
+        case FORCE_STORE: go(std::integral_constant<int, FORCE_STORE>{}); break;
+        case FORCE_KICK: go(std::integral_constant<int, FORCE_KICK>{}); break;
+        case FORCE_KICK_EXP: go(std::integral_constant<int, FORCE_KICK_EXP>{}); break;
+        case FORCE_KICK_S64:
+        case FORCE_KICK_EXP_S64:
+            if constexpr (sizeof(T) == 4) {  // FP32 force kernels only
+                if (fmode == FORCE_KICK_S64)
+                    go(std::integral_constant<int, FORCE_KICK_S64>{});
+                else
+                    go(std::integral_constant<int, FORCE_KICK_EXP_S64>{});
+                break;
+            } else {
+                return hipErrorInvalidValue;
+            }
+        default: go(std::integral_constant<int, -1>{});
+    }
     return hipGetLastError();
 }
-// K6b alone (the thin-link level, or any level whose lower neighbour is not chained)
 template <typename T>
-hipError_t launch_stout_back_stencil(const Geo& g, const T* Uin, const T* Lc, T* Din, double rho, hipStream_t st,
-                                     int fmode, T* FP, double eps, T* Unew, double eps_u, double* U64) {
-    const int nb = grid_sites_mu(g.V);
-    if (fmode == FORCE_STORE)
-        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_STORE, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
-    else if (fmode == FORCE_KICK)
-        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
-    else if (fmode == FORCE_KICK_EXP)
-        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_EXP, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
-    else if (fmode == FORCE_KICK_S64 || fmode == FORCE_KICK_EXP_S64) {
-        if constexpr (sizeof(T) == 4) {  // FP32 force kernels only
-            if (!U64 && fmode == FORCE_KICK_EXP_S64) return hipErrorInvalidValue;
-            if (fmode == FORCE_KICK_S64)
-                by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_S64, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
-            else
-                by_rows(g, [&](auto rows) { k_stout_back_stencil<T, FORCE_KICK_EXP_S64, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
-        } else {
-            return hipErrorInvalidValue;
+hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, int nlev, T* D, T* D2, T* Lc, T* Lc2, double rho,
+                                 hipStream_t st) {
+    const int groups = grid_sites_mu(g.V);
+    if (stencil_form<T>(g) == ST_WIDE) {
+        const int nb = stencil_groups(ST_WIDE, groups), nt = stencil_threads(ST_WIDE);
+        T *la = Lc, *lb = Lc2;
+        k_stout_back_local<T, ST_WIDE><<<nb, nt, 0, st>>>(g, Uin[nlev - 1], D, D2, la, rho);
+        for (int l = nlev - 1; l >= 1; l--, std::swap(la, lb))
+            k_stout_back_chain_wide<T><<<nb, nt, 0, st>>>(g, Uin[l], la, D2, rho, Uin[l - 1], lb);
+        k_stout_back_stencil<T, ST_WIDE><<<nb, nt, 0, st>>>(g, Uin[0], la, D2, rho);
+        return hipGetLastError();
+    }
+    by_rows(g, [&](auto rows) {
+        constexpr int ST = decltype(rows)::value ? ST_ROWS : ST_CUT;
+        for (int l = nlev - 1; l >= 0; l--) {
+            k_stout_back_local<T, ST><<<groups, kBlock, 0, st>>>(g, Uin[l], l == nlev - 1 ? D : D2, D2, Lc, rho);
+            k_stout_back_stencil<T, ST><<<groups, kBlock, 0, st>>>(g, Uin[l], Lc, D2, rho);
         }
-    } else
-        by_rows(g, [&](auto rows) { k_stout_back_stencil<T, -1, decltype(rows)::value><<<nb, kBlock, 0, st>>>(g, Uin, Lc, Din, rho, FP, eps, Unew, eps_u, U64); });
+    });
     return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_stout_backward(const Geo& g, const T* Uin, const T* Cst, const T* Dout, T* Din, T* Lc, double rho,
-                                 hipStream_t st, int fmode, T* FP, double eps, T* Unew, double eps_u, double* U64) {
-    hipError_t e = launch_stout_back_local<T>(g, Uin, Cst, Dout, Din, Lc, rho, st);
-    if (e != hipSuccess) return e;
-    return launch_stout_back_stencil<T>(g, Uin, Lc, Din, rho, st, fmode, FP, eps, Unew, eps_u, U64);
 }
 
 #define GF_INST2(T)                                                                                       \
     template hipError_t launch_flow_stage<T>(const Geo&, const T*, T*, T*, double, double, hipStream_t);  \
     template hipError_t launch_stout_forward<T>(const Geo&, const T*, T*, T*, double, hipStream_t);       \
-    template hipError_t launch_stout_backward<T>(const Geo&, const T*, const T*, const T*, T*, T*, double, \
-                                                 hipStream_t, int, T*, double, T*, double, double*);       \
-    template hipError_t launch_stout_back_local<T>(const Geo&, const T*, const T*, const T*, T*, T*, double, \
-                                                   hipStream_t);                                            \
-    template hipError_t launch_stout_back_stencil<T>(const Geo&, const T*, const T*, T*, double, hipStream_t, \
-                                                     int, T*, double, T*, double, double*);                 \
-    template hipError_t launch_stout_back_chain<T>(const Geo&, const T*, const T*, T*, double, const T*,      \
-                                                   const T*, T*, hipStream_t);                              \
-    template hipError_t launch_dsdu_chain<T>(const Geo&, const T*, double, const T*, const T*, T*, T*, hipStream_t);
+    template hipError_t launch_stout_top<T>(const Geo&, const T*, double, const T*, T*, T*, hipStream_t); \
+    template hipError_t launch_stout_pair<T>(const Geo&, const T*, const T*, T*, T*, double, hipStream_t); \
+    template hipError_t launch_stout_gather<T>(const Geo&, const T*, T*, double, const T*, T*, hipStream_t, int, \
+                                               const T*, T*, double, T*, double, double*);                \
+    template hipError_t launch_stout_backward<T>(const Geo&, const T* const*, int, T*, T*, T*, T*, double,  \
+                                                 hipStream_t);
 
 GF_INST2(double)
 GF_INST2(float)

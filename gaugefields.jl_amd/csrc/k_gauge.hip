@@ -184,35 +184,7 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
     R6<T> own;
     T c[8];
     if (!ta_force<ST, T>(g, U, s, mu, own, c)) return;
-    const unsigned V = g.V;
-    const M3<T> umu = full_of(own);
-    if constexpr (MODE == FORCE_KICK_S64 || MODE == FORCE_KICK_EXP_S64) {
-        double* P64 = reinterpret_cast<double*>(FP);
-        double p[8];
-        ldp<double, GF_LD_NT>(P64, V, mu, s, p);
-#pragma unroll
-        for (int a = 0; a < 8; a++) p[a] = fma(eps_p, (double)scale1(fac, c[a]), p[a]);
-        stp<double, GF_ST_NT>(P64, V, mu, s, p);
-        if constexpr (MODE == FORCE_KICK_EXP_S64) {
-            const M3<double> un = exp_coeffs_times(p, eps_u, ldu<double, GF_LD_NT>(U64, V, mu, s));
-            stu<double, GF_ST_NT>(U64, V, mu, s, un);
-            stu<T, GF_ST_NT>(Unew, V, mu, s, round_link<T>(un));
-        }
-    } else if (MODE == FORCE_STORE) {
-#pragma unroll
-        for (int a = 0; a < 8; a++) c[a] = scale1(fac, c[a]);
-        stp<T, GF_ST_NT>(FP, V, mu, s, c);
-    } else {
-        T p[8];
-        ldp<T, GF_LD_NT>(FP, V, mu, s, p);
-#pragma unroll
-        for (int a = 0; a < 8; a++) p[a] = fma1(fac, c[a], p[a]);
-        stp<T, GF_ST_NT>(FP, V, mu, s, p);
-        if (MODE == FORCE_KICK_EXP) {
-            const M3<T> un = exp_coeffs_times(p, eps_u, umu);
-            stu<T, GF_ST_NT>(Unew, V, mu, s, un);
-        }
-    }
+    force_out<T, MODE>(c, [&] { return full_of(own); }, (unsigned)g.V, mu, s, FP, Unew, fac, eps_u, eps_p, U64);
 }
 
 // K4: U_mu <- exp(eps P_mu) U_mu  (exptU! + mul!, molecular_dynamics.jl:513-531)

@@ -421,6 +421,49 @@ __device__ __forceinline__ void ldp(const T* __restrict__ p, unsigned V, int mu,
     }
 }
 
+// The coefficients of a link per lane in LDS as memory holds them: planes of 16 bytes per lane (FP64
+// four pairs, FP32 two quads).  ldp_lds loads them there from memory without passing registers; the
+// wave has to wait_lds_loads() before it reads the place (the compiler does not see the dependence),
+// other waves need a barrier after that.
+template <typename T>
+constexpr int kC8Planes = sizeof(T) == 8 ? 4 : 2;
+template <typename T>
+struct alignas(16) C8Lds {
+    T v[kC8Planes<T>][64][16 / sizeof(T)];
+};
+template <typename T>
+__device__ __forceinline__ void ldp_lds(const T* __restrict__ p, unsigned V, int mu, unsigned s, C8Lds<T>* at) {
+    const __amdgpu_buffer_rsrc_t r = planes_rsrc(p, V, 4u * mu, 4u);
+#pragma unroll
+    for (int e = 0; e < kC8Planes<T>; e++)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)&at->v[e][0][0], 16,
+                                                 (int)(s * 16u), (int)(e * V * 16u), 0, 0);
+}
+__device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+template <typename T>
+__device__ __forceinline__ void get_c8(const C8Lds<T>* at, int lane, T c[8]) {
+    constexpr int N = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(N)));
+#pragma unroll
+    for (int e = 0; e < kC8Planes<T>; e++) {
+        const vec v = *reinterpret_cast<const vec*>(at->v[e][lane]);
+#pragma unroll
+        for (int k = 0; k < N; k++) c[N * e + k] = v[k];
+    }
+}
+template <typename T>
+__device__ __forceinline__ void put_c8(C8Lds<T>* at, int lane, const T c[8]) {
+    constexpr int N = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(N)));
+#pragma unroll
+    for (int e = 0; e < kC8Planes<T>; e++) {
+        vec v;
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = c[N * e + k];
+        *reinterpret_cast<vec*>(at->v[e][lane]) = v;
+    }
+}
+
 template <typename T, int AUX = GF_ST_DEFAULT>
 __device__ __forceinline__ void stp(T* __restrict__ p, unsigned V, int mu, unsigned s, const T c[8]) {
     const __amdgpu_buffer_rsrc_t r = planes_rsrc(p, V, 4u * mu, 4u);
@@ -753,19 +796,29 @@ __device__ __forceinline__ bool in_lattice(const Geo& g, const SiteMu& sm) {
 }
 
 // ---------------------------------------------------------------------------
-// ta_force_xrow for small lattices, where a kernel's time is the length of one wave's chain: a workgroup of
-// three waves over 64 sites and one direction mu, wave j forming the two staples of U_mu in the j-th
-// plane and TA(U_mu times them), the three added in LDS.  A wave waits for two batches of loads instead
-// of a dozen links one after another and multiplies a third of the matrices, and the work is spread over
-// four times as many CUs; no product is shared between directions, so the whole lattice costs 1.3 times
-// the operations, which one that leaves CUs empty does not notice.  Wave 0 returns true and goes on with
-// c and own.
+// Small lattices, where a kernel's time is the length of one wave's chain: a workgroup of three waves over
+// 64 sites and one direction mu, wave j working in the j-th plane of mu, what they find added in LDS.  A
+// wave waits for two batches of loads instead of a dozen links one after another and multiplies a third
+// of the matrices, and the work is spread over four times as many CUs; no product is shared between
+// directions, so the whole lattice costs 1.3 times the operations, which one that leaves CUs empty does
+// not notice.
+struct WideIndex {
+    int site, s;  // the lane's site, and clamped to the lattice
+    int mu, j;
+};
+__device__ __forceinline__ WideIndex wide_index(const Geo& g) {
+    const unsigned b = xcd_block();
+    WideIndex r;
+    r.site = (int)((b >> 2) * 64u + (threadIdx.x & 63u));
+    r.s = min(r.site, g.V - 1);
+    r.mu = (int)(b & 3u);
+    r.j = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    return r;
+}
+// the two staples of U_mu(x) in the plane of nu, and U_mu(x) as loaded
 template <typename T>
-__device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict__ U, unsigned V, int s, const int x[4],
-                                              int mu, R6<T>& own, T2<T> (*tp)[4][64], T c[8]) {
-    const int lane = (int)(threadIdx.x & 63u);
-    const int j = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nu = j + (j >= mu ? 1 : 0);
+__device__ __forceinline__ M3<T> staples_of_plane(const Geo& g, const T* __restrict__ U, unsigned V, int s,
+                                                  const int x[4], int mu, int nu, R6<T>& own) {
     int fw[4], bw[4];
 #pragma unroll
     for (int d = 0; d < 4; d++) {
@@ -775,31 +828,59 @@ __device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict_
     const int fmu = sel4(mu, fw[0], fw[1], fw[2], fw[3]), fnu = sel4(nu, fw[0], fw[1], fw[2], fw[3]);
     const int bnu = sel4(nu, bw[0], bw[1], bw[2], bw[3]);
     M3<T> sig = zero3<T>();
-    {
-        const R6<T> a = ldr(U, V, nu, (unsigned)(s + fmu)), b = ldr(U, V, mu, (unsigned)(s + fnu)),
-                    d = ldr(U, V, nu, (unsigned)s);
-        __builtin_amdgcn_sched_barrier(0);
-        const M3<T> X = su3_mul_nd(a, full_of(b));
-        const R6<T> e = ldr(U, V, mu, (unsigned)(s + bnu)), f = ldr(U, V, nu, (unsigned)(s + fmu + bnu));
-        __builtin_amdgcn_sched_barrier(0);
-        acc_mul_nd(sig, X, full_of(d));
-        const R6<T> h = ldr(U, V, nu, (unsigned)(s + bnu));
-        own = ldr(U, V, mu, (unsigned)s);
-        __builtin_amdgcn_sched_barrier(0);
-        acc_mul_dn(sig, su3_mul(e, full_of(f)), full_of(h));
-    }
-    ta_coeffs(mul(full_of(own), sig), c);
+    const R6<T> a = ldr(U, V, nu, (unsigned)(s + fmu)), b = ldr(U, V, mu, (unsigned)(s + fnu)),
+                d = ldr(U, V, nu, (unsigned)s);
+    __builtin_amdgcn_sched_barrier(0);
+    const M3<T> X = su3_mul_nd(a, full_of(b));
+    const R6<T> e = ldr(U, V, mu, (unsigned)(s + bnu)), f = ldr(U, V, nu, (unsigned)(s + fmu + bnu));
+    __builtin_amdgcn_sched_barrier(0);
+    acc_mul_nd(sig, X, full_of(d));
+    const R6<T> h = ldr(U, V, nu, (unsigned)(s + bnu));
+    own = ldr(U, V, mu, (unsigned)s);
+    __builtin_amdgcn_sched_barrier(0);
+    acc_mul_dn(sig, su3_mul(e, full_of(f)), full_of(h));
+    return sig;
+}
+// m of the workgroup's three waves added up in wave 0 (true), in the order of the waves
+template <typename T>
+__device__ __forceinline__ bool wide_sum(M3<T>& m, int j, T2<T> (*red)[9][64]) {
+    const int lane = (int)(threadIdx.x & 63u);
     if (j > 0) {
+#pragma unroll
+        for (int e = 0; e < 9; e++) red[j - 1][e][lane] = t2_of(m.m[e]);
+    }
+    __syncthreads();
+    if (j > 0) return false;
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int e = 0; e < 9; e++) {
+            const T2<T> v = red[k][e][lane];
+            m.m[e].r += v.x;
+            m.m[e].i += v.y;
+        }
+    return true;
+}
+// TA(U_mu Sigma_mu) in wave 0 (true), each wave's from its own plane's staples
+template <typename T>
+__device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict__ U, const WideIndex& wi,
+                                              R6<T>& own, T2<T> (*tp)[4][64], T c[8]) {
+    const int lane = (int)(threadIdx.x & 63u);
+    int x[4];
+    decode(g, wi.s, x);
+    const M3<T> sig = staples_of_plane(g, U, (unsigned)g.V, wi.s, x, wi.mu, wi.j + (wi.j >= wi.mu ? 1 : 0), own);
+    ta_coeffs(mul(full_of(own), sig), c);
+    if (wi.j > 0) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             T2<T> v;
             v.x = c[2 * e];
             v.y = c[2 * e + 1];
-            tp[j - 1][e][lane] = v;
+            tp[wi.j - 1][e][lane] = v;
         }
     }
     __syncthreads();
-    if (j > 0) return false;
+    if (wi.j > 0) return false;
 #pragma unroll
     for (int k = 0; k < 2; k++)
 #pragma unroll
@@ -841,16 +922,14 @@ struct ForceShare<T, ST_WIDE> {
 template <int ST, typename T>
 __device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, T c[8]) {
     __shared__ ForceShare<T, ST> sh;
-    int x[4];
     if constexpr (ST == ST_WIDE) {
-        const unsigned b = xcd_block();
-        const int site = (int)((b >> 2) * 64u + (threadIdx.x & 63u));
-        mu = (int)(b & 3u);
-        s = min(site, g.V - 1);
-        decode(g, s, x);
-        return ta_force_wide<T>(g, U, (unsigned)g.V, s, x, mu, own, sh.tp, c) && site < g.V;
+        const WideIndex wi = wide_index(g);
+        s = wi.s;
+        mu = wi.mu;
+        return ta_force_wide<T>(g, U, wi, own, sh.tp, c) && wi.site < g.V;
     } else {
         const SiteMu sm = site_mu_index(g);
+        int x[4];
         mu = sm.mu;
         s = stencil_site<ST == ST_ROWS>(g, sm);
         decode(g, s, x);

@@ -436,6 +436,104 @@ __device__ __forceinline__ M3<T> times_i(const M3<T>& m) {
     return c;
 }
 
+// element (i, j) of a Hermitian matrix
+template <typename T>
+__device__ __forceinline__ cx<T> herm_el(const Herm<T>& h, int i, int j) {
+    if (i == j) return cx<T>{h.d[i], T(0)};
+    return herm_off(h, i, j);
+}
+// coefficients of the traceless part of h as sum_a c_a lambda_a / 2 (inverse of herm_of_coeffs)
+template <typename T>
+__device__ __forceinline__ void coeffs_of_herm(const Herm<T>& h, T c[8]) {
+    c[0] = T(2) * h.u[0].r;
+    c[1] = T(-2) * h.u[0].i;
+    c[2] = h.d[0] - h.d[1];
+    c[3] = T(2) * h.u[1].r;
+    c[4] = T(-2) * h.u[1].i;
+    c[5] = T(2) * h.u[2].r;
+    c[6] = T(-2) * h.u[2].i;
+    c[7] = scale1(GF_SR3I, h.d[0] + h.d[1] - T(2) * h.d[2]);
+}
+// the Hermitian product m p^dag (or, DAG, m p) known to be Hermitian: upper triangle only
+template <bool DAG, typename T>
+__device__ __forceinline__ Herm<T> herm_product(const M3<T>& m, const M3<T>& p) {
+    Herm<T> r;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        T d = T(0);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const cx<T> a = m.m[3 * i + k], b = DAG ? p.m[3 * k + i] : p.m[3 * i + k];
+            d = fma(a.r, b.r, d);
+            d = DAG ? fma(-a.i, b.i, d) : fma(a.i, b.i, d);
+        }
+        r.d[i] = d;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = i + 1; j < 3; j++) {
+            cx<T> t;
+            t.r = t.i = T(0);
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                if (DAG)
+                    cmac(t, m.m[3 * i + k], p.m[3 * k + j]);
+                else
+                    cmac_nc(t, m.m[3 * i + k], p.m[3 * j + k]);
+            }
+            r.u[herm_up(i, j)] = t;
+        }
+    return r;
+}
+// u h u^dag and u^dag h u
+template <typename T>
+__device__ __forceinline__ Herm<T> herm_conj(const M3<T>& u, const Herm<T>& h) {
+    return herm_product<false>(mul_mh(u, h), u);
+}
+template <typename T>
+__device__ __forceinline__ Herm<T> herm_conj_dag(const M3<T>& u, const Herm<T>& h) {
+    return herm_product<true>(mul_dh(u, h), u);
+}
+// h m - m h
+template <typename T>
+__device__ __forceinline__ M3<T> herm_comm(const Herm<T>& h, const M3<T>& m) {
+    M3<T> c;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            cx<T> t;
+            const T d = h.d[i] - h.d[j];
+            t.r = i == j ? T(0) : m.m[3 * i + j].r * d;
+            t.i = i == j ? T(0) : m.m[3 * i + j].i * d;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                if (k != i) cmac(t, herm_off(h, i, k), m.m[3 * k + j]);
+                if (k != j) {
+                    cx<T> n = herm_off(h, k, j);
+                    n.r = -n.r;
+                    n.i = -n.i;
+                    cmac(t, m.m[3 * i + k], n);
+                }
+            }
+            c.m[3 * i + j] = t;
+        }
+    return c;
+}
+// coefficients of TA(i m)
+template <typename T>
+__device__ __forceinline__ void ta_coeffs_i(const M3<T>& m, T c[8]) {
+    c[0] = m.m[1].r + m.m[3].r;
+    c[1] = m.m[3].i - m.m[1].i;
+    c[2] = m.m[0].r - m.m[4].r;
+    c[3] = m.m[2].r + m.m[6].r;
+    c[4] = m.m[6].i - m.m[2].i;
+    c[5] = m.m[5].r + m.m[7].r;
+    c[6] = m.m[7].i - m.m[5].i;
+    c[7] = scale1(GF_SR3I, m.m[0].r + m.m[4].r - T(2) * m.m[8].r);
+}
+
 // ---------------------------------------------------------------------------
 // Cayley-Hamilton coefficients in double (Morningstar & Peardon, PRD 69 054501)
 // ---------------------------------------------------------------------------
@@ -747,59 +845,8 @@ __device__ __forceinline__ M3<T> exp_antiherm(const M3<T>& Q) {
     return expi_herm(H);
 }
 
-// L = C star d exp(Q)/dQ:  d tr(C e^Q) = tr(L dQ) for anti-Hermitian traceless Q
-// (CdexpQdQ!, stout_fast.jl:888-946, 1031-1081)
-template <typename T>
-__device__ __forceinline__ M3<T> cdexpqdq(const M3<T>& C, const M3<T>& Q) {
-    M3<T> H;  // H = -iQ (Hermitian)
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        H.m[k].r = Q.m[k].i;
-        H.m[k].i = -Q.m[k].r;
-    }
-    double c0, c1;
-    herm_invariants(H, c0, c1);
-    dc f[3], b1[3], b2[3];
-    exp_coeffs<true>(c0, c1, f, b1, b2);
-    M3<T> H2 = herm_sq(H);
-    // traces tr(C), tr(C H), tr(C H^2) in double
-    dc t0 = {0.0, 0.0}, t1 = {0.0, 0.0}, t2 = {0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        t0.r += double(C.m[4 * i].r);
-        t0.i += double(C.m[4 * i].i);
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const cx<T> c = C.m[3 * i + k];
-            const cx<T> h = H.m[3 * k + i];
-            const cx<T> g = H2.m[3 * k + i];
-            t1.r += double(c.r) * double(h.r) - double(c.i) * double(h.i);
-            t1.i += double(c.r) * double(h.i) + double(c.i) * double(h.r);
-            t2.r += double(c.r) * double(g.r) - double(c.i) * double(g.i);
-            t2.i += double(c.r) * double(g.i) + double(c.i) * double(g.r);
-        }
-    }
-    const dc tB1 = dca(dca(dcm(b1[0], t0), dcm(b1[1], t1)), dcm(b1[2], t2));
-    const dc tB2 = dca(dca(dcm(b2[0], t0), dcm(b2[1], t1)), dcm(b2[2], t2));
-    const T a1r = T(tB1.r), a1i = T(tB1.i), a2r = T(tB2.r), a2i = T(tB2.i);
-    const T f1r = T(f[1].r), f1i = T(f[1].i), f2r = T(f[2].r), f2i = T(f[2].i);
-    M3<T> HC = mul(H, C);
-    acc_mul(HC, C, H);  // H C + C H
-    M3<T> Lh;
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        T r = a1r * H.m[k].r - a1i * H.m[k].i + a2r * H2.m[k].r - a2i * H2.m[k].i + f1r * C.m[k].r -
-              f1i * C.m[k].i + f2r * HC.m[k].r - f2i * HC.m[k].i;
-        T im = a1r * H.m[k].i + a1i * H.m[k].r + a2r * H2.m[k].i + a2i * H2.m[k].r + f1r * C.m[k].i +
-               f1i * C.m[k].r + f2r * HC.m[k].i + f2i * HC.m[k].r;
-        // divide by i: (r + i im)/i = im - i r
-        Lh.m[k].r = im;
-        Lh.m[k].i = -r;
-    }
-    return Lh;
-}
-
-// exp(Q) and L = X star d exp(Q)/dQ together, sharing one evaluation of the invariants and
+// exp(Q) and L = X star d exp(Q)/dQ (d tr(X e^Q) = tr(L dQ) for anti-Hermitian traceless Q; CdexpQdQ!,
+// stout_fast.jl:888-946, 1031-1081) together, sharing one evaluation of the invariants and
 // Cayley-Hamilton coefficients (stout backward: E = e^{Q_mu}, L = CdexpQdQ(U_mu Dout_mu, Q_mu))
 template <typename T>
 __device__ __forceinline__ void exp_dexp(const M3<T>& Q, const M3<T>& X, M3<T>& E, M3<T>& L) {
@@ -860,6 +907,105 @@ __device__ __forceinline__ void exp_dexp(const M3<T>& Q, const M3<T>& X, M3<T>& 
     E.m[8].i += f0i;
 }
 
+
+// ---------------------------------------------------------------------------
+// One smearing level's site-local pullback in the algebra.  U' = e^Q U with Q = sum_a q_a i lambda_a / 2;
+// F' = TA(U' dS/dU') (coefficients f) is all of dS/dU' that a variation on the group sees.  With
+// dU' U'^dag = d(e^Q) e^-Q + e^Q (dU U^dag) e^-Q,
+//   Lam = TA(CdexpQdQ(e^-Q F', Q)):  the derivative with respect to Q   (-> lam)
+//   Floc = e^-Q F' e^Q = F' - [Q, Lam]:  that with respect to U at fixed Q   (-> floc)
+// With Q = iH, F' = i Hf, e^-Q = conj(f0) + conj(f1) H + conj(f2) H^2 and X = e^-Q F', the derivative
+// of the exponential (CdexpQdQ!, stout_fast.jl:888-946) is i L = a1 H + a2 H^2 + f1 X + f2 (H X + X H),
+// a_k = sum_j b_kj tr(X H^j); H commutes with e^-Q, so f1 X + f2 (HX + XH) = i e^-Q (f1 Hf + f2 (H Hf + Hf H)),
+// and the traces follow from tr(H^n Hf), n = 1, 2, by H^3 = c1 H + c0.
+// ---------------------------------------------------------------------------
+template <typename T>
+__device__ __forceinline__ void stout_local(const T q[8], const T f[8], T lam[8], T floc[8]) {
+    const Herm<T> H = herm_of_coeffs(q), F = herm_of_coeffs(f);
+    M3<T> Hm;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) Hm.m[3 * i + j] = herm_el(H, i, j);
+    double c0, c1;
+    herm_invariants(Hm, c0, c1);
+    const M3<T> H2 = herm_sq(Hm);
+    double s1 = 0.0, s2 = 0.0;  // tr(H Hf), tr(H^2 Hf)
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        s1 = fma((double)H.d[i], (double)F.d[i], s1);
+        s2 = fma((double)H2.m[4 * i].r, (double)F.d[i], s2);
+#pragma unroll
+        for (int j = i + 1; j < 3; j++) {
+            const cx<T> b = F.u[herm_up(i, j)], a = H.u[herm_up(i, j)], a2 = H2.m[3 * i + j];
+            s1 = fma(2.0 * (double)a.r, (double)b.r, fma(2.0 * (double)a.i, (double)b.i, s1));
+            s2 = fma(2.0 * (double)a2.r, (double)b.r, fma(2.0 * (double)a2.i, (double)b.i, s2));
+        }
+    }
+    dc fc[3], b1[3], b2[3];
+    exp_coeffs<true>(c0, c1, fc, b1, b2);
+    // tr(X H^j) = i tr(e^-Q H^j Hf)
+    const double s3 = c1 * s1, s4 = fma(c1, s2, c0 * s1);
+    auto itr = [&](double p0, double p1, double p2) -> dc {  // i (conj(f0) p0 + conj(f1) p1 + conj(f2) p2)
+        return dc{fc[0].i * p0 + fc[1].i * p1 + fc[2].i * p2, fc[0].r * p0 + fc[1].r * p1 + fc[2].r * p2};
+    };
+    const dc t0 = itr(0.0, s1, s2), t1 = itr(s1, s2, s3), t2 = itr(s2, s3, s4);
+    // only Re a_k enters the antihermitian part of -i (a1 H + a2 H^2)
+    const double a1 = b1[0].r * t0.r - b1[0].i * t0.i + b1[1].r * t1.r - b1[1].i * t1.i + b1[2].r * t2.r - b1[2].i * t2.i;
+    const double a2 = b2[0].r * t0.r - b2[0].i * t0.i + b2[1].r * t1.r - b2[1].i * t1.i + b2[2].r * t2.r - b2[2].i * t2.i;
+    const T f0r = T(fc[0].r), f0i = T(fc[0].i), f1r = T(fc[1].r), f1i = T(fc[1].i), f2r = T(fc[2].r), f2i = T(fc[2].i);
+    M3<T> W, E;  // f1 Hf + f2 (H Hf + Hf H);  e^-Q
+    {
+        M3<T> Fm;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) Fm.m[3 * i + j] = herm_el(F, i, j);
+        const M3<T> M = mul_hm(H, Fm);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const cx<T> m = M.m[3 * i + j], n = M.m[3 * j + i], b = Fm.m[3 * i + j];
+                const T kr = m.r + n.r, ki = m.i - n.i;
+                W.m[3 * i + j].r = f1r * b.r - f1i * b.i + f2r * kr - f2i * ki;
+                W.m[3 * i + j].i = f1r * b.i + f1i * b.r + f2r * ki + f2i * kr;
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const cx<T> h = Hm.m[k], g = H2.m[k];
+        E.m[k].r = f1r * h.r + f1i * h.i + f2r * g.r + f2i * g.i + (k % 4 == 0 ? f0r : T(0));
+        E.m[k].i = f1r * h.i - f1i * h.r + f2r * g.i - f2i * g.r - (k % 4 == 0 ? f0i : T(0));
+    }
+    ta_coeffs(mul(E, W), lam);
+    {
+        Herm<T> h2;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            h2.d[i] = H2.m[4 * i].r;
+#pragma unroll
+            for (int j = i + 1; j < 3; j++) h2.u[herm_up(i, j)] = H2.m[3 * i + j];
+        }
+        T c2[8];
+        coeffs_of_herm(h2, c2);
+#pragma unroll
+        for (int k = 0; k < 8; k++) lam[k] = (T)fma(-a1, (double)q[k], fma(-a2, (double)c2[k], (double)lam[k]));
+    }
+    // [Q, Lam] = -(M - M^dag), M = H Hlam
+    T m[8];
+    {
+        const Herm<T> Hl = herm_of_coeffs(lam);
+        M3<T> Lm;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) Lm.m[3 * i + j] = herm_el(Hl, i, j);
+        ta_coeffs(mul_hm(H, Lm), m);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) floc[k] = fma(T(2), m[k], f[k]);
+}
 
 // ---------------------------------------------------------------------------
 // SU(3) link updates U' = exp(X) U.  For float storage the exponential, the product and the

@@ -264,7 +264,7 @@ class Lattice:
 
     # -- stout ----------------------------------------------------------------------------
     def stout_config(self, nlev, rho, mode="store"):
-        """mode: "store" (keep C per level), "recompute", or "auto" (store if it fits)"""
+        """mode: "store" (keep Q per level), "recompute", or "auto" (store if it fits)"""
         m = {"store": _lib.GF_STOUT_STORE, "recompute": _lib.GF_STOUT_RECOMPUTE, "auto": _lib.GF_STOUT_AUTO}[mode]
         self._c(self._L.gf_stout_config(self._ctx, int(nlev), ctypes.c_double(rho), m))
         self.nlev = int(nlev)

@@ -183,10 +183,10 @@ int gf_flow_measure(gf_ctx *ctx, double eps, int nsteps, int every, double *out)
 
 /* ---- stout smearing ---------------------------------------------------------------- */
 /* nlev stout layers at rho (STOUT_Layer + CovNeuralnet, stout_fast.jl:6-122,
- * Abstractsmearing.jl:61-99); mode GF_STOUT_STORE keeps C_mu per level, GF_STOUT_RECOMPUTE
- * recomputes it in the backward pass, GF_STOUT_AUTO stores when the device has room for the
- * nlev extra link fields (plus a 10 % margin) and recomputes otherwise.  The smeared levels
- * themselves are always kept.  nlev = 0 disables smearing. */
+ * Abstractsmearing.jl:61-99); mode GF_STOUT_STORE keeps every level's Q_mu (8 reals a link),
+ * GF_STOUT_RECOMPUTE forms it again in the backward pass, GF_STOUT_AUTO stores when the device has
+ * room for the nlev momentum-sized fields (plus a 10 % margin) and recomputes otherwise.  The smeared
+ * levels themselves are always kept.  nlev = 0 disables smearing. */
 int gf_stout_config(gf_ctx *ctx, int nlev, double rho, int mode);
 /* the memory mode in effect after gf_stout_config (GF_STOUT_STORE or GF_STOUT_RECOMPUTE) */
 int gf_stout_mode(const gf_ctx *ctx, int *mode);
