@@ -54,6 +54,8 @@ struct gf_ctx {
     void* U64 = nullptr;
     void* P64 = nullptr;
     void* U64bak = nullptr;
+    void* loops = nullptr;  // loop coefficients of the field strengths, a block of t-slices
+    size_t loops_bytes = 0;
     // scratch for layout conversion and reductions
     double* staging = nullptr;  // 72 V doubles
     double* partial = nullptr;
@@ -239,10 +241,18 @@ int fstrength(gf_ctx* c, int sets, double out[4], double* dens_host, int dens_me
         TRY(need_staging(c));
         dens = c->staging;
     }
+    const size_t need = field_strength_bytes(c->geo, sets);
+    if (need > c->loops_bytes) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        release(c, &c->loops, c->loops_bytes);
+        c->loops_bytes = 0;
+        TRY(alloc(c, &c->loops, need));
+        c->loops_bytes = need;
+    }
     TRY(dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->partial, c->dres, dens, dens_method,
-                                           c->stream));
+        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->loops, c->partial, c->dres, dens,
+                                           dens_method, c->stream));
         return GF_OK;
     }));
     HIPCHK(c, hipMemcpyAsync(c->hres, c->dres, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -544,7 +554,7 @@ int gf_create(const int* dims, int precision, int device, gf_ctx** out) {
         if (hipEventCreate(&c->ev[i]) != hipSuccess) return bail(GF_EDEVICE);
     if (alloc(c, &c->U, link_bytes(c)) || alloc(c, &c->Ualt, link_bytes(c)) || alloc(c, &c->P, mom_bytes(c)) ||
         alloc(c, &c->F, mom_bytes(c)) ||
-        alloc(c, (void**)&c->partial, sizeof(double) * (4 * std::max(grid_for(c->V), grid_sites_mu(c->V)) + 16)) ||
+        alloc(c, (void**)&c->partial, sizeof(double) * (4 * ((size_t)grid_sites_mu(c->V) + c->dims[3]) + 16)) ||
         alloc(c, (void**)&c->dres, 4 * sizeof(double)))
         return bail(GF_ENOMEM);
     if (hipHostMalloc((void**)&c->hres, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(GF_ENOMEM);
@@ -570,6 +580,7 @@ int gf_destroy(gf_ctx* c) {
         if (c->lev[l]) (void)hipFree(c->lev[l]);
         if (c->Qst[l]) (void)hipFree(c->Qst[l]);
     }
+    if (c->loops) (void)hipFree(c->loops);
     if (c->staging) (void)hipFree(c->staging);
     if (c->partial) (void)hipFree(c->partial);
     if (c->dres) (void)hipFree(c->dres);

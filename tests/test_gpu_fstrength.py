@@ -53,6 +53,33 @@ def test_topological_charge_parity(Lat, oracle, dims):
     assert L.energy_density_clover() == pytest.approx(Eref, rel=1e-12)
 
 
+@pytest.mark.parametrize("dims,precision", [
+    ((1, 2, 3, 5), "f64"),          # two steps wrap more than once
+    ((2, 1, 1, 2), "f32"),
+    ((66, 3, 2, 4), "f64"),         # rows longer than a wave, groups that start inside a row
+    ((3, 131, 2, 3), "f32"),        # slices no multiple of 64
+    ((16, 16, 10, 4), "f32"),       # followed through t, x rows cut by nothing
+    ((24, 16, 8, 5), "f64"),        # followed through t, rows cut by the groups
+    ((32, 32, 32, 7), "f64"),       # several blocks of t-slices, the last one shorter for the improved charge
+    ((30, 26, 25, 11), "f64"),       # the same, not followed through t
+])
+def test_loops_by_blocks(Lat, oracle, dims, precision):
+    """Edges of the waves, blocks and orders of the two-kernel form.  FP32 links: the oracle on the rounded links,
+    with rows 2 to single rounding (bound of test_fp32_bulk_topological_charge)."""
+    print(f"[fstrength] blocks {dims} {precision}", flush=True)
+    U = alg_links(oracle, dims, 0.6, 41)
+    L = Lat(dims, precision)
+    L.upload_links(U)
+    W = U if precision == "f64" else U.astype(np.complex64).astype(np.complex128)
+    tol, rel = (1e-13, 1e-12) if precision == "f64" else (1e-6, 1e-6)
+    for m in ("clover", "rectangle", "improved"):
+        Qref, qref = oracle.topological_charge_density(dims, W, m)
+        bound = tol if precision == "f64" else tol * max(np.abs(qref).max(), 1e-3)
+        assert np.abs(L.topological_charge_density(m) - qref).max() < bound, m
+        assert abs(L.topological_charge(m) - Qref) <= max(rel * abs(Qref), np.sqrt(qref.size) * bound), m
+    assert L.energy_density_clover() == pytest.approx(oracle.energy_density_clover(dims, W), rel=rel)
+
+
 def test_constant_abelian_field_closed_form(Lat):
     dims = (4, 6, 6, 4)
     U, t, tp = lt.abelian_flux_links(dims, 2, -1)
