@@ -12,6 +12,7 @@
 
 #include "../../include/gfhip.h"
 #include "internal.hpp"
+#include "transfer.hpp"
 
 using namespace gf;
 
@@ -56,8 +57,9 @@ struct gf_ctx {
     void* U64bak = nullptr;
     void* loops = nullptr;  // loop coefficients of the field strengths, a block of t-slices
     size_t loops_bytes = 0;
-    // scratch for layout conversion and reductions
-    double* staging = nullptr;  // 72 V doubles
+    // scratch for per-site outputs and reductions
+    double* staging = nullptr;  // 18 V doubles
+    HostRing ring;              // host arrays in and out
     double* partial = nullptr;
     double* dres = nullptr;   // device scalar
     double* hres = nullptr;   // pinned host scalar
@@ -203,7 +205,92 @@ void make_geometry(const int* dims, long long V, Geo& g, char* seen) {
     }
 }
 
-int need_staging(gf_ctx* c) { return alloc(c, (void**)&c->staging, (size_t)72 * c->V * sizeof(double)); }
+// Arrays that go up in one copy by the runtime and a layout kernel behind it rather than through the ring: for
+// pages that are there already its copy is as fast as ours, and a single one spares the launches and waits
+// (momenta 8^4 66 us against 96, 12^4 183 / 245, 16^4 of 17 MB 514 / 518, 20^3x10 of 20 MB 661 / 588)
+constexpr size_t kSingleUp = (size_t)16 << 20;
+// and plain ones that come down so (densities 8^4 40 / 41 us, 16^4 67 / 71, 24^3x48 of 5 MB 481 / 384)
+constexpr size_t kSingleDown = (size_t)1 << 20;
+int need_staging(gf_ctx* c) {
+    const size_t links = (size_t)72 * c->V * sizeof(double);
+    return alloc(c, (void**)&c->staging, std::max(links / 4, std::min(links, kSingleUp)));
+}
+
+// Host arrays.  (4, V, W) doubles go in units of a wave's links (group q: k_links_to_ref), plain ones by 4 KB.
+int need_ring(gf_ctx* c) {
+    const hipError_t e = c->ring.need((size_t)72 * c->V * sizeof(double), c->device);
+    return e == hipSuccess ? GF_OK : fail(c, GF_ENOMEM, "pinned host memory: %s", hipGetErrorString(e));
+}
+struct GroupBytes {
+    size_t V, groups, link;  // link: bytes
+    GroupBytes(const gf_ctx* c, int reals) : V(c->V), groups((V + 63) / 64), link(8 * (size_t)reals) {}
+    long units() const { return 4 * (long)groups; }
+    size_t operator()(long q) const { return (q / groups * V + q % groups * 64) * link; }
+};
+// launch(q0, n, slot) on the groups q0 .. q0 + n
+template <typename F>
+int pull_groups(gf_ctx* c, double* dst, int reals, F launch) {
+    TRY(need_ring(c));
+    const GroupBytes at(c, reals);
+    HIPCHK(c, c->ring.pull((char*)dst, at.units(), 64 * at.link, at, launch, c->stream));
+    return GF_OK;
+}
+template <typename F>
+int push_groups(gf_ctx* c, const double* src, int reals, F launch) {
+    const GroupBytes at(c, reals);
+    if (at(at.units()) <= kSingleUp) {
+        TRY(need_staging(c));
+        HIPCHK(c, hipMemcpyAsync(c->staging, src, at(at.units()), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, launch(0, at.units(), (const char*)c->staging));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return GF_OK;
+    }
+    TRY(need_ring(c));
+    HIPCHK(c, c->ring.push((const char*)src, at.units(), 64 * at.link, at, launch, c->stream));
+    return GF_OK;
+}
+int pull_plain(gf_ctx* c, double* dst, const double* src, size_t n) {
+    const size_t bytes = n * sizeof(double), unit = 4096;
+    if (bytes <= kSingleDown) {
+        HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return GF_OK;
+    }
+    TRY(need_ring(c));
+    HIPCHK(c, c->ring.pull(
+                  (char*)dst, (long)((bytes + unit - 1) / unit), unit, [&](long q) { return std::min(bytes, q * unit); },
+                  [&](long q, long k, char* p) {
+                      const size_t a = q * unit, b = std::min(bytes, a + k * unit);
+                      return hipMemcpyAsync(p, (const char*)src + a, b - a, hipMemcpyDeviceToHost, c->stream);
+                  },
+                  c->stream));
+    return GF_OK;
+}
+
+template <typename T>
+int upload_links_as(gf_ctx* c, T* field, const double* ref, bool general) {
+    return push_groups(c, ref, 18, [&](long q, long n, const char* p) {
+        return launch_links_from_ref<T>((const double*)p, field, c->V, general, (int)q, (int)n, c->stream);
+    });
+}
+template <typename T>
+int download_links_as(gf_ctx* c, const T* field, double* ref, bool general) {
+    return pull_groups(c, ref, 18, [&](long q, long n, char* p) {
+        return launch_links_to_ref<T>(field, (double*)p, c->V, general, (int)q, (int)n, c->stream);
+    });
+}
+template <typename T>
+int upload_mom_as(gf_ctx* c, T* field, const double* mom) {
+    return push_groups(c, mom, 8, [&](long q, long n, const char* p) {
+        return launch_momenta_from_ref<T>((const double*)p, field, c->V, (int)q, (int)n, c->stream);
+    });
+}
+template <typename T>
+int download_mom_as(gf_ctx* c, const T* field, double* mom) {
+    return pull_groups(c, mom, 8, [&](long q, long n, char* p) {
+        return launch_momenta_to_ref<T>(field, (double*)p, c->V, (int)q, (int)n, c->stream);
+    });
+}
 
 // typed dispatch: f.template operator()<T>()
 template <typename F>
@@ -257,8 +344,9 @@ int fstrength(gf_ctx* c, int sets, double out[4], double* dens_host, int dens_me
     }));
     HIPCHK(c, hipMemcpyAsync(c->hres, c->dres, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     if (dens_host)
-        HIPCHK(c, hipMemcpyAsync(dens_host, dens, sizeof(double) * (size_t)c->V, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+        TRY(pull_plain(c, dens_host, dens, c->V));
+    else
+        HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int k = 0; k < 4; k++) out[k] = c->hres[k];
     return GF_OK;
 }
@@ -489,7 +577,6 @@ int hamiltonian(gf_ctx* c, double coeff, double* H) {
 
 }  // namespace
 
-
 // ---- plaquette sum of caller-held device links, allocating nothing --------------------------
 // The per-workgroup partial sums of k_plaquette go to `scratch`, a file-scope device array
 // that every device holds once for the life of the process.  Host code never passes the
@@ -582,6 +669,7 @@ int gf_destroy(gf_ctx* c) {
     }
     if (c->loops) (void)hipFree(c->loops);
     if (c->staging) (void)hipFree(c->staging);
+    c->ring.free();
     if (c->partial) (void)hipFree(c->partial);
     if (c->dres) (void)hipFree(c->dres);
     if (c->hres) (void)hipHostFree(c->hres);
@@ -629,9 +717,10 @@ struct Su3Check {
     size_t link = 0;     // link index (mu * V + site) of the largest deviation
     const char* what = "";
 };
-static Su3Check su3_deviation(const double* ref, size_t nlinks) {
+// links first .. last of ref: the largest deviation, the first of equal ones; the first NaN ends the search
+static Su3Check su3_deviation(const double* ref, size_t first, size_t last) {
     Su3Check r;
-    for (size_t l = 0; l < nlinks; l++) {
+    for (size_t l = first; l < last; l++) {
         const double* m = ref + 18 * l;  // element (i, j) at complex offset i + 3 j
         auto re = [&](int i, int j) { return m[2 * (i + 3 * j)]; };
         auto im = [&](int i, int j) { return m[2 * (i + 3 * j) + 1]; };
@@ -664,53 +753,48 @@ static Su3Check su3_deviation(const double* ref, size_t nlinks) {
     return r;
 }
 
+// the same over all links, by several threads in parts that are joined in order
+static Su3Check su3_deviation(gf_ctx* c, const double* ref, size_t nlinks) {
+    constexpr size_t kPart = 2048, kParts = 64;  // links of a part at least (50 us), and parts at most
+    const size_t parts = std::min(kParts, (nlinks + kPart - 1) / kPart);
+    Su3Check part[kParts];
+    in_parts(c->ring, (long)parts,
+             [&](long k) { part[k] = su3_deviation(ref, nlinks * k / parts, nlinks * (k + 1) / parts); });
+    Su3Check r;
+    for (size_t k = 0; k < parts; k++) {
+        if (std::isnan(part[k].worst)) return part[k];
+        if (part[k].worst > r.worst) r = part[k];
+    }
+    return r;
+}
+
+// general: the field holds general 3x3 matrices (derivatives) rather than SU(3) links
+static int download_linkfield(gf_ctx* c, const void* field, double* ref, bool general = false) {
+    return dispatch(c, [&](auto* tag) -> int {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        return download_links_as<T>(c, (const T*)field, ref, general);
+    });
+}
+static int upload_linkfield(gf_ctx* c, void* field, const double* ref, bool general = false) {
+    return dispatch(c, [&](auto* tag) -> int {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        return upload_links_as<T>(c, (T*)field, ref, general);
+    });
+}
+
 int gf_upload_links(gf_ctx* c, const double* ref) {
     CTXCHK(c);
     if (!ref) return fail(c, GF_EINVAL, "null links");
     {
-        const Su3Check chk = su3_deviation(ref, (size_t)4 * c->V);
+        const Su3Check chk = su3_deviation(c, ref, (size_t)4 * c->V);
         if (!(chk.worst <= kSu3Tol))
             return fail(c, GF_EINVAL,
                         "links must be SU(3): at direction %d, site %zu %s by %g (limit %g)",
                         (int)(chk.link / (size_t)c->V) + 1, chk.link % (size_t)c->V, chk.what, chk.worst, kSu3Tol);
     }
-    TRY(need_staging(c));
-    HIPCHK(c, hipMemcpyAsync(c->staging, ref, (size_t)72 * c->V * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (c->s64) {
-        HIPCHK(c, launch_links_from_ref<double>(c->staging, (double*)c->U64, c->V, false, c->stream));
-        TRY(state64_step(c, 3, 0.0));
-    } else {
-        TRY(dispatch(c, [&](auto* tag) -> int {
-            using T = std::remove_pointer_t<decltype(tag)>;
-            HIPCHK(c, launch_links_from_ref<T>(c->staging, (T*)c->U, c->V, false, c->stream));
-            return GF_OK;
-        }));
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return GF_OK;
-}
-
-// general: the field holds general 3x3 matrices (derivatives) rather than SU(3) links
-static int download_linkfield(gf_ctx* c, const void* field, double* ref, bool general = false) {
-    TRY(need_staging(c));
-    TRY(dispatch(c, [&](auto* tag) -> int {
-        using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_links_to_ref<T>((const T*)field, c->staging, c->V, general, c->stream));
-        return GF_OK;
-    }));
-    HIPCHK(c, hipMemcpyAsync(ref, c->staging, (size_t)72 * c->V * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return GF_OK;
-}
-
-static int upload_linkfield(gf_ctx* c, void* field, const double* ref, bool general = false) {
-    TRY(need_staging(c));
-    HIPCHK(c, hipMemcpyAsync(c->staging, ref, (size_t)72 * c->V * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    TRY(dispatch(c, [&](auto* tag) -> int {
-        using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_links_from_ref<T>(c->staging, (T*)field, c->V, general, c->stream));
-        return GF_OK;
-    }));
+    if (!c->s64) return upload_linkfield(c, c->U, ref);
+    TRY(upload_links_as<double>(c, (double*)c->U64, ref, false));
+    TRY(state64_step(c, 3, 0.0));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return GF_OK;
 }
@@ -718,47 +802,23 @@ static int upload_linkfield(gf_ctx* c, void* field, const double* ref, bool gene
 int gf_download_links(gf_ctx* c, double* ref) {
     CTXCHK(c);
     if (!ref) return fail(c, GF_EINVAL, "null links");
-    if (c->s64) {
-        TRY(need_staging(c));
-        HIPCHK(c, launch_links_to_ref<double>((const double*)c->U64, c->staging, c->V, false, c->stream));
-        HIPCHK(c, hipMemcpyAsync(ref, c->staging, (size_t)72 * c->V * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return GF_OK;
-    }
-    return download_linkfield(c, c->U, ref);
+    return c->s64 ? download_links_as<double>(c, (const double*)c->U64, ref, false) : download_linkfield(c, c->U, ref);
 }
 
 // f64: the field is an FP64 momentum field whatever the context's arithmetic
 static int upload_mom(gf_ctx* c, void* field, const double* mom, bool f64 = false) {
-    TRY(need_staging(c));
-    HIPCHK(c, hipMemcpyAsync(c->staging, mom, (size_t)32 * c->V * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (f64) {
-        HIPCHK(c, launch_momenta_from_ref<double>(c->staging, (double*)field, c->V, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return GF_OK;
-    }
-    TRY(dispatch(c, [&](auto* tag) -> int {
+    if (f64) return upload_mom_as<double>(c, (double*)field, mom);
+    return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_momenta_from_ref<T>(c->staging, (T*)field, c->V, c->stream));
-        return GF_OK;
-    }));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return GF_OK;
+        return upload_mom_as<T>(c, (T*)field, mom);
+    });
 }
 static int download_mom(gf_ctx* c, const void* field, double* mom, bool f64 = false) {
-    TRY(need_staging(c));
-    if (f64) {
-        HIPCHK(c, launch_momenta_to_ref<double>((const double*)field, c->staging, c->V, c->stream));
-    } else {
-        TRY(dispatch(c, [&](auto* tag) -> int {
-            using T = std::remove_pointer_t<decltype(tag)>;
-            HIPCHK(c, launch_momenta_to_ref<T>((const T*)field, c->staging, c->V, c->stream));
-            return GF_OK;
-        }));
-    }
-    HIPCHK(c, hipMemcpyAsync(mom, c->staging, (size_t)32 * c->V * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return GF_OK;
+    if (f64) return download_mom_as<double>(c, (const double*)field, mom);
+    return dispatch(c, [&](auto* tag) -> int {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        return download_mom_as<T>(c, (const T*)field, mom);
+    });
 }
 
 int gf_upload_momenta(gf_ctx* c, const double* mom) {
@@ -832,9 +892,7 @@ int gf_action_untraced(gf_ctx* c, double coeff, double* ref) {
         HIPCHK(c, launch_action_untraced<T>(c->geo, (const T*)c->U, coeff, c->staging, c->stream));
         return GF_OK;
     }));
-    HIPCHK(c, hipMemcpyAsync(ref, c->staging, (size_t)18 * c->V * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return GF_OK;
+    return pull_plain(c, ref, c->staging, (size_t)18 * c->V);
 }
 int gf_momenta_dot(gf_ctx* c, double* value) {
     CTXCHK(c);

@@ -114,13 +114,13 @@ hipError_t launch_links_widen(const float* Uf, double* Ud, int V, hipStream_t st
 hipError_t launch_state64_step(int mode, const Geo& g, const double* P64, double* U64, float* U32, double eps_u,
                                hipStream_t st);
 template <typename T>
-hipError_t launch_links_from_ref(const double* ref, T* soa, int V, bool general, hipStream_t st);
+hipError_t launch_links_from_ref(const double* ref, T* soa, int V, bool general, int q0, int nq, hipStream_t st);
 template <typename T>
-hipError_t launch_links_to_ref(const T* soa, double* ref, int V, bool general, hipStream_t st);
+hipError_t launch_links_to_ref(const T* soa, double* ref, int V, bool general, int q0, int nq, hipStream_t st);
 template <typename T>
-hipError_t launch_momenta_from_ref(const double* ref, T* soa, int V, hipStream_t st);
+hipError_t launch_momenta_from_ref(const double* ref, T* soa, int V, int q0, int nq, hipStream_t st);
 template <typename T>
-hipError_t launch_momenta_to_ref(const T* soa, double* ref, int V, hipStream_t st);
+hipError_t launch_momenta_to_ref(const T* soa, double* ref, int V, int q0, int nq, hipStream_t st);
 template <typename T>
 hipError_t launch_set_identity(T* U, int V, hipStream_t st);
 template <typename T>

@@ -267,68 +267,125 @@ hipError_t launch_state64_step(int mode, const Geo& g, const double* P64, double
 // layout conversion between the reference's (3,3,X,Y,Z,T) complex column-major arrays
 // (FP64, per direction) and the SoA planes
 // ---------------------------------------------------------------------------
+// A wave moves the 64-site group q of the direction-major order (group q % G of direction q / G, G = ceil(V / 64)):
+// its links are one piece of the host array, which lies in pinned host memory as often as on the device, so the
+// wave reads or writes that piece in whole lines, 16 B per lane, and turns it in LDS.  A thread per link, as these
+// were, touches a line in each of 64 places per instruction (12^4 links: 14 -> 5 us on the device).
+__device__ __forceinline__ bool group_at(int V, int q0, int nq, int& mu, int& s0, int& m) {
+    const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
+    const int G = (V + 63) / 64;
+    mu = (q0 + w) / G;
+    s0 = (q0 + w) % G * 64;
+    m = V - s0 < 64 ? V - s0 : 64;
+    return w < nq;
+}
+// the piece of group q in an array that starts at group q0, W doubles per link
+template <int W>
+__device__ __forceinline__ size_t piece(int V, int q0, int mu, int s0) {
+    const int G = (V + 63) / 64;
+    return ((size_t)mu * V + s0 - ((size_t)(q0 / G) * V + q0 % G * 64)) * W;
+}
+typedef double dvec2 __attribute__((ext_vector_type(2)));
+// n 16-byte words between memory and the wave's LDS, where a link's words are PITCH apart
+template <int WORDS, int PITCH>
+__device__ __forceinline__ void words_in(const double* __restrict__ at, dvec2* sh, int lane, int n) {
+    const dvec2* const p = (const dvec2*)at;
+#pragma unroll
+    for (int k = 0; k < WORDS; k++) {
+        const int i = 64 * k + lane;
+        if (i < n) sh[i / WORDS * PITCH + i % WORDS] = __builtin_nontemporal_load(p + i);
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+template <int WORDS, int PITCH>
+__device__ __forceinline__ void words_out(double* __restrict__ at, const dvec2* sh, int lane, int n) {
+    __builtin_amdgcn_wave_barrier();
+    dvec2* const p = (dvec2*)at;
+#pragma unroll
+    for (int k = 0; k < WORDS; k++) {
+        const int i = 64 * k + lane;
+        if (i < n) __builtin_nontemporal_store(sh[i / WORDS * PITCH + i % WORDS], p + i);
+    }
+}
 // GEN = false: SU(3) link field (rows 0 and 1 stored); GEN = true: general 3x3 matrix field
 template <typename T, bool GEN>
-__global__ __launch_bounds__(kBlock) void k_links_from_ref(const double* __restrict__ ref, T* __restrict__ soa, int V) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    for (int mu = 0; mu < 4; mu++) {
-        const double* r = ref + ((size_t)mu * V + s) * 18;
-        M3<T> m;
+__global__ __launch_bounds__(kBlock) void k_links_from_ref(const double* __restrict__ ref, T* __restrict__ soa, int V,
+                                                           int q0, int nq) {
+    __shared__ dvec2 buf[kBlock / 64][64 * 9];
+    const int lane = (int)(threadIdx.x & 63u);
+    dvec2* const sh = buf[threadIdx.x >> 6];
+    int mu, s0, n;
+    if (!group_at(V, q0, nq, mu, s0, n)) return;
+    words_in<9, 9>(ref + piece<18>(V, q0, mu, s0), sh, lane, 9 * n);
+    if (lane >= n) return;
+    M3<T> m;
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+    for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const int c = i + 3 * j;  // column-major complex index of the reference
-                m.m[3 * i + j].r = (T)r[2 * c];
-                m.m[3 * i + j].i = (T)r[2 * c + 1];
-            }
-        if (GEN)
-            stm(soa, (unsigned)V, mu, (unsigned)s, m);
-        else
-            stu(soa, (unsigned)V, mu, (unsigned)s, m);
-    }
+        for (int j = 0; j < 3; j++) {
+            const dvec2 v = sh[9 * lane + i + 3 * j];  // column-major complex index of the reference
+            m.m[3 * i + j].r = (T)v.x;
+            m.m[3 * i + j].i = (T)v.y;
+        }
+    if (GEN)
+        stm(soa, (unsigned)V, mu, (unsigned)(s0 + lane), m);
+    else
+        stu(soa, (unsigned)V, mu, (unsigned)(s0 + lane), m);
 }
 template <typename T, bool GEN>
-__global__ __launch_bounds__(kBlock) void k_links_to_ref(const T* __restrict__ soa, double* __restrict__ ref, int V) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    for (int mu = 0; mu < 4; mu++) {
-        double* r = ref + ((size_t)mu * V + s) * 18;
+__global__ __launch_bounds__(kBlock) void k_links_to_ref(const T* __restrict__ soa, double* __restrict__ ref, int V,
+                                                         int q0, int nq) {
+    __shared__ dvec2 buf[kBlock / 64][64 * 9];
+    const int lane = (int)(threadIdx.x & 63u);
+    dvec2* const sh = buf[threadIdx.x >> 6];
+    int mu, s0, n;
+    if (!group_at(V, q0, nq, mu, s0, n)) return;
+    if (lane < n) {
+        const unsigned s = (unsigned)(s0 + lane);
         // SU(3) links: the stored rows widened, row 2 rebuilt in double (as the FP64 sums use them)
-        const M3<double> m = GEN ? to_f64(ldm(soa, (unsigned)V, mu, (unsigned)s))
-                                 : full_of(r6_f64(ldr(soa, (unsigned)V, mu, (unsigned)s)));
+        const M3<double> m =
+            GEN ? to_f64(ldm(soa, (unsigned)V, mu, s)) : full_of(r6_f64(ldr(soa, (unsigned)V, mu, s)));
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const int c = i + 3 * j;
-                r[2 * c] = (double)m.m[3 * i + j].r;
-                r[2 * c + 1] = (double)m.m[3 * i + j].i;
-            }
+            for (int j = 0; j < 3; j++) sh[9 * lane + i + 3 * j] = dvec2{m.m[3 * i + j].r, m.m[3 * i + j].i};
     }
+    words_out<9, 9>(ref + piece<18>(V, q0, mu, s0), sh, lane, 9 * n);
 }
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_momenta_from_ref(const double* __restrict__ ref, T* __restrict__ soa, int V) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    for (int mu = 0; mu < 4; mu++) {
-        T c[8];
+__global__ __launch_bounds__(kBlock) void k_momenta_from_ref(const double* __restrict__ ref, T* __restrict__ soa,
+                                                             int V, int q0, int nq) {
+    __shared__ dvec2 buf[kBlock / 64][64 * 5];
+    const int lane = (int)(threadIdx.x & 63u);
+    dvec2* const sh = buf[threadIdx.x >> 6];
+    int mu, s0, n;
+    if (!group_at(V, q0, nq, mu, s0, n)) return;
+    words_in<4, 5>(ref + piece<8>(V, q0, mu, s0), sh, lane, 4 * n);
+    if (lane >= n) return;
+    T c[8];
 #pragma unroll
-        for (int a = 0; a < 8; a++) c[a] = (T)ref[((size_t)mu * V + s) * 8 + a];
-        stp(soa, (unsigned)V, mu, (unsigned)s, c);
+    for (int a = 0; a < 4; a++) {
+        const dvec2 v = sh[5 * lane + a];
+        c[2 * a] = (T)v.x;
+        c[2 * a + 1] = (T)v.y;
     }
+    stp(soa, (unsigned)V, mu, (unsigned)(s0 + lane), c);
 }
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_momenta_to_ref(const T* __restrict__ soa, double* __restrict__ ref, int V) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= V) return;
-    for (int mu = 0; mu < 4; mu++) {
+__global__ __launch_bounds__(kBlock) void k_momenta_to_ref(const T* __restrict__ soa, double* __restrict__ ref, int V,
+                                                           int q0, int nq) {
+    __shared__ dvec2 buf[kBlock / 64][64 * 5];
+    const int lane = (int)(threadIdx.x & 63u);
+    dvec2* const sh = buf[threadIdx.x >> 6];
+    int mu, s0, n;
+    if (!group_at(V, q0, nq, mu, s0, n)) return;
+    if (lane < n) {
         T c[8];
-        ldp(soa, (unsigned)V, mu, (unsigned)s, c);
+        ldp(soa, (unsigned)V, mu, (unsigned)(s0 + lane), c);
 #pragma unroll
-        for (int a = 0; a < 8; a++) ref[((size_t)mu * V + s) * 8 + a] = (double)c[a];
+        for (int a = 0; a < 4; a++) sh[5 * lane + a] = dvec2{(double)c[2 * a], (double)c[2 * a + 1]};
     }
+    words_out<4, 5>(ref + piece<8>(V, q0, mu, s0), sh, lane, 4 * n);
 }
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_set_identity(T* __restrict__ U, int V) {
@@ -487,29 +544,29 @@ hipError_t launch_links_widen(const float* Uf, double* Ud, int V, hipStream_t st
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_links_from_ref(const double* ref, T* soa, int V, bool general, hipStream_t st) {
+hipError_t launch_links_from_ref(const double* ref, T* soa, int V, bool general, int q0, int nq, hipStream_t st) {
     if (general)
-        k_links_from_ref<T, true><<<grid_for(V), kBlock, 0, st>>>(ref, soa, V);
+        k_links_from_ref<T, true><<<(nq + 3) / 4, kBlock, 0, st>>>(ref, soa, V, q0, nq);
     else
-        k_links_from_ref<T, false><<<grid_for(V), kBlock, 0, st>>>(ref, soa, V);
+        k_links_from_ref<T, false><<<(nq + 3) / 4, kBlock, 0, st>>>(ref, soa, V, q0, nq);
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_links_to_ref(const T* soa, double* ref, int V, bool general, hipStream_t st) {
+hipError_t launch_links_to_ref(const T* soa, double* ref, int V, bool general, int q0, int nq, hipStream_t st) {
     if (general)
-        k_links_to_ref<T, true><<<grid_for(V), kBlock, 0, st>>>(soa, ref, V);
+        k_links_to_ref<T, true><<<(nq + 3) / 4, kBlock, 0, st>>>(soa, ref, V, q0, nq);
     else
-        k_links_to_ref<T, false><<<grid_for(V), kBlock, 0, st>>>(soa, ref, V);
+        k_links_to_ref<T, false><<<(nq + 3) / 4, kBlock, 0, st>>>(soa, ref, V, q0, nq);
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_momenta_from_ref(const double* ref, T* soa, int V, hipStream_t st) {
-    k_momenta_from_ref<T><<<grid_for(V), kBlock, 0, st>>>(ref, soa, V);
+hipError_t launch_momenta_from_ref(const double* ref, T* soa, int V, int q0, int nq, hipStream_t st) {
+    k_momenta_from_ref<T><<<(nq + 3) / 4, kBlock, 0, st>>>(ref, soa, V, q0, nq);
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_momenta_to_ref(const T* soa, double* ref, int V, hipStream_t st) {
-    k_momenta_to_ref<T><<<grid_for(V), kBlock, 0, st>>>(soa, ref, V);
+hipError_t launch_momenta_to_ref(const T* soa, double* ref, int V, int q0, int nq, hipStream_t st) {
+    k_momenta_to_ref<T><<<(nq + 3) / 4, kBlock, 0, st>>>(soa, ref, V, q0, nq);
     return hipGetLastError();
 }
 template <typename T>
@@ -538,10 +595,10 @@ hipError_t launch_axpby(T* y, const T* x, double a, double b, size_t n, hipStrea
     template hipError_t launch_force<T>(int, const Geo&, const T*, T*, T*, double, double, double,       \
                                         hipStream_t, double*);                                           \
     template hipError_t launch_exp_update<T>(const Geo&, const T*, T*, const T*, double, hipStream_t);   \
-    template hipError_t launch_links_from_ref<T>(const double*, T*, int, bool, hipStream_t);             \
-    template hipError_t launch_links_to_ref<T>(const T*, double*, int, bool, hipStream_t);               \
-    template hipError_t launch_momenta_from_ref<T>(const double*, T*, int, hipStream_t);                 \
-    template hipError_t launch_momenta_to_ref<T>(const T*, double*, int, hipStream_t);                   \
+    template hipError_t launch_links_from_ref<T>(const double*, T*, int, bool, int, int, hipStream_t);   \
+    template hipError_t launch_links_to_ref<T>(const T*, double*, int, bool, int, int, hipStream_t);     \
+    template hipError_t launch_momenta_from_ref<T>(const double*, T*, int, int, int, hipStream_t);       \
+    template hipError_t launch_momenta_to_ref<T>(const T*, double*, int, int, int, hipStream_t);         \
     template hipError_t launch_set_identity<T>(T*, int, hipStream_t);                                    \
     template hipError_t launch_fill<T>(T*, size_t, T, hipStream_t);                                      \
     template hipError_t launch_axpby<T>(T*, const T*, double, double, size_t, hipStream_t);
