@@ -1038,6 +1038,7 @@ static int heatbath_sweep(gf_ctx* c, int mode, double beta, unsigned long long s
         HIPCHK(c, launch_heatbath<T>(c->geo, (T*)c->U, mode, beta, seed, sweep, itmax, c->partial, c->dres, c->stream));
         return GF_OK;
     }));
+    if (mode != 0) return GF_OK;  // overrelaxation always succeeds: nothing to read back
     double f;
     TRY(read_scalar(c, &f));
     if (failures) *failures = (long long)f;

@@ -209,6 +209,10 @@ __device__ __forceinline__ M3<double> to_f64(const M3<T>& a) {
 // projection itself runs in double and only its result is rounded: a float Gram-Schmidt leaves
 // the row norms about 1e-7 too large on average (1/sqrt rounds asymmetrically next to 1), a bias
 // that shows up directly in the plaquette.
+// WRITTEN: which of two products is fused into the sum is spelt out rather than left to the compiler, which
+// decides by the code around it.  An ensemble's links follow its last bits after some twenty sweeps, so a change
+// elsewhere in the overrelaxation kernel would otherwise give another (equally good) ensemble.
+template <bool WRITTEN = false>
 __device__ __forceinline__ void reunitarize_f64(M3<double>& u) {
     cx<double> r1[3], r2[3];
 #pragma unroll
@@ -219,9 +223,15 @@ __device__ __forceinline__ void reunitarize_f64(M3<double>& u) {
     double w2 = 0.0, w1r = 0.0, w1i = 0.0;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        w2 += r1[c].r * r1[c].r + r1[c].i * r1[c].i;
-        w1r += r2[c].r * r1[c].r + r2[c].i * r1[c].i;  // row2 . conj(row1)
-        w1i += r2[c].i * r1[c].r - r2[c].r * r1[c].i;
+        if constexpr (WRITTEN) {
+            w2 += fma(r1[c].i, r1[c].i, r1[c].r * r1[c].r);
+            w1r += fma(r2[c].i, r1[c].i, r2[c].r * r1[c].r);
+            w1i += fma(r2[c].i, r1[c].r, -(r2[c].r * r1[c].i));
+        } else {
+            w2 += r1[c].r * r1[c].r + r1[c].i * r1[c].i;
+            w1r += r2[c].r * r1[c].r + r2[c].i * r1[c].i;  // row2 . conj(row1)
+            w1i += r2[c].i * r1[c].r - r2[c].r * r1[c].i;
+        }
     }
     // Rows that are unit to within |d| <= 2^-14 (every updated link: an exactly unitary factor
     // times a stored link) take 1/(1+d) and 1/sqrt(1+d) from their series to d^4 (truncation

@@ -63,6 +63,24 @@ def test_overrelaxation_matches_oracle_and_keeps_action(Lat, oracle, dims):
     assert L.plaquette_sum() == pytest.approx(p0, rel=1e-13)
 
 
+@pytest.mark.parametrize("dims", [(2, 2, 2, 2), (6, 10, 2, 2), (4, 6, 2, 8), (16, 8, 8, 8), (18, 4, 6, 10)])
+def test_sweep_edges(Lat, oracle, dims):
+    """Idle lanes, remainders, rows cut by the waves, the tiled order, all three subgroups; refused proposals are counted and leave the
+    link alone.  Bounds as above."""
+    print(f"[heatbath] edges {dims}", flush=True)
+    U = oracle.hot_links(dims, 21)
+    for itmax in (1000, 1):
+        L = Lat(dims)
+        L.upload_links(U)
+        W = U.copy()
+        f = L.heatbath(2.0, 7, 3, itmax=itmax)
+        fo = oracle.heatbath_sweep(dims, W, 2.0, 7, 3, itmax=itmax)
+        assert f == fo and (f == 0) == (itmax > 1)
+        L.overrelaxation(7, 4)
+        oracle.heatbath_sweep(dims, W, 2.0, 7, 4, overrelax=True)
+        assert np.abs(L.download_links() - W).max() < 1e-9
+
+
 def test_heatbath_strong_coupling_and_fp32(Lat):
     dims = (8, 8, 8, 8)
     for prec in ("f64", "f32"):
