@@ -217,9 +217,9 @@ int need_staging(gf_ctx* c) {
 }
 
 // Host arrays.  (4, V, W) doubles go in units of a wave's links (group q: k_links_to_ref), plain ones by 4 KB.
-int need_ring(gf_ctx* c) {
-    const hipError_t e = c->ring.need((size_t)72 * c->V * sizeof(double), c->device);
-    return e == hipSuccess ? GF_OK : fail(c, GF_ENOMEM, "pinned host memory: %s", hipGetErrorString(e));
+int ring_result(gf_ctx* c, hipError_t e) {
+    if (e == hipSuccess) return GF_OK;
+    return fail(c, e == hipErrorOutOfMemory ? GF_ENOMEM : GF_EDEVICE, "copy to or from the host: %s", hipGetErrorString(e));
 }
 struct GroupBytes {
     size_t V, groups, link;  // link: bytes
@@ -230,10 +230,8 @@ struct GroupBytes {
 // launch(q0, n, slot) on the groups q0 .. q0 + n
 template <typename F>
 int pull_groups(gf_ctx* c, double* dst, int reals, F launch) {
-    TRY(need_ring(c));
     const GroupBytes at(c, reals);
-    HIPCHK(c, c->ring.pull((char*)dst, at.units(), 64 * at.link, at, launch, c->stream));
-    return GF_OK;
+    return ring_result(c, c->ring.pull((char*)dst, at.units(), 64 * at.link, at, launch, c->stream));
 }
 template <typename F>
 int push_groups(gf_ctx* c, const double* src, int reals, F launch) {
@@ -245,9 +243,7 @@ int push_groups(gf_ctx* c, const double* src, int reals, F launch) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return GF_OK;
     }
-    TRY(need_ring(c));
-    HIPCHK(c, c->ring.push((const char*)src, at.units(), 64 * at.link, at, launch, c->stream));
-    return GF_OK;
+    return ring_result(c, c->ring.push((const char*)src, at.units(), 64 * at.link, at, launch, c->stream));
 }
 int pull_plain(gf_ctx* c, double* dst, const double* src, size_t n) {
     const size_t bytes = n * sizeof(double), unit = 4096;
@@ -256,15 +252,14 @@ int pull_plain(gf_ctx* c, double* dst, const double* src, size_t n) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return GF_OK;
     }
-    TRY(need_ring(c));
-    HIPCHK(c, c->ring.pull(
-                  (char*)dst, (long)((bytes + unit - 1) / unit), unit, [&](long q) { return std::min(bytes, q * unit); },
-                  [&](long q, long k, char* p) {
-                      const size_t a = q * unit, b = std::min(bytes, a + k * unit);
-                      return hipMemcpyAsync(p, (const char*)src + a, b - a, hipMemcpyDeviceToHost, c->stream);
-                  },
-                  c->stream));
-    return GF_OK;
+    const hipError_t e = c->ring.pull(
+        (char*)dst, (long)((bytes + unit - 1) / unit), unit, [&](long q) { return std::min(bytes, q * unit); },
+        [&](long q, long k, char* p) {
+            const size_t a = q * unit, b = std::min(bytes, a + k * unit);
+            return hipMemcpyAsync(p, (const char*)src + a, b - a, hipMemcpyDeviceToHost, c->stream);
+        },
+        c->stream);
+    return ring_result(c, e);
 }
 
 template <typename T>
@@ -644,7 +639,12 @@ int gf_create(const int* dims, int precision, int device, gf_ctx** out) {
         alloc(c, (void**)&c->partial, sizeof(double) * (4 * ((size_t)grid_sites_mu(c->V) + c->dims[3]) + 16)) ||
         alloc(c, (void**)&c->dres, 4 * sizeof(double)))
         return bail(GF_ENOMEM);
-    if (hipHostMalloc((void**)&c->hres, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) return bail(GF_ENOMEM);
+    const size_t largest = (size_t)72 * c->V * sizeof(double), page = 4096;
+    c->ring.shape(largest, c->device);
+    const int n_slots = c->ring.slots_at_hand(largest);
+    if (hipHostMalloc((void**)&c->hres, page + c->ring.slot * n_slots, hipHostMallocDefault) != hipSuccess)
+        return bail(GF_ENOMEM);
+    c->ring.adopt((char*)c->hres + page, n_slots);
     if (c->s64 && (alloc(c, &c->U64, link64_bytes(c)) || alloc(c, &c->P64, (size_t)32 * c->V * sizeof(double))))
         return bail(GF_ENOMEM);
     int r = gf_set_cold(c);

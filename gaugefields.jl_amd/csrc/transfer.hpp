@@ -150,29 +150,48 @@ constexpr int kSlots = 16;
 constexpr size_t kSlotMin = 256 << 10, kSlotMax = 2 << 20, kUnitMax = 64 * 144;  // a group's links
 
 struct HostRing {
-    char* pinned = nullptr;
-    size_t slot = 0;  // bytes
-    int slots = 0, device = 0;
-    bool helped = false;
+    char* slot_at[kSlots] = {};  // pinned, as transfers come to need them
+    char* piece[kSlots] = {};    // the allocations they lie in
     hipEvent_t ev[kSlots] = {};
+    size_t slot = 0;  // bytes
+    int device = 0;
+    bool helped = false;
 
     // `most`: the largest transfer of the context.  A slot holds 1/32 of it, 256 KB to 2 MB: each costs a launch and
-    // an event, 4 us during which the link is idle (512 KB slots 29 GB/s, 1 MB 43, 2 MB 48, 4 MB 50), and the ring
-    // has to be pinned first, which takes about as long as a transfer of its size.
-    hipError_t need(size_t most, int dev) {
-        if (pinned) return hipSuccess;
+    // an event, 4 us during which the link is idle (512 KB slots 29 GB/s, 1 MB 43, 2 MB 48, 4 MB 50).
+    void shape(size_t most, int dev) {
         device = dev;
         slot = most <= kSlotMin ? std::max(most, kUnitMax) : std::min(std::max(most / 32, kSlotMin), kSlotMax);
         slot = (slot + 4095) / 4096 * 4096;
-        slots = (int)std::min<size_t>(kSlots, (most + slot - 1) / slot);
-        for (int k = 0; k < slots; k++)
-            if (!ev[k]) {
-                const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-                if (e != hipSuccess) return e;
+    }
+    // Slots that the context pins with its other host memory: all that a small lattice needs (up to 1 MB)
+    int slots_at_hand(size_t most) const { return slot <= kSlotMin ? (int)std::min<size_t>(4, (most + slot - 1) / slot) : 0; }
+    void adopt(char* p, int n) {
+        for (int k = 0; k < n; k++) slot_at[k] = p + slot * k;
+    }
+    // Slots for a transfer of `chunks` slots: half of them, 4 to 16, as pinning takes about as long as copying,
+    // and in one piece, as pinning any piece takes 0.3 ms; what there is if there is no more pinned memory, and 0 if
+    // there is none at all (err).
+    int slots_for(long chunks, hipError_t& err) {
+        const int n = (int)std::min<long>(chunks, std::min<long>(std::max(chunks / 2, 4L), kSlots));
+        int have = 0;
+        while (have < kSlots && slot_at[have]) have++;
+        for (int more = n - have; more > 0 && have < n; more = std::min(more / 2, n - have)) {
+            char* p = nullptr;
+            err = hipHostMalloc((void**)&p, slot * more, hipHostMallocDefault);
+            if (err != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
             }
-        const hipError_t e = hipHostMalloc((void**)&pinned, slot * slots, hipHostMallocDefault);
-        if (e != hipSuccess) pinned = nullptr;
-        return e;
+            piece[have] = p;
+            for (int k = 0; k < more; k++) slot_at[have + k] = p + slot * k;
+            have += more;
+        }
+        for (int k = 0; k < std::min(n, have); k++) {
+            if (!ev[k]) err = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+            if (!ev[k]) return k;
+        }
+        return std::min(n, have);
     }
     void need_helpers() {
         if (!helped) Helpers::get().retain();
@@ -181,8 +200,11 @@ struct HostRing {
     void free() {
         if (helped) Helpers::get().release();
         helped = false;
-        if (pinned) (void)hipHostFree(pinned);
-        pinned = nullptr;
+        for (char*& p : piece) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+        }
+        for (char*& p : slot_at) p = nullptr;
         for (hipEvent_t& e : ev) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
@@ -197,19 +219,22 @@ struct HostRing {
         char* const host;
         const bool down;
         const long units, per;
-        long last[kSlots];  // last chunk copied between the slot and the host array
         hipError_t err = hipSuccess;
+        int slots;
+        long last[kSlots];  // last chunk copied between the slot and the host array
         Transfer(HostRing& ring, char* h, bool d, long n, size_t unit_bytes, const O& o)
             : r(ring), offset(o), host(h), down(d), units(n), per((long)(ring.slot / unit_bytes)) {
             total = (units + per - 1) / per;
+            slots = ring.slots_for(total, err);
+            if (slots > 0) err = hipSuccess;
             for (long& k : last) k = -1;
         }
-        char* at(long i) const { return r.pinned + (size_t)(i % r.slots) * r.slot; }
-        bool copied(long i) const { return last[i % r.slots] == i; }
+        char* at(long i) const { return r.slot_at[i % slots]; }
+        bool copied(long i) const { return last[i % slots] == i; }
         void run(long i) override {
             if (down) {
                 (void)hipSetDevice(r.device);
-                const hipError_t e = hipEventSynchronize(r.ev[i % r.slots]);
+                const hipError_t e = hipEventSynchronize(r.ev[i % slots]);
                 if (e != hipSuccess) {
                     Helpers::get().check([&] { return err = e, true; });
                     return;
@@ -221,11 +246,11 @@ struct HostRing {
             else
                 memcpy(at(i), host + a, b - a);
         }
-        void ran(long i) override { last[i % r.slots] = i; }
+        void ran(long i) override { last[i % slots] = i; }
         template <typename F>
         hipError_t launch(long i, F f, hipStream_t st) {
             const hipError_t e = f(i * per, std::min(per, units - i * per), at(i));
-            return e == hipSuccess ? hipEventRecord(r.ev[i % r.slots], st) : e;
+            return e == hipSuccess ? hipEventRecord(r.ev[i % slots], st) : e;
         }
     };
 
@@ -235,6 +260,8 @@ struct HostRing {
     hipError_t pull(char* dst, long units, size_t unit_bytes, const O& offset, F fill, hipStream_t st) {
         Helpers& h = Helpers::get();
         Transfer<O> t(*this, dst, true, units, unit_bytes, offset);
+        if (t.slots == 0) return t.err;
+        const int slots = t.slots;
         const bool share = t.total >= 4;
         if (share) need_helpers();
         hipError_t e = hipSuccess;
@@ -271,6 +298,8 @@ struct HostRing {
     hipError_t push(const char* src, long units, size_t unit_bytes, const O& offset, F drain, hipStream_t st) {
         Helpers& h = Helpers::get();
         Transfer<O> t(*this, const_cast<char*>(src), false, units, unit_bytes, offset);
+        if (t.slots == 0) return t.err;
+        const int slots = t.slots;
         hipError_t e = hipSuccess;
         long issued = 0, freed = 0;  // chunks on the device's side, and those it has read
         t.limit = slots;
