@@ -20,6 +20,8 @@ using namespace gf;
 #define GF_MAX_LEV 8
 #define GF_NEVENTS 16
 
+constexpr int kRes = 512;
+
 struct gf_ctx {
     int dims[4] = {0, 0, 0, 0};
     Geo geo{};
@@ -61,8 +63,7 @@ struct gf_ctx {
     double* staging = nullptr;  // 18 V doubles
     HostRing ring;              // host arrays in and out
     double* partial = nullptr;
-    double* dres = nullptr;   // device scalar
-    double* hres = nullptr;   // pinned host scalar
+    double* hres = nullptr;   // kRes pinned scalars, which the kernels write
     size_t bytes = 0;
     hipEvent_t ev[GF_NEVENTS] = {};
     std::string err;
@@ -293,36 +294,31 @@ int dispatch(gf_ctx* c, F&& f) {
     return c->prec == GF_F64 ? f((double*)nullptr) : f((float*)nullptr);
 }
 
+// The sums of a measurement are written to pinned memory by the kernels that add them up, and are there after the
+// next wait.  What is measured along a trajectory or flow is read with one wait at its end.
 int read_scalar(gf_ctx* c, double* out) {
-    HIPCHK(c, hipMemcpyAsync(c->hres, c->dres, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     *out = *c->hres;
     return GF_OK;
 }
 
-int plaq_of(gf_ctx* c, void* U, double* sum) {
-    TRY(dispatch(c, [&](auto* tag) -> int {
+int plaq_queue(gf_ctx* c, const void* U, double* at) {
+    return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_plaquette<T>(c->geo, (const T*)U, c->partial, c->dres, c->stream));
+        HIPCHK(c, launch_plaquette<T>(c->geo, (const T*)U, c->partial, at, c->stream));
         return GF_OK;
-    }));
-    return read_scalar(c, sum);
+    });
 }
 
 void swap_links(gf_ctx* c) { std::swap(c->U, c->Ualt); }
 
 // field-strength observables of the current links: out = {clover energy sum, Q plaquette,
 // Q clover, Q rectangle}; dens_host (V doubles) receives the density of dens_method if non-null
-int fstrength(gf_ctx* c, int sets, double out[4], double* dens_host, int dens_method) {
+int fstrength_queue(gf_ctx* c, int sets, double* at, double* dens, int dens_method) {
     if (c->s64)
         return fail(c, GF_ESTATE,
                     "field-strength measurements are not available in the FP32-force form (FP64 links and momenta, "
                     "forces in FP32); use a GF_F64 or GF_F32 context");
-    double* dens = nullptr;
-    if (dens_host) {
-        TRY(need_staging(c));
-        dens = c->staging;
-    }
     const size_t need = field_strength_bytes(c->geo, sets);
     if (need > c->loops_bytes) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -331,15 +327,18 @@ int fstrength(gf_ctx* c, int sets, double out[4], double* dens_host, int dens_me
         TRY(alloc(c, &c->loops, need));
         c->loops_bytes = need;
     }
-    TRY(dispatch(c, [&](auto* tag) -> int {
+    return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->loops, c->partial, c->dres, dens,
-                                           dens_method, c->stream));
+        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->loops, c->partial, at, dens, dens_method,
+                                           c->stream));
         return GF_OK;
-    }));
-    HIPCHK(c, hipMemcpyAsync(c->hres, c->dres, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    });
+}
+int fstrength(gf_ctx* c, int sets, double out[4], double* dens_host, int dens_method) {
+    if (dens_host && !c->s64) TRY(need_staging(c));
+    TRY(fstrength_queue(c, sets, c->hres, dens_host ? c->staging : nullptr, dens_method));
     if (dens_host)
-        TRY(pull_plain(c, dens_host, dens, c->V));
+        TRY(pull_plain(c, dens_host, c->staging, c->V));
     else
         HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int k = 0; k < 4; k++) out[k] = c->hres[k];
@@ -524,14 +523,20 @@ int kick_exp(gf_ctx* c, double coeff, double eps_p, double eps_u) {
 // add configuration-dependent noise of ~2e-3 to the smeared action at 32^4, more than the
 // deviation the FP32 trajectory itself causes; the forces stay FP32.
 // With an FP64 state the held FP64 links are smeared directly.
-int action_plaq_fp64(gf_ctx* c, double* plaq) {
+// Leaves the sums over the workgroups to the caller (partial).
+int action_plaq_fp64(gf_ctx* c, double* partial) {
     if (c->prec == GF_F64) {
         if (c->nlev > 0) TRY(stout_forward_all(c));
-        return plaq_of(c, (void*)top_links(c), plaq);
+        HIPCHK(c, launch_plaquette<double>(c->geo, (const double*)top_links(c), partial, nullptr, c->stream));
+        return GF_OK;
+    }
+    if (!c->s64 && c->nlev == 0) {  // widened as they are read
+        HIPCHK(c, launch_plaquette<float>(c->geo, (const float*)c->U, partial, nullptr, c->stream));
+        return GF_OK;
     }
     const size_t b64 = link64_bytes(c);
-    if (!c->s64 || c->nlev > 0) TRY(alloc(c, &c->W64[0], b64));
-    if (c->nlev > 1 || (!c->s64 && c->nlev > 0)) TRY(alloc(c, &c->W64[1], b64));
+    if (c->nlev > 0) TRY(alloc(c, &c->W64[0], b64));
+    if (c->nlev > 1 || !c->s64) TRY(alloc(c, &c->W64[1], b64));
     if (!c->s64) HIPCHK(c, launch_links_widen((const float*)c->U, (double*)c->W64[0], c->V, c->stream));
     // level l reads src and writes W64[l & 1] (the FP64 state is never overwritten)
     const double* src = c->s64 ? (const double*)c->U64 : (const double*)c->W64[0];
@@ -540,33 +545,49 @@ int action_plaq_fp64(gf_ctx* c, double* plaq) {
         HIPCHK(c, launch_stout_forward<double>(c->geo, src, (double*)c->W64[cur], nullptr, c->rho, c->stream));
         src = (const double*)c->W64[cur];
     }
-    HIPCHK(c, launch_plaquette<double>(c->geo, src, c->partial, c->dres, c->stream));
-    return read_scalar(c, plaq);
+    HIPCHK(c, launch_plaquette<double>(c->geo, src, partial, nullptr, c->stream));
+    return GF_OK;
 }
 // plaquette sum of the configuration's links (the FP64 state where there is one)
+int plaq_state_queue(gf_ctx* c, double* at) {
+    if (!c->s64) return plaq_queue(c, c->U, at);
+    HIPCHK(c, launch_plaquette<double>(c->geo, (const double*)c->U64, c->partial, at, c->stream));
+    return GF_OK;
+}
 int plaq_state(gf_ctx* c, double* sum) {
-    if (!c->s64) return plaq_of(c, c->U, sum);
-    HIPCHK(c, launch_plaquette<double>(c->geo, (const double*)c->U64, c->partial, c->dres, c->stream));
+    TRY(plaq_state_queue(c, c->hres));
     return read_scalar(c, sum);
 }
-int momenta_dot(gf_ctx* c, double* pp) {
+// p*p, its sum over the workgroups left to the caller where at is null
+int momenta_dot_queue(gf_ctx* c, double* partial, double* at) {
     if (c->s64) {
-        HIPCHK(c, launch_momenta_dot<double>(c->geo, (const double*)c->P64, c->partial, c->dres, c->stream));
-    } else {
-        TRY(dispatch(c, [&](auto* tag) -> int {
-            using T = std::remove_pointer_t<decltype(tag)>;
-            HIPCHK(c, launch_momenta_dot<T>(c->geo, (const T*)c->P, c->partial, c->dres, c->stream));
-            return GF_OK;
-        }));
+        HIPCHK(c, launch_momenta_dot<double>(c->geo, (const double*)c->P64, partial, at, c->stream));
+        return GF_OK;
     }
+    return dispatch(c, [&](auto* tag) -> int {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        HIPCHK(c, launch_momenta_dot<T>(c->geo, (const T*)c->P, partial, at, c->stream));
+        return GF_OK;
+    });
+}
+int momenta_dot(gf_ctx* c, double* pp) {
+    TRY(momenta_dot_queue(c, c->partial, c->hres));
     return read_scalar(c, pp);
 }
 
+// at[0] p*p, at[1] the action's plaquette sum
+int hamiltonian_queue(gf_ctx* c, double* at) {
+    const int nb = grid_sites_mu(c->V);
+    TRY(momenta_dot_queue(c, c->partial, nullptr));
+    TRY(action_plaq_fp64(c, c->partial + nb));
+    HIPCHK(c, launch_sum_partials(c->partial, nb, 2, at, c->stream));
+    return GF_OK;
+}
+double hamiltonian_of(double coeff, const double* at) { return -2.0 * coeff * at[1] / 3.0 + 0.5 * at[0]; }
 int hamiltonian(gf_ctx* c, double coeff, double* H) {
-    double pp = 0.0, plaq = 0.0;
-    TRY(momenta_dot(c, &pp));
-    TRY(action_plaq_fp64(c, &plaq));
-    *H = -2.0 * coeff * plaq / 3.0 + 0.5 * pp;
+    TRY(hamiltonian_queue(c, c->hres));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    *H = hamiltonian_of(coeff, c->hres);
     return GF_OK;
 }
 
@@ -636,10 +657,9 @@ int gf_create(const int* dims, int precision, int device, gf_ctx** out) {
         if (hipEventCreate(&c->ev[i]) != hipSuccess) return bail(GF_EDEVICE);
     if (alloc(c, &c->U, link_bytes(c)) || alloc(c, &c->Ualt, link_bytes(c)) || alloc(c, &c->P, mom_bytes(c)) ||
         alloc(c, &c->F, mom_bytes(c)) ||
-        alloc(c, (void**)&c->partial, sizeof(double) * (4 * ((size_t)grid_sites_mu(c->V) + c->dims[3]) + 16)) ||
-        alloc(c, (void**)&c->dres, 4 * sizeof(double)))
+        alloc(c, (void**)&c->partial, sizeof(double) * (4 * ((size_t)grid_sites_mu(c->V) + c->dims[3]) + 16)))
         return bail(GF_ENOMEM);
-    const size_t largest = (size_t)72 * c->V * sizeof(double), page = 4096;
+    const size_t largest = (size_t)72 * c->V * sizeof(double), page = kRes * sizeof(double);
     c->ring.shape(largest, c->device);
     const int n_slots = c->ring.slots_at_hand(largest);
     if (hipHostMalloc((void**)&c->hres, page + c->ring.slot * n_slots, hipHostMallocDefault) != hipSuccess)
@@ -671,7 +691,6 @@ int gf_destroy(gf_ctx* c) {
     if (c->staging) (void)hipFree(c->staging);
     c->ring.free();
     if (c->partial) (void)hipFree(c->partial);
-    if (c->dres) (void)hipFree(c->dres);
     if (c->hres) (void)hipHostFree(c->hres);
     for (int i = 0; i < GF_NEVENTS; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -951,8 +970,7 @@ int gf_md_trajectory(gf_ctx* c, double coeff, int integrator, double lambda, int
     if (tau == 0.0) return fail(c, GF_EINVAL, "trajectory_length must not be zero");
     if (kind != GF_QPQ && kind != GF_PQP && kind != GF_OMELYAN2MN)
         return fail(c, GF_EINVAL, "unknown integrator %d", integrator);
-    double h0 = 0.0;
-    if (H) TRY(hamiltonian(c, coeff, &h0));
+    if (H) TRY(hamiltonian_queue(c, c->hres));
     const double e = tau / steps;
     // Neighbouring sub-steps of the same kind are one: the links do not change between the closing
     // kick of one step and the opening kick of the next, so their forces are the same and one kick of
@@ -976,21 +994,22 @@ int gf_md_trajectory(gf_ctx* c, double coeff, int integrator, double lambda, int
         TRY(kick(c, coeff, lambda * e));
     }
     if (H) {
-        double h1 = 0.0;
-        TRY(hamiltonian(c, coeff, &h1));
-        H[0] = h0;
-        H[1] = h1;
-        H[2] = h1 - h0;
+        TRY(hamiltonian_queue(c, c->hres + 2));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        H[0] = hamiltonian_of(coeff, c->hres);
+        H[1] = hamiltonian_of(coeff, c->hres + 2);
+        H[2] = H[1] - H[0];
     }
     return GF_OK;
 }
 
+static double energy_density_of(const gf_ctx* c, double plaq) { return 2.0 * (18.0 - plaq / (double)c->V); }
 int gf_energy_density(gf_ctx* c, double* E) {
     CTXCHK(c);
     if (!E) return GF_EINVAL;
     double s;
     TRY(plaq_state(c, &s));
-    *E = 2.0 * (18.0 - s / (double)c->V);
+    *E = energy_density_of(c, s);
     return GF_OK;
 }
 
@@ -1035,7 +1054,7 @@ static int heatbath_sweep(gf_ctx* c, int mode, double beta, unsigned long long s
     if (mode == 0 && !(beta > 0.0 && std::isfinite(beta))) return fail(c, GF_EINVAL, "beta must be positive; got %g", beta);
     TRY(dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_heatbath<T>(c->geo, (T*)c->U, mode, beta, seed, sweep, itmax, c->partial, c->dres, c->stream));
+        HIPCHK(c, launch_heatbath<T>(c->geo, (T*)c->U, mode, beta, seed, sweep, itmax, c->partial, c->hres, c->stream));
         return GF_OK;
     }));
     if (mode != 0) return GF_OK;  // overrelaxation always succeeds: nothing to read back
@@ -1090,25 +1109,28 @@ int gf_flow_measure(gf_ctx* c, double eps, int nsteps, int every, double* out) {
     NOT_S64(c, "flow!");
     if (every <= 0) return fail(c, GF_EINVAL, "every must be positive; got %d", every);
     if (!out) return fail(c, GF_EINVAL, "out is required");
-    int k = 0;
-    for (int done = 0; done < nsteps;) {
-        const int n = std::min(every, nsteps - done);
-        TRY(gf_flow(c, eps, n, 0, nullptr));
-        done += n;
-        if (n == every) {
-            double plaq, o[4];
-            TRY(plaq_of(c, c->U, &plaq));
-            TRY(fstrength(c, 7, o, nullptr, 0));
-            double* r = out + (size_t)GF_FLOW_NOBS * k++;
-            r[0] = eps * done;
-            r[1] = plaq / (18.0 * (double)c->V);
-            r[2] = 2.0 * (18.0 - plaq / (double)c->V);
-            r[3] = o[0] / (double)c->V;
-            r[4] = o[1];
-            r[5] = o[2];
-            r[6] = topo_of(GF_TOPO_IMPROVED, o);
+    // a row's five sums: plaquette, {clover energy, Q plaquette, Q clover, Q rectangle}
+    const int rows = nsteps / every;
+    for (int k = 0, read = 0; k < rows; k++) {
+        TRY(gf_flow(c, eps, every, 0, nullptr));
+        double* const at = c->hres + 5 * (k - read);
+        TRY(plaq_queue(c, c->U, at));
+        TRY(fstrength_queue(c, 7, at + 1, nullptr, 0));
+        if (k + 1 < rows && 5 * (k + 2 - read) <= kRes) continue;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        for (; read <= k; read++) {
+            const double* const a = c->hres + (at - c->hres) - 5 * (k - read);
+            double* const r = out + (size_t)GF_FLOW_NOBS * read;
+            r[0] = eps * (every * (read + 1));
+            r[1] = a[0] / (18.0 * (double)c->V);
+            r[2] = energy_density_of(c, a[0]);
+            r[3] = a[1] / (double)c->V;
+            r[4] = a[2];
+            r[5] = a[3];
+            r[6] = topo_of(GF_TOPO_IMPROVED, a + 1);
         }
     }
+    if (nsteps % every > 0) TRY(gf_flow(c, eps, nsteps % every, 0, nullptr));
     return GF_OK;
 }
 
@@ -1119,7 +1141,7 @@ int gf_flow(gf_ctx* c, double eps, int nsteps, int every, double* E_out) {
     if (!(eps > 0.0) || !std::isfinite(eps)) return fail(c, GF_EINVAL, "step_size must be positive; got %g", eps);
     if (every > 0 && !E_out) return fail(c, GF_EINVAL, "E_out is required when every > 0");
     TRY(alloc(c, &c->A, mom_bytes(c)));
-    int k = 0;
+    int k = 0, read = 0;  // energies queued and read
     for (int step = 1; step <= nsteps; step++) {
         TRY(dispatch(c, [&](auto* tag) -> int {
             using T = std::remove_pointer_t<decltype(tag)>;
@@ -1131,7 +1153,11 @@ int gf_flow(gf_ctx* c, double eps, int nsteps, int every, double* E_out) {
             return GF_OK;
         }));
         swap_links(c);
-        if (every > 0 && step % every == 0) TRY(gf_energy_density(c, &E_out[k++]));
+        if (every <= 0 || step % every != 0) continue;
+        TRY(plaq_queue(c, c->U, c->hres + (k++ - read)));
+        if (step + every <= nsteps && k - read < kRes) continue;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        for (const int first = read; read < k; read++) E_out[read] = energy_density_of(c, c->hres[read - first]);
     }
     return GF_OK;
 }

@@ -87,7 +87,8 @@ hipError_t launch_stream_copy(const void* src, void* dst, size_t bytes, hipStrea
 // FP64 link rows 0-1 (optionally SU(3)-projected first) and/or momenta rounded to float in place
 hipError_t launch_round_f32(double* U, double* P, int V, bool links, bool project, bool momenta, hipStream_t st);
 // out[0] = sum of partial[0..n) (one workgroup, fixed order)
-hipError_t launch_sum_partials(const double* partial, int n, double* out, hipStream_t st);
+hipError_t launch_sum_partials(const double* partial, int n, int sums, double* out, hipStream_t st);
+// out null: the per-workgroup partials (grid_sites_mu(V) of them) only
 template <typename T>
 hipError_t launch_plaquette(const Geo& g, const T* U, double* partial, double* out, hipStream_t st);
 template <typename T>

@@ -347,15 +347,6 @@ __global__ __launch_bounds__(192) void k_charge(Geo g, const T* __restrict__ U, 
     }
 }
 
-// out[k] = sum of partial[k * n .. k * n + n), one workgroup per k (fixed order)
-__global__ __launch_bounds__(1024) void k_sum_partials4(const double* __restrict__ partial, int n,
-                                                        double* __restrict__ out) {
-    const double* const p = partial + (size_t)blockIdx.x * n;
-    double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += 1024) v += p[i];
-    block_sum_store<1024>(v, out);
-}
-
 static int fields_of(int sets) { return (sets & 1) + 2 * ((sets >> 1) & 1) + 3 * ((sets >> 2) & 1); }
 // Blocks of whole t-slices: as many as keep the fields of a block near kFieldBytes, evenly, at least one; all
 // of them where there are no fields (the plaquette set alone, whose sites are then visited as the stencil
@@ -404,8 +395,7 @@ hipError_t launch_field_strength(const Geo& g, const T* U, int sets, void* field
         case 7: launch_sets<T, 7>(g, U, f, partial, stride, dens, dens_method, st); break;
         default: return hipErrorInvalidValue;
     }
-    k_sum_partials4<<<4, 1024, 0, st>>>(partial, stride, out4);
-    return hipGetLastError();
+    return launch_sum_partials(partial, stride, 4, out4, st);
 }
 
 #define GF_INST_FS(T)                                                                                            \

@@ -132,19 +132,28 @@ __global__ __launch_bounds__(kBlock) void k_momenta_dot(Geo g, const T* __restri
     block_sum_store<kBlock>(v, partial);
 }
 
-// deterministic final sum of per-block partials (one block)
-__global__ __launch_bounds__(1024) void k_sum_partials(const double* __restrict__ partial, int n,
-                                                       double* __restrict__ out) {
-    __shared__ double red[1024];
+// deterministic final sums of per-block partials: workgroup b adds partial[b n .. b n + n) into out[b], which may lie
+// in pinned host memory (a copy of 8 bytes behind the kernel took longer than the kernel)
+template <int NT>
+__global__ __launch_bounds__(NT) void k_sum_partials(const double* __restrict__ partial, int n,
+                                                     double* __restrict__ out) {
+    __shared__ double red[NT];
+    const double* const p = partial + (size_t)blockIdx.x * n;
     double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += 1024) v += partial[i];
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    for (int i = threadIdx.x; i < n; i += NT) v += p[i];
+    if (NT > 64) {
+        red[threadIdx.x] = v;
         __syncthreads();
+        for (int w = NT / 2; w >= 64; w >>= 1) {
+            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x >= 64) return;
+        v = red[threadIdx.x];
     }
-    if (threadIdx.x == 0) out[0] = red[0];
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+    if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 // K2: dSdU_mu = coeff * Sigma_mu
@@ -469,8 +478,11 @@ hipError_t launch_round_f32(double* U, double* P, int V, bool links, bool projec
     return hipGetLastError();
 }
 
-hipError_t launch_sum_partials(const double* partial, int n, double* out, hipStream_t st) {
-    k_sum_partials<<<1, 1024, 0, st>>>(partial, n, out);
+hipError_t launch_sum_partials(const double* partial, int n, int sums, double* out, hipStream_t st) {
+    if (n <= 64)
+        k_sum_partials<64><<<sums, 64, 0, st>>>(partial, n, out);
+    else
+        k_sum_partials<1024><<<sums, 1024, 0, st>>>(partial, n, out);
     return hipGetLastError();
 }
 
@@ -483,8 +495,7 @@ hipError_t launch_plaquette(const Geo& g, const T* U, double* partial, double* o
         k_plaquette_xrow<T><<<nb, kBlock, 0, st>>>(g, U, partial);
     else
         k_plaquette<T><<<nb, kBlock, 0, st>>>(g, U, partial);
-    k_sum_partials<<<1, 1024, 0, st>>>(partial, nb, out);
-    return hipGetLastError();
+    return out ? launch_sum_partials(partial, nb, 1, out, st) : hipGetLastError();
 }
 template <typename T>
 hipError_t launch_action_untraced(const Geo& g, const T* U, double coeff, double* ref, hipStream_t st) {
@@ -495,8 +506,7 @@ template <typename T>
 hipError_t launch_momenta_dot(const Geo& g, const T* P, double* partial, double* out, hipStream_t st) {
     const int nb = grid_sites_mu(g.V);
     k_momenta_dot<T><<<nb, kBlock, 0, st>>>(g, P, partial);
-    k_sum_partials<<<1, 1024, 0, st>>>(partial, nb, out);
-    return hipGetLastError();
+    return out ? launch_sum_partials(partial, nb, 1, out, st) : hipGetLastError();
 }
 template <typename T>
 hipError_t launch_dsdu(const Geo& g, const T* U, double coeff, T* D, hipStream_t st) {

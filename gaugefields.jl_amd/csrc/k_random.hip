@@ -382,7 +382,7 @@ hipError_t launch_heatbath(const Geo& g, T* U, int mode, double beta, unsigned l
                 k_heatbath<T, 1><<<nb, kBlock, lds, st>>>(g, U, mu, par, beta, seed, sweep, itmax, part);
         }
     hipError_t err = hipGetLastError();
-    if (err == hipSuccess && mode == 0) err = launch_sum_partials(partial, 8 * nb, failures, st);
+    if (err == hipSuccess && mode == 0) err = launch_sum_partials(partial, 8 * nb, 1, failures, st);
     return err;
 }
 

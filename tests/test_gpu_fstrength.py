@@ -164,3 +164,32 @@ def test_api_topological_charge(gf):
     cold = api.gauge_configuration((4, 4, 4, 4), start="cold")
     assert api.topological_charge(cold, method="improved") == 0.0
     assert api.calculate_energy_density(cold) == 0.0
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_rows_beyond_one_wait(Lat, oracle, precision):
+    """More energies, and more rows of observables, than are read with one wait: bit for bit those of single steps
+    (the same kernels on the same links)."""
+    dims = (4, 4, 2, 4)
+    print(f"[fstrength] rows {precision}", flush=True)
+    U = alg_links(oracle, dims, 0.5, 36)
+    L, S = Lat(dims, precision), Lat(dims, precision)
+    L.upload_links(U)
+    S.upload_links(U)
+    n = 515
+    E = L.flow(1e-3, n + 1, 1)
+    one = []
+    for _ in range(n + 1):
+        S.flow(1e-3, 1)
+        one.append(S.energy_density())
+    assert np.array_equal(E, one)
+    assert np.array_equal(L.download_links(), S.download_links())
+    L.upload_links(U)
+    S.upload_links(U)
+    rows = L.flow_measure(2e-3, 2 * 105 + 1, 2)
+    assert rows.shape == (105, 7)
+    for k in range(105):
+        assert rows[k, 0] == 2e-3 * (2 * (k + 1))
+        assert np.array_equal(rows[k, 1:], S.flow_measure(2e-3, 2, 2)[0, 1:])  # one row: one wait
+    S.flow(2e-3, 1)
+    assert np.array_equal(L.download_links(), S.download_links())
