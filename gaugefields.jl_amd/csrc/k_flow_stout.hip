@@ -127,8 +127,10 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
 // pairs of a site share comes from L1) up to one exchange in LDS of the near contributions.  Three waves
 // per SIMD are too few to hide memory behind each other, so a wave asks for a pair's inputs at once: the
 // four links and the site's two Lam into registers, the neighbours' Lam straight into LDS, where the near
-// contributions will go.  ROWS: the far contribution to U_b(z + x) of the pairs (0, b) goes to a site of
-// the workgroup and is added to the near ones there, a quarter of the far fields less.
+// contributions will go.  The far contribution to U_b(z + x) of the pairs (0, b) mostly goes to a site of the
+// workgroup and is added to the near ones there: up to a quarter of the far fields less, also where the groups
+// cut the rows (force with three levels, FP64 24^4 1.40 -> 1.36 ms, 24x24x16x12 475 -> 459 us; FP32 24^4 774 -> 760).
+__device__ __forceinline__ bool same_group(int s, int r) { return (s >> 6) == (r >> 6); }
 template <typename T, bool ROWS, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_pair(
     Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Fl, T* __restrict__ far, double rho) {
@@ -193,17 +195,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
         const R6<T> ra = ldr(U, V, a, (unsigned)s1), rb = ldr(U, V, b, (unsigned)s1);
         T t[8];
         coeffs_of_herm(herm_conj_dag(full_of(ra), herm_of_coeffs(fb)), t);
-        if (ROWS && a == 0) {
-            // the contribution to lane x + 1, through this wave's place in LDS (its lanes in step)
+        bool store = in_lattice<ROWS>(g, sm);
+        if (a == 0) {
+            // the contribution to the lane of x + 1, through this wave's place in LDS (its lanes in step)
+            const int from = s + dlt(g, x, 0, -1);
             put_c8(&near_[2 * p + 1], lane, t);
             __builtin_amdgcn_wave_barrier();
-            get_c8(&near_[2 * p + 1], xrow_of<true>(g, s, x[0], lane).m, t);
-            __builtin_amdgcn_wave_barrier();
+            if (ROWS || same_group(from, s)) {
+                T n[8];
+                get_c8(&near_[2 * p + 1], from & 63, n);
 #pragma unroll
-            for (int k = 0; k < 8; k++) c[k] += t[k];
-        } else if (in_lattice<ROWS>(g, sm)) {
-            stp<T, GF_ST_NT>(far + (size_t)a * 32 * V, V, b, (unsigned)s, t);
+                for (int k = 0; k < 8; k++) c[k] += n[k];
+            }
+            __builtin_amdgcn_wave_barrier();
+            store = !ROWS && store && !same_group(fw[0], s);
         }
+        if (store) stp<T, GF_ST_NT>(far + (size_t)a * 32 * V, V, b, (unsigned)s, t);
         put_c8(&near_[2 * p + 1], lane, c);
 #pragma unroll
         for (int k = 0; k < 8; k++) fa[k] = -fa[k];
@@ -259,9 +266,13 @@ __global__ __launch_bounds__(kBlock) void k_stout_gather(Geo g, const T* __restr
     ldp<T, GF_LD_NT>(Fl, V, mu, (unsigned)s, f);
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        if (ROWS && j == 0 && mu > 0) continue;  // the x-neighbour's is in Fl
-        const int nu = j + (j >= mu ? 1 : 0);
-        ldp(far + (size_t)j * 32 * V, V, mu, (unsigned)(s + dlt(g, x, nu, -1)), t[j]);
+        const int nu = j + (j >= mu ? 1 : 0), from = s + dlt(g, x, nu, -1);
+        if (j == 0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) t[0][k] = T(0);
+            if (mu > 0 && (ROWS || same_group(from, s))) continue;  // in Fl
+        }
+        ldp(far + (size_t)j * 32 * V, V, mu, (unsigned)from, t[j]);
     }
 #pragma unroll
     for (int k = 0; k < 8; k++) {
