@@ -266,6 +266,19 @@ __device__ __forceinline__ void or_subgroup(M3<double>& u, const M3<double>& V, 
     }
 }
 
+// the three steps of a link
+__device__ __forceinline__ void or_steps(M3<double>& u, const M3<double>& St, unsigned long long seed,
+                                         unsigned long long sweep, unsigned s, int mu) {
+#pragma unroll 1
+    for (int i = 0; i < 3; i++) {
+        unsigned w[4];
+        link_block(seed, sweep, s, mu, 6, i, w);
+        const int n = (int)(((unsigned long long)w[0] * 2ull) >> 32);
+        const int k = n + 1 + (int)(((unsigned long long)w[1] * (unsigned long long)(2 - n)) >> 32);
+        or_subgroup(u, St, n, k);
+    }
+}
+
 // one heatbath subgroup step; false (u unchanged) if no proposal was accepted
 template <int n, int k>
 __device__ __forceinline__ bool hb_subgroup(M3<double>& u, const M3<double>& St, unsigned long long seed,
@@ -334,14 +347,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
                  hb_subgroup<1, 2>(u, St, seed, sweep, (unsigned)s, mu, 4, beta, itmax) &&
                  hb_subgroup<0, 2>(u, St, seed, sweep, (unsigned)s, mu, 5, beta, itmax);
         } else {
-#pragma unroll 1
-            for (int i = 0; i < 3; i++) {
-                unsigned w[4];
-                link_block(seed, sweep, (unsigned)s, mu, 6, i, w);
-                const int n = (int)(((unsigned long long)w[0] * 2ull) >> 32);
-                const int k = n + 1 + (int)(((unsigned long long)w[1] * (unsigned long long)(2 - n)) >> 32);
-                or_subgroup(u, St, n, k);
-            }
+            or_steps(u, St, seed, sweep, (unsigned)s, mu);
         }
         if (ok) {
             reunitarize_f64<MODE == 1>(u);
@@ -359,6 +365,79 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
     if (MODE == 0) block_sum_store<kBlock>(fail, partial);  // an overrelaxation always succeeds
 }
 
+// what is pinned is formed before anything behind it: not sunk past a branch, nor loads hoisted before it
+template <typename M>
+__device__ __forceinline__ void pin_rows(M& m) {
+#pragma unroll
+    for (int e = 0; e < 6; e++) asm volatile("" : "+v"(m.v[e].x), "+v"(m.v[e].y));
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void pin(M3<double>& m) {
+#pragma unroll
+    for (int e = 0; e < 9; e++) asm volatile("" : "+v"(m.m[e].r), "+v"(m.m[e].i));
+    __builtin_amdgcn_sched_barrier(0);
+}
+// Overrelaxation of FP64 links on large tiled lattices (split_overrelax), the same sums in the same order: a
+// workgroup of three waves per 64 sites of the colour.  Wave j forms the two products of the j-th plane of mu, all
+// waves at the same time, and adds its staples to the sum that the wave before it has left in LDS; the last one
+// updates the links.  A third as many sites are in flight, whose links then meet in L2, at the price of a longer
+// chain.  Sites in the order of heatbath_half_site.
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_overrelax_split(
+    Geo g, double* __restrict__ U, int mu, int par, unsigned long long seed, unsigned long long sweep) {
+    __shared__ double2 sum[9][64];
+    const int j = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
+    const int grp = tsweep_group(g, 2u * xcd_block() + (unsigned)(lane >> 5), 2u * gridDim.x);
+    const unsigned V = g.V;
+    int x[4];
+    const int s = colour_site(g, grp * 32 + (lane & 31), par, x);
+    const int nu = j + (j >= mu ? 1 : 0);
+    const int fmu = sel4(mu, dlt(g, x, 0, 1), dlt(g, x, 1, 1), dlt(g, x, 2, 1), dlt(g, x, 3, 1));
+    const int fnu = sel4(nu, dlt(g, x, 0, 1), dlt(g, x, 1, 1), dlt(g, x, 2, 1), dlt(g, x, 3, 1));
+    const int bnu = sel4(nu, dlt(g, x, 0, -1), dlt(g, x, 1, -1), dlt(g, x, 2, -1), dlt(g, x, 3, -1));
+    const double* const Uc = U;
+    const R6<double> a = ldr(Uc, V, nu, (unsigned)(s + fmu)), b = ldr(Uc, V, mu, (unsigned)(s + fnu)),
+                     e = ldr(Uc, V, mu, (unsigned)(s + bnu));
+    __builtin_amdgcn_sched_barrier(0);
+    const R6<double> f = ldr(Uc, V, nu, (unsigned)(s + fmu + bnu));
+    R6<double> X = rows_of(su3_mul_nd(a, full_of(b)));  // U_nu(x+mu) U_mu(x+nu)^dag
+    __builtin_amdgcn_sched_barrier(0);
+    const R6<double> d = ldr(Uc, V, nu, (unsigned)s), c = ldr(Uc, V, nu, (unsigned)(s + bnu));
+    R6<double> Y = rows_of(su3_mul(e, full_of(f)));  // U_mu(x-nu) U_nu(x+mu-nu)
+    pin_rows(X);
+    pin_rows(Y);
+    M3<double> sig = zero3<double>();
+    if (j > 0) __syncthreads();
+    if (j > 1) __syncthreads();
+    if (j > 0) {
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            sig.m[k].r = sum[k][lane].x;
+            sig.m[k].i = sum[k][lane].y;
+        }
+    }
+    acc_mul_nd(sig, full_of(X), full_of(d));
+    pin(sig);
+    R6<double> own;
+    if (j == 2) own = ldr(Uc, V, mu, (unsigned)s);
+    acc_mul_dn(sig, full_of(Y), full_of(c));
+    pin(sig);
+    if (j < 2) {  // two barriers for every wave
+#pragma unroll
+        for (int k = 0; k < 9; k++) sum[k][lane] = t2_of(sig.m[k]);
+        __syncthreads();
+        if (j == 0) __syncthreads();
+        return;
+    }
+    M3<double> u = full_of(own);
+    or_steps(u, sig, seed, sweep, (unsigned)s, mu);
+    reunitarize_f64<true>(u);
+    stu<double>(U, V, mu, (unsigned)s, u);
+}
+// Thread per site / split, sweep in us: 16^4 103 / 117, 24^4 390 / 398, 24^3x32 515 / 507, 32^3x16 622 / 591, 24^3x48
+// 776 / 714, 32^4 1265 / 1218, 32^3x48 1806 / 1670; in linear order, where neighbours do not meet, 28^4 796 / 815.
+// Pieces of 64 pairs have to fill the lattice and its eight parts.
+static bool split_overrelax(const Geo& g) { return g.tile[0] > 0 && g.V >= 400000 && g.V % 1024 == 0; }
+
 // Dynamic LDS (unused) of an FP64 heatbath launch: 56 KB per workgroup leaves room for two
 // workgroups per CU instead of three.  A heatbath thread owns one site of one colour, so the sites
 // in flight per XCD are eight times the stencil kernels'; with a third fewer of them the links their
@@ -373,6 +452,14 @@ hipError_t launch_heatbath(const Geo& g, T* U, int mode, double beta, unsigned l
                            unsigned long long sweep, int itmax, double* partial, double* failures, hipStream_t st) {
     const int nb = grid_for(g.V / 2);
     const size_t lds = sizeof(T) == 8 ? kHeatbathOccLds : 0;
+    if constexpr (sizeof(T) == 8) {
+        if (mode != 0 && split_overrelax(g)) {
+            for (int mu = 0; mu < 4; mu++)
+                for (int par = 0; par < 2; par++)
+                    k_overrelax_split<<<g.V / 128, 192, 0, st>>>(g, U, mu, par, seed, sweep);
+            return hipGetLastError();
+        }
+    }
     for (int mu = 0; mu < 4; mu++)
         for (int par = 0; par < 2; par++) {
             double* part = partial + (size_t)(2 * mu + par) * nb;

@@ -81,6 +81,22 @@ def test_sweep_edges(Lat, oracle, dims):
         assert np.abs(L.download_links() - W).max() < 1e-9
 
 
+def test_overrelaxation_split_over_waves(Lat, oracle):
+    """The smallest kind of lattice whose sweeps are split: bounds of test_overrelaxation_matches_oracle..."""
+    dims = (32, 32, 16, 32)
+    print(f"[overrelaxation] split {dims}", flush=True)
+    L = Lat(dims)
+    L.set_cold()
+    L.gaussian_momenta(23, sigma=0.3)
+    L.exp_update(1.0)
+    W = L.download_links()
+    p0 = L.plaquette_sum()
+    L.overrelaxation(5, 0)
+    oracle.heatbath_sweep(dims, W, 6.0, 5, 0, overrelax=True)
+    assert np.abs(L.download_links() - W).max() < 1e-12
+    assert L.plaquette_sum() == pytest.approx(p0, rel=1e-13)
+
+
 def test_heatbath_strong_coupling_and_fp32(Lat):
     dims = (8, 8, 8, 8)
     for prec in ("f64", "f32"):
