@@ -102,8 +102,9 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
 // (Replaces a gather that evaluated every plaquette once per link, 3258 instead of 1390 x 6/4 FMAs per
 // link and four times the loads, and carried dS/dU and C.)
 // ---------------------------------------------------------------------------
+// FP32: four waves per SIMD at the price of two spilled registers (force with three levels 32^4 2.34 -> 2.32 ms).
 template <typename T, int ST>
-__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_top(
+__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4))) void k_stout_top(
     Geo g, const T* __restrict__ Utop, double coeff, const T* __restrict__ Qst, T* __restrict__ Lc,
     T* __restrict__ Fl) {
     int s, mu;

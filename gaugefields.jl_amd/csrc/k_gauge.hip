@@ -278,8 +278,9 @@ hipError_t launch_state64_step(int mode, const Geo& g, const double* P64, double
 // ---------------------------------------------------------------------------
 // A wave moves the 64-site group q of the direction-major order (group q % G of direction q / G, G = ceil(V / 64)):
 // its links are one piece of the host array, which lies in pinned host memory as often as on the device, so the
-// wave reads or writes that piece in whole lines, 16 B per lane, and turns it in LDS.  A thread per link, as these
-// were, touches a line in each of 64 places per instruction (12^4 links: 14 -> 5 us on the device).
+// wave reads or writes that piece in whole lines, 16 B per lane, and turns it in LDS.  (A thread per link, as these
+// were, touches a line in each of 64 places per instruction: 290 us for 32^4 links to device memory, and a copy
+// behind it.)  Bound by the link: 2 MB in 39 us, 54 GB/s.
 __device__ __forceinline__ bool group_at(int V, int q0, int nq, int& mu, int& s0, int& m) {
     const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
     const int G = (V + 63) / 64;
