@@ -60,7 +60,7 @@ struct gf_ctx {
     void* loops = nullptr;  // loop coefficients of the field strengths, a block of t-slices
     size_t loops_bytes = 0;
     // scratch for per-site outputs and reductions
-    double* staging = nullptr;  // 18 V doubles
+    double* staging = nullptr;  // per-site outputs (18 V doubles) and arrays that go up in one copy
     HostRing ring;              // host arrays in and out
     double* partial = nullptr;
     double* hres = nullptr;   // kRes pinned scalars, which the kernels write

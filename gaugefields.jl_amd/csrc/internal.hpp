@@ -11,10 +11,6 @@ namespace gf {
 
 constexpr int kBlock = 256;
 
-// FP32-bulk kernels re-project every link they update onto SU(3)
-template <typename T>
-inline constexpr bool kFloatBulk = std::is_same<T, float>::value;
-
 inline int grid_for(int V, int block = kBlock) { return (V + block - 1) / block; }
 // gridDim.y of the streaming link kernels: threads per site (4: one per link) on lattices of so few
 // workgroups of sites that CUs stay empty (4^4: 5.2 -> 3.5 us, 12^3x8: 7.6 -> 3.7; 16^4: 12.4 -> 12.9, hence

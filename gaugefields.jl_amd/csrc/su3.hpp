@@ -278,17 +278,6 @@ __device__ __forceinline__ void reunitarize_f64(M3<double>& u) {
     }
 }
 
-template <typename T>
-__device__ __forceinline__ void reunitarize(M3<T>& u) {
-    M3<double> d = to_f64(u);
-    reunitarize_f64(d);
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        u.m[k].r = (T)d.m[k].r;
-        u.m[k].i = (T)d.m[k].i;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // su(3) projections (basis i lambda_a / 2, order of TA_gaugefields_4D_serial.jl:243-260)
 // ---------------------------------------------------------------------------
@@ -843,18 +832,6 @@ __device__ __forceinline__ M3<T> expi_herm(const M3<T>& H) {
     return E;
 }
 
-// exp(Q) for anti-Hermitian traceless Q  (H = -iQ)
-template <typename T>
-__device__ __forceinline__ M3<T> exp_antiherm(const M3<T>& Q) {
-    M3<T> H;
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        H.m[k].r = Q.m[k].i;
-        H.m[k].i = -Q.m[k].r;
-    }
-    return expi_herm(H);
-}
-
 // exp(Q) and L = X star d exp(Q)/dQ (d tr(X e^Q) = tr(L dQ) for anti-Hermitian traceless Q; CdexpQdQ!,
 // stout_fast.jl:888-946, 1031-1081) together, sharing one evaluation of the invariants and
 // Cayley-Hamilton coefficients (stout backward: E = e^{Q_mu}, L = CdexpQdQ(U_mu Dout_mu, Q_mu))
@@ -1045,24 +1022,6 @@ __device__ __forceinline__ M3<T> exp_coeffs_times(const T c[8], double t, const 
         return round_link<T>(r);
     } else {
         return mul(expi_herm(herm_from_coeffs(c, t)), u);
-    }
-}
-
-// exp(Q) U for a traceless anti-Hermitian Q given in double (FP32 links: rounded once)
-__device__ __forceinline__ M3<float> exp_antiherm_times(const M3<double>& Q, const M3<float>& u) {
-    M3<double> r = mul(exp_antiherm(Q), to_f64(u));
-    reunitarize_f64(r);
-    return round_link<float>(r);
-}
-// exp(Q) U for a traceless anti-Hermitian Q
-template <typename T>
-__device__ __forceinline__ M3<T> exp_antiherm_times(const M3<T>& Q, const M3<T>& u) {
-    if constexpr (std::is_same<T, float>::value) {
-        M3<double> r = mul(exp_antiherm(to_f64(Q)), to_f64(u));
-        reunitarize_f64(r);
-        return round_link<T>(r);
-    } else {
-        return mul(exp_antiherm(Q), u);
     }
 }
 
