@@ -509,7 +509,7 @@ OmelyanPQP() = OmelyanPQP(OMELYAN_LAMBDA)
 
 """MD action provider: `action` on `nn`'s stout-smeared links (test/HMCstout_test_nowing.jl:36-118),
 with the smearing forward/backward and the force on the device.  mode: :store, :recompute or
-:auto (store each level's C when the device has room)."""
+:auto (store each level's Q when the device has room)."""
 struct StoutGaugeAction
     action::GaugeAction
     levels::Int
