@@ -1,6 +1,7 @@
 // capi.hip -- the C ABI of libgfhip.so: context, device buffers, host-side MD/flow/stout drivers.
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -59,6 +60,7 @@ struct gf_ctx {
     void* U64bak = nullptr;
     void* loops = nullptr;  // loop coefficients of the field strengths, a block of t-slices
     size_t loops_bytes = 0;
+    bool loops_short = false;  // less than asked for
     // scratch for per-site outputs and reductions
     double* staging = nullptr;  // per-site outputs (18 V doubles) and arrays that go up in one copy
     HostRing ring;              // host arrays in and out
@@ -104,6 +106,7 @@ int alloc(gf_ctx* c, void** p, size_t n) {
     hipError_t e = hipMalloc(p, n);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // reported here; not to be found by the next launch's check
         return fail(c, GF_ENOMEM, "hipMalloc(%zu bytes): %s", n, hipGetErrorString(e));
     }
     c->bytes += n;
@@ -319,18 +322,25 @@ int fstrength_queue(gf_ctx* c, int sets, double* at, double* dens, int dens_meth
         return fail(c, GF_ESTATE,
                     "field-strength measurements are not available in the FP32-force form (FP64 links and momenta, "
                     "forces in FP32); use a GF_F64 or GF_F32 context");
-    const size_t need = field_strength_bytes(c->geo, sets);
-    if (need > c->loops_bytes) {
+    // smaller blocks of t-slices where the device has no room for the usual ones
+    size_t need = field_strength_bytes(c->geo, sets, SIZE_MAX);
+    const size_t least = field_strength_bytes(c->geo, sets, 1);
+    if (need > c->loops_bytes && !(c->loops_short && c->loops_bytes >= least)) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
         release(c, &c->loops, c->loops_bytes);
         c->loops_bytes = 0;
-        TRY(alloc(c, &c->loops, need));
+        int r;
+        while ((r = alloc(c, &c->loops, need)) != GF_OK && need > least) {
+            need = field_strength_bytes(c->geo, sets, need / 2);
+            c->loops_short = true;
+        }
+        TRY(r);
         c->loops_bytes = need;
     }
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->loops, c->partial, at, dens, dens_method,
-                                           c->stream));
+        HIPCHK(c, launch_field_strength<T>(c->geo, (const T*)c->U, sets, c->loops, c->loops_bytes, c->partial, at,
+                                           dens, dens_method, c->stream));
         return GF_OK;
     });
 }

@@ -127,13 +127,14 @@ hipError_t launch_axpby(T* y, const T* x, double a, double b, size_t n, hipStrea
 
 // ---- k_fstrength.hip ----
 // Field strengths of the loop sets in `sets` (bit 0 plaquette, 1 clover, 2 rectangle); out4 =
-// {clover energy sum, plaquette Q, clover Q, rectangle Q} (device doubles); dens (device, V) if
+// {clover energy sum, plaquette Q, clover Q, rectangle Q}; dens (device, V) if
 // non-null receives the density of dens_method (0 plaquette, 1 clover, 2 improved, 3 rectangle).
-// fields: scratch of field_strength_bytes; partial: 4 (V / 64 + NT + 1) doubles
-size_t field_strength_bytes(const Geo& g, int sets);
+// fields: scratch of `bytes`, field_strength_bytes for the speed it is meant to have and at least that for
+// most = 1 (one t-slice); partial: 4 (V / 64 + NT + 1) doubles
+size_t field_strength_bytes(const Geo& g, int sets, size_t most);
 template <typename T>
-hipError_t launch_field_strength(const Geo& g, const T* U, int sets, void* fields, double* partial, double* out4,
-                                 double* dens, int dens_method, hipStream_t st);
+hipError_t launch_field_strength(const Geo& g, const T* U, int sets, void* fields, size_t bytes, double* partial,
+                                 double* out4, double* dens, int dens_method, hipStream_t st);
 
 // ---- k_random.hip ----
 template <typename T>

@@ -352,22 +352,23 @@ static int fields_of(int sets) { return (sets & 1) + 2 * ((sets >> 1) & 1) + 3 *
 // of them where there are no fields (the plaquette set alone, whose sites are then visited as the stencil
 // kernels visit theirs)
 constexpr double kFieldBytes = 256e6;
-static int slices_per_block(const Geo& g, int sets) {
+static size_t slice_bytes(const Geo& g, int sets) { return (size_t)(g.V / g.n[3]) * 6 * 64 * fields_of(sets); }
+static int slices_per_block(const Geo& g, int sets, size_t bytes) {
     if (sets == 1) return g.n[3];
-    const double slice = (double)(g.V / g.n[3]) * 6 * 64 * fields_of(sets);
-    const int most = std::max(1, (int)(kFieldBytes / slice)), blocks = (g.n[3] + most - 1) / most;
+    const int most = std::max(1, (int)((double)bytes / (double)slice_bytes(g, sets)));
+    const int blocks = (g.n[3] + most - 1) / most;
     return (g.n[3] + blocks - 1) / blocks;
 }
-size_t field_strength_bytes(const Geo& g, int sets) {
+size_t field_strength_bytes(const Geo& g, int sets, size_t most) {
     if (sets == 1) return 0;
-    return (size_t)slices_per_block(g, sets) * (size_t)(g.V / g.n[3]) * 6 * 64 * fields_of(sets);
+    return slices_per_block(g, sets, std::min(most, (size_t)kFieldBytes)) * slice_bytes(g, sets);
 }
 
 template <typename T, int SETS>
-void launch_sets(const Geo& g, const T* U, double2* fields, double* partial, int stride, double* dens, int dens_method,
+void launch_sets(const Geo& g, const T* U, double2* fields, int per, double* partial, int stride, double* dens, int dens_method,
                  hipStream_t st) {
     constexpr int NT = ((SETS & 3) ? 1 : 0) + ((SETS & 4) ? 1 : 0);
-    const int slice = g.V / g.n[3], per = slices_per_block(g, SETS);
+    const int slice = g.V / g.n[3];
     int base = 0;
     for (int t = 0; t < g.n[3]; t += per) {
         const int n = slice * std::min(per, g.n[3] - t), groups = (n + 63) / 64;
@@ -381,26 +382,26 @@ void launch_sets(const Geo& g, const T* U, double2* fields, double* partial, int
 
 // partial: 4 (V / 64 + NT + 1) doubles
 template <typename T>
-hipError_t launch_field_strength(const Geo& g, const T* U, int sets, void* fields, double* partial, double* out4,
-                                 double* dens, int dens_method, hipStream_t st) {
-    const int slice = g.V / g.n[3], per = slices_per_block(g, sets);
+hipError_t launch_field_strength(const Geo& g, const T* U, int sets, void* fields, size_t bytes, double* partial,
+                                 double* out4, double* dens, int dens_method, hipStream_t st) {
+    const int slice = g.V / g.n[3], per = slices_per_block(g, sets, std::min(bytes, (size_t)kFieldBytes));
     int stride = 0;
     for (int t = 0; t < g.n[3]; t += per) stride += (slice * std::min(per, g.n[3] - t) + 63) / 64;
     double2* const f = (double2*)fields;
     switch (sets) {
-        case 1: launch_sets<T, 1>(g, U, f, partial, stride, dens, dens_method, st); break;
-        case 2: launch_sets<T, 2>(g, U, f, partial, stride, dens, dens_method, st); break;
-        case 4: launch_sets<T, 4>(g, U, f, partial, stride, dens, dens_method, st); break;
-        case 6: launch_sets<T, 6>(g, U, f, partial, stride, dens, dens_method, st); break;
-        case 7: launch_sets<T, 7>(g, U, f, partial, stride, dens, dens_method, st); break;
+        case 1: launch_sets<T, 1>(g, U, f, per, partial, stride, dens, dens_method, st); break;
+        case 2: launch_sets<T, 2>(g, U, f, per, partial, stride, dens, dens_method, st); break;
+        case 4: launch_sets<T, 4>(g, U, f, per, partial, stride, dens, dens_method, st); break;
+        case 6: launch_sets<T, 6>(g, U, f, per, partial, stride, dens, dens_method, st); break;
+        case 7: launch_sets<T, 7>(g, U, f, per, partial, stride, dens, dens_method, st); break;
         default: return hipErrorInvalidValue;
     }
     return launch_sum_partials(partial, stride, 4, out4, st);
 }
 
 #define GF_INST_FS(T)                                                                                            \
-    template hipError_t launch_field_strength<T>(const Geo&, const T*, int, void*, double*, double*, double*, int, \
-                                                 hipStream_t);
+    template hipError_t launch_field_strength<T>(const Geo&, const T*, int, void*, size_t, double*, double*, double*,  \
+                                                 int, hipStream_t);
 GF_INST_FS(double)
 GF_INST_FS(float)
 #undef GF_INST_FS
