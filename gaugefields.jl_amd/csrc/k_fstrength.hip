@@ -359,9 +359,13 @@ static int slices_per_block(const Geo& g, int sets, size_t bytes) {
     const int blocks = (g.n[3] + most - 1) / most;
     return (g.n[3] + blocks - 1) / blocks;
 }
+// the block of these sets, and no less than the blocks of the other sets take where a t-slice of theirs fits into
+// kFieldBytes: a density and then an energy of one context grow the buffer once
 size_t field_strength_bytes(const Geo& g, int sets, size_t most) {
     if (sets == 1) return 0;
-    return slices_per_block(g, sets, std::min(most, (size_t)kFieldBytes)) * slice_bytes(g, sets);
+    most = std::min(most, (size_t)kFieldBytes);
+    return std::max(slices_per_block(g, sets, most) * slice_bytes(g, sets),
+                    std::min(most, g.n[3] * slice_bytes(g, 7)));
 }
 
 template <typename T, int SETS>

@@ -80,6 +80,22 @@ def test_loops_by_blocks(Lat, oracle, dims, precision):
     assert L.energy_density_clover() == pytest.approx(oracle.energy_density_clover(dims, W), rel=rel)
 
 
+def test_loops_in_the_links_partner(Lat, oracle):
+    """A lattice whose blocks lie in the links' ping-pong partner, after a flow step that has used it."""
+    dims = (30, 26, 25, 27)
+    print(f"[fstrength] partner {dims}", flush=True)
+    L = Lat(dims)
+    L.upload_links(alg_links(oracle, dims, 0.6, 43))
+    L.flow(0.01, 1)
+    U = L.download_links()
+    Qref, qref = oracle.topological_charge_density(dims, U, "improved")
+    for _ in range(2):
+        assert np.abs(L.topological_charge_density("improved") - qref).max() < 1e-13
+        assert abs(L.topological_charge("improved") - Qref) <= max(1e-12 * abs(Qref), np.sqrt(qref.size) * 1e-13)
+        assert L.energy_density_clover() == pytest.approx(oracle.energy_density_clover(dims, U), rel=1e-12)
+        assert np.array_equal(L.download_links(), U)
+
+
 def test_constant_abelian_field_closed_form(Lat):
     dims = (4, 6, 6, 4)
     U, t, tp = lt.abelian_flux_links(dims, 2, -1)
