@@ -286,7 +286,12 @@ struct HostRing {
             if (issued == t.total) break;
             h.wait([&] { return t.err != hipSuccess || t.copied(issued - slots); });
         }
-        h.allow(t, e == hipSuccess ? t.total : 0);
+        // after an error no chunk is claimed any more: what the slots hold is not its own
+        h.check([&] {
+            if (e == hipSuccess) e = t.err;
+            if (e != hipSuccess) t.limit = 0;
+            return true;
+        });
         h.close(t);
         if (e == hipSuccess) e = t.err;
         if (e != hipSuccess) (void)hipStreamSynchronize(st);  // nothing writes to the slots any more

@@ -1,0 +1,52 @@
+// Scenarios of transfer.hpp on the CPU; argv[1] names one.  Exit status 0: as it should be.
+#include <cstdio>
+#include <string>
+#include <vector>
+
+#include "transfer.hpp"
+
+using gf::HostRing;
+
+namespace {
+constexpr size_t kUnit = 64 * 144;  // bytes of a unit, a group's links
+
+// one download of `chunks` slots, chunk k filled with the byte 1 + k % 200; bytes of dst that hold neither that nor
+// what was there before
+long wrong_bytes(HostRing& r, long chunks, hipError_t& e) {
+    const long per = (long)(r.slot / kUnit), units = chunks * per;
+    std::vector<char> dst(units * kUnit, 0);
+    e = r.pull(
+        dst.data(), units, kUnit, [](long q) { return (size_t)q * kUnit; },
+        [&](long q, long n, char* p) { return memset(p, (int)(1 + q / per % 200), n * kUnit), hipSuccess; }, nullptr);
+    long wrong = 0;
+    for (long k = 0; k < chunks; k++)
+        for (size_t b = 0; b < per * kUnit; b++) {
+            const int v = (unsigned char)dst[k * per * kUnit + b];
+            wrong += v != (int)(1 + k % 200) && (v != 0 || e == hipSuccess);
+        }
+    return wrong;
+}
+
+// a whole transfer, and one whose wait for a chunk fails: an error, and nothing in the array that is not its own
+int failed_wait() {
+    HostRing r;
+    r.shape(96 * kUnit, 0);  // several units a slot
+    hipError_t e;
+    if (wrong_bytes(r, 64, e) || e != hipSuccess) return printf("whole transfer: error %d\n", e), 1;
+    long wrong = 0;
+    for (int rep = 0; rep < 400; rep++) {
+        fake.records = 0;
+        fake.fail_wait_of = 16 + rep % 24;
+        wrong += wrong_bytes(r, 64, e);
+        if (e != hipErrorUnknown) return printf("the failed wait was not reported: %d\n", e), 1;
+    }
+    r.free();
+    return wrong ? printf("%ld bytes of slots that were never filled\n", wrong), 1 : 0;
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "failed_wait") return failed_wait();
+    return printf("no scenario %s\n", what.c_str()), 2;
+}
