@@ -683,8 +683,7 @@ int gf_create(const int* dims, int precision, int device, gf_ctx** out) {
     const size_t largest = (size_t)72 * c->V * sizeof(double), page = kRes * sizeof(double);
     c->ring.shape(largest, c->device);
     const int n_slots = c->ring.slots_at_hand(largest);
-    if (hipHostMalloc((void**)&c->hres, page + c->ring.slot * n_slots, hipHostMallocDefault) != hipSuccess)
-        return bail(GF_ENOMEM);
+    if (pin_alloc((void**)&c->hres, page + c->ring.slot * n_slots) != hipSuccess) return bail(GF_ENOMEM);
     c->ring.adopt((char*)c->hres + page, n_slots);
     if (c->s64 && (alloc(c, &c->U64, link64_bytes(c)) || alloc(c, &c->P64, (size_t)32 * c->V * sizeof(double))))
         return bail(GF_ENOMEM);

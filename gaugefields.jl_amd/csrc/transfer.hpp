@@ -146,6 +146,10 @@ class Helpers {
     bool stop_ = false;
 };
 
+// Host memory that kernels write and the host reads behind an event or a wait: coherent by name, as the default for
+// it is the environment's (HIP_HOST_COHERENT).
+inline hipError_t pin_alloc(void** p, size_t bytes) { return hipHostMalloc(p, bytes, hipHostMallocCoherent); }
+
 constexpr int kSlots = 16;
 constexpr size_t kSlotMin = 256 << 10, kSlotMax = 2 << 20, kUnitMax = 64 * 144;  // a group's links
 
@@ -178,7 +182,7 @@ struct HostRing {
         while (have < kSlots && slot_at[have]) have++;
         for (int more = n - have; more > 0 && have < n; more = std::min(more / 2, n - have)) {
             char* p = nullptr;
-            err = hipHostMalloc((void**)&p, slot * more, hipHostMallocDefault);
+            err = pin_alloc((void**)&p, slot * more);
             if (err != hipSuccess) {
                 (void)hipGetLastError();
                 continue;

@@ -43,10 +43,22 @@ int failed_wait() {
     r.free();
     return wrong ? printf("%ld bytes of slots that were never filled\n", wrong), 1 : 0;
 }
+
+// every allocation that the device writes and the host reads is coherent whatever the environment's default
+int coherent() {
+    HostRing r;
+    r.shape(96 * kUnit, 0);
+    hipError_t e;
+    if (wrong_bytes(r, 64, e) || e != hipSuccess) return 1;
+    r.free();
+    if (fake.host_allocs > 0 && (fake.host_flags & hipHostMallocCoherent)) return 0;
+    return printf("flags %#x\n", fake.host_flags), 1;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "failed_wait") return failed_wait();
+    if (what == "coherent") return coherent();
     return printf("no scenario %s\n", what.c_str()), 2;
 }
