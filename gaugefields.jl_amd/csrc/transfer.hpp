@@ -8,10 +8,10 @@
 #pragma once
 #include <pthread.h>
 #include <sched.h>
+#include <time.h>
 #include <unistd.h>
 
 #include <algorithm>
-#include <atomic>
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
@@ -28,14 +28,25 @@ struct Job {
     virtual ~Job() = default;
 };
 
-// Helper threads of the process, for the copies and checks of all contexts.  A call never waits for a helper to be
-// scheduled: its own thread takes pieces like any other, and a helper that comes too late finds nothing to claim.
-// (Threads started and joined by each call did wait for the processors: 3 ms behind the spinning threads of an
-// OpenMP loop that had just ended.)  Started when the first large array comes, ended when the last context that
-// has used them is destroyed; none in a forked child, which has only the thread that forked.
+// Helper threads of the process, for the copies and checks of all contexts.  A call never waits for a helper to start:
+// its own thread takes pieces like any other, and a helper that comes too late finds nothing to claim.  It does wait for
+// a piece that a helper has claimed, and where the processors are taken (behind an OpenMP loop its threads go on
+// spinning) the scheduler may take a helper off in the middle of one, or the caller off for a helper, for 3 ms.  So
+// helpers are called one at a time, each by the one before it, and one that the scheduler brought late (kLate) takes
+// nothing: where the processors are taken the call is mostly its own thread's.
+// Links down behind an OpenMP loop of 16 threads on 16 processors, mean and 99th percentile in us, all seven called at
+// once / one by one: 8^4 211-256, 2725-4028 / 132-151, 306-377 (without helpers, by the runtime's copy, 190, 697); 12^4
+// 665-697, 4288-4419 / 569-663, 1261-1634 (725, 1349); 16^4 and larger means within 6 %.  What is computed and not only
+// copied (the SU(3) check) gets less help there: links up 24^4 8.5 / 10.3 ms (19.8).  With the processors free the same:
+// down 8^4 177 / 142 us, 12^4 423 / 430, 16^4 908 / 923, 24^4 4453 / 4368, 32^4 13.4 / 13.3 ms.  As SCHED_BATCH, which never
+// takes the caller off for a helper: means 10-20 % longer from 16^4 on.
+// (Threads started and joined by each call waited for the processors as well.)  Started when the first large array
+// comes, ended when the last context that has used them is destroyed; none in a forked child, which has only the
+// thread that forked.
 class Helpers {
   public:
     static constexpr int kMax = 7;  // and the caller: 32^4 links with 8 threads 15.0 ms, four 15.4, two 25
+    static constexpr long long kLate = 200 * 1000;  // ns from the call
     static Helpers& get() {
         static Helpers* const h = new Helpers;  // outlives every static destructor
         return *h;
@@ -49,7 +60,7 @@ class Helpers {
         pthread_attr_t at;
         if (pthread_attr_init(&at) != 0) return;
         (void)pthread_attr_setstacksize(&at, 2 << 20);
-        while (n_ < std::min(kMax, cpus - 1) && pthread_create(&th_[n_], &at, loop, this) == 0) n_++;
+        while (n_ < std::min(kMax, cpus - 1) && pthread_create(&one_[n_].thread, &at, loop, &one_[n_]) == 0) n_++;
         pthread_attr_destroy(&at);
     }
     void release() {
@@ -59,10 +70,12 @@ class Helpers {
         {
             std::lock_guard<std::mutex> lk(m_);
             stop_ = true;
-            work_.notify_all();
+            for (One& o : one_) o.work.notify_one();
         }
-        for (; n_ > 0; n_--) pthread_join(th_[n_ - 1], nullptr);
-        stop_ = false;
+        for (; n_ > 0; n_--) pthread_join(one_[n_ - 1].thread, nullptr);
+        for (One& o : one_) o.called = 0;
+        idle_ = 0;
+        calling_ = stop_ = false;
     }
 
     // offers the job to the helpers (if there is room: a job that is not offered is its caller's alone)
@@ -73,13 +86,12 @@ class Helpers {
                 p = &j;
                 break;
             }
-        wake(j.limit - j.next);
+        call(j);
     }
     void allow(Job& j, long limit) {
         std::lock_guard<std::mutex> lk(m_);
-        const long more = limit - j.limit;
         j.limit = limit;
-        wake(more);
+        call(j);
     }
     // the calling thread takes a piece; false if there is none to claim
     bool step(Job& j) {
@@ -106,10 +118,30 @@ class Helpers {
     }
 
   private:
+    struct One {
+        pthread_t thread;
+        std::condition_variable work;
+        long long called = 0;  // when; 0: not
+    };
+    static long long now() {
+        timespec t;
+        clock_gettime(CLOCK_MONOTONIC, &t);
+        return t.tv_sec * 1000000000ll + t.tv_nsec;
+    }
+    static bool claimable(const Job& j) { return j.next < std::min(j.limit, j.total); }
+    // a helper, if there is a piece for it and none is on its way
+    void call(const Job& j) {
+        if (!claimable(j) || calling_ || idle_ == 0) return;
+        One& o = *idle_at_[--idle_];
+        o.called = now();
+        calling_ = true;
+        o.work.notify_one();
+    }
     bool one(Job& j, std::unique_lock<std::mutex>& lk) {
-        if (j.next >= std::min(j.limit, j.total)) return false;
+        if (!claimable(j)) return false;
         const long i = j.next++;
         j.active++;
+        call(j);
         lk.unlock();
         j.run(i);
         lk.lock();
@@ -118,31 +150,38 @@ class Helpers {
         done_.notify_all();
         return true;
     }
-    void wake(long pieces) {
-        for (long k = 0; k < pieces && k < n_; k++) work_.notify_one();
-    }
     static void* loop(void* p) {
-        Helpers& h = *(Helpers*)p;
+        Helpers& h = get();
+        One& me = *(One*)p;
         std::unique_lock<std::mutex> lk(h.m_);
         while (!h.stop_) {
-            bool any = false;
-            for (Job*& j : h.jobs_)
-                if (j && h.one(*j, lk)) {
-                    any = true;
-                    break;
-                }
-            if (!any) h.work_.wait(lk);
+            h.idle_at_[h.idle_++] = &me;
+            me.work.wait(lk, [&] { return h.stop_ || me.called != 0; });
+            if (h.stop_) break;
+            bool any = now() - me.called <= kLate;
+            me.called = 0;
+            h.calling_ = false;
+            while (any) {
+                any = false;
+                for (Job*& j : h.jobs_)
+                    if (j && h.one(*j, lk)) {
+                        any = true;
+                        break;
+                    }
+            }
         }
         return nullptr;
     }
 
     const pid_t pid_ = getpid();
     std::mutex life_, m_;
-    std::condition_variable work_, done_;
+    std::condition_variable done_;
     Job* jobs_[8] = {};
-    pthread_t th_[kMax];
-    std::atomic<int> n_{0};
-    int users_ = 0;
+    One one_[kMax];
+    One* idle_at_[kMax];
+    int idle_ = 0;
+    bool calling_ = false;  // a helper that has been called has not come yet
+    int n_ = 0, users_ = 0;
     bool stop_ = false;
 };
 

@@ -1,8 +1,29 @@
 // Scenarios of transfer.hpp on the CPU; argv[1] names one.  Exit status 0: as it should be.
+#include <pthread.h>
+#include <sched.h>
+#include <time.h>
+#include <unistd.h>
+
+#include <atomic>
+#include <condition_variable>
 #include <cstdio>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
+// the clock of all threads but the main one may be made to run ahead
+static const std::thread::id main_thread = std::this_thread::get_id();
+static std::atomic<long> ahead_ns{0};
+static int skewed_clock(clockid_t id, timespec* t) {
+    const int r = clock_gettime(id, t);
+    if (std::this_thread::get_id() == main_thread) return r;
+    t->tv_nsec += ahead_ns;
+    t->tv_sec += t->tv_nsec / 1000000000;
+    t->tv_nsec %= 1000000000;
+    return r;
+}
+#define clock_gettime skewed_clock
 #include "transfer.hpp"
 
 using gf::HostRing;
@@ -54,11 +75,35 @@ int coherent() {
     if (fake.host_allocs > 0 && (fake.host_flags & hipHostMallocCoherent)) return 0;
     return printf("flags %#x\n", fake.host_flags), 1;
 }
+
+// pieces of 1 ms that helpers took
+int by_helpers(HostRing& r) {
+    std::atomic<int> others{0};
+    gf::in_parts(r, 40, [&](long) {
+        others += std::this_thread::get_id() != main_thread;
+        usleep(1000);
+    });
+    return others;
+}
+// helpers that come 10 ms after they were called take nothing; the next ones that come at once do
+int late_helper() {
+    cpu_set_t set;
+    if (sched_getaffinity(0, sizeof set, &set) == 0 && CPU_COUNT(&set) < 2) return 0;  // no helpers
+    HostRing r;
+    r.shape(96 * kUnit, 0);
+    ahead_ns = 10000000;
+    const int late = by_helpers(r);
+    ahead_ns = 0;
+    const int in_time = by_helpers(r);
+    r.free();
+    return late == 0 && in_time > 0 ? 0 : (printf("pieces taken late %d, in time %d\n", late, in_time), 1);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "failed_wait") return failed_wait();
     if (what == "coherent") return coherent();
+    if (what == "late_helper") return late_helper();
     return printf("no scenario %s\n", what.c_str()), 2;
 }
