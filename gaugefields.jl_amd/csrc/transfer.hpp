@@ -8,6 +8,7 @@
 #pragma once
 #include <pthread.h>
 #include <sched.h>
+#include <signal.h>
 #include <time.h>
 #include <unistd.h>
 
@@ -60,7 +61,12 @@ class Helpers {
         pthread_attr_t at;
         if (pthread_attr_init(&at) != 0) return;
         (void)pthread_attr_setstacksize(&at, 2 << 20);
+        sigset_t all, mask;  // the program's signals are for its own threads
+        sigfillset(&all);
+        for (const int own : {SIGSEGV, SIGBUS, SIGFPE, SIGILL, SIGTRAP}) sigdelset(&all, own);
+        (void)pthread_sigmask(SIG_SETMASK, &all, &mask);
         while (n_ < std::min(kMax, cpus - 1) && pthread_create(&one_[n_].thread, &at, loop, &one_[n_]) == 0) n_++;
+        (void)pthread_sigmask(SIG_SETMASK, &mask, nullptr);
         pthread_attr_destroy(&at);
     }
     void release() {

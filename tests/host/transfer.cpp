@@ -1,6 +1,7 @@
 // Scenarios of transfer.hpp on the CPU; argv[1] names one.  Exit status 0: as it should be.
 #include <pthread.h>
 #include <sched.h>
+#include <signal.h>
 #include <time.h>
 #include <unistd.h>
 
@@ -98,6 +99,22 @@ int late_helper() {
     r.free();
     return late == 0 && in_time > 0 ? 0 : (printf("pieces taken late %d, in time %d\n", late, in_time), 1);
 }
+
+// a signal to the process that the program has blocked stays pending: no helper takes it
+int blocked_signal() {
+    HostRing r;
+    r.shape(96 * kUnit, 0);
+    (void)by_helpers(r);
+    sigset_t set;
+    sigemptyset(&set);
+    sigaddset(&set, SIGUSR1);
+    pthread_sigmask(SIG_BLOCK, &set, nullptr);
+    kill(getpid(), SIGUSR1);
+    usleep(100000);
+    sigpending(&set);
+    r.free();
+    return sigismember(&set, SIGUSR1) ? 0 : 1;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -105,5 +122,6 @@ int main(int argc, char** argv) {
     if (what == "failed_wait") return failed_wait();
     if (what == "coherent") return coherent();
     if (what == "late_helper") return late_helper();
+    if (what == "blocked_signal") return blocked_signal();
     return printf("no scenario %s\n", what.c_str()), 2;
 }
