@@ -192,7 +192,7 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
     int s, mu;
     R6<T> own;
     T c[8];
-    if (!ta_force<ST, T>(g, U, s, mu, own, c)) return;
+    if (!ta_force<ST>(g, U, s, mu, own, c)) return;
     force_out<T, MODE>(c, [&] { return full_of(own); }, (unsigned)g.V, mu, s, FP, Unew, fac, eps_u, eps_p, U64);
 }
 

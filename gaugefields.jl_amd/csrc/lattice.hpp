@@ -708,6 +708,19 @@ __device__ __forceinline__ R6<T> shared_link(XLinks<T> ol, int d, int l) {
     return r;
 }
 
+// TA(u m), in the precision of the coefficients
+template <typename T, typename A>
+__device__ __forceinline__ void ta_of_product(const R6<T>& u, const M3<T>& m, A c[8]) {
+    if constexpr (std::is_same<T, A>::value)
+        ta_coeffs(mul(full_of(u), m), c);
+    else {
+        R6<T> t = u;  // opaque: what it is widened to is not kept for a later use of u (142 -> 118 VGPRs)
+#pragma unroll
+        for (int e = 0; e < 6; e++) asm volatile("" : "+v"(t.v[e].x), "+v"(t.v[e].y));
+        ta_coeffs(mul(full_of(r6_f64(t)), to_f64(m)), c);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // TA(U_mu(x) Sigma_mu(x)) (8 su(3) coefficients, ta_coeffs) with the upper staples taken as
 // whole plaquettes shared between directions.  U_mu(x) X_mu,nu U_nu(x)^dag is the plaquette
@@ -720,12 +733,14 @@ __device__ __forceinline__ R6<T> shared_link(XLinks<T> ol, int d, int l) {
 // TA(U_mu Sigma_mu) up to rounding.  Two workgroup barriers (every lane must reach them: lanes past
 // the last site work on a clamped one, and the kernels store nothing for them).
 // LDS: ol[4][6][kXW] links and tp[6][4][64] coefficient pairs (50 KB FP64: three workgroups per CU).
+// A: the type of the coefficients.  A = double over float links (the stout levels' Q and exp(Q) U): staples in float,
+// their products with U_mu, the TA projection and the sums in double.
 template <typename T>
 using PairShare = T2<T> (*)[4][64];
-template <bool ROWS, typename T>
+template <bool ROWS, typename T, typename A>
 __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict__ U, unsigned V, int s,
                                               const int x[4], int mu, R6<T>& own, XLinks<T> ol,
-                                              PairShare<T> tp, T c[8]) {
+                                              PairShare<A> tp, A c[8]) {
     const int lane = (int)(threadIdx.x & 63u);
     const XRow xr = xrow_of<ROWS>(g, s, x[0], lane);
     int fw[4];
@@ -744,7 +759,7 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
         acc_mul_dn(sig, X, full_of(lds_link(0, xr.m)));
     }
     own = lds_link(mu, lane);  // read back rather than held through the staples
-    ta_coeffs(mul(full_of(own), sig), c);
+    ta_of_product(own, sig, c);
     // pin c here: otherwise the staple arithmetic is sunk past the pairs to its use
     asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]),
                  "+v"(c[7]));
@@ -757,12 +772,15 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
         // X_ab = U_b(x+a) U_a(x+b)^dag
         const R6<T> ub = a == 0 ? lds_link(b, xr.p) : ldr(U, V, b, (unsigned)(s + sel4(a, fw[0], fw[1], fw[2], fw[3])));
         const M3<T> X = su3_mul_nd(ub, ldu(U, V, a, (unsigned)(s + sel4(b, fw[0], fw[1], fw[2], fw[3]))));
-        T q8[8];
-        ta_coeffs(su3_mul_nd(rows_of(su3_mul(lds_link(a, lane), X)), full_of(lds_link(b, lane))), q8);
+        A q8[8];
+        if constexpr (std::is_same<T, A>::value)
+            ta_coeffs(su3_mul_nd(rows_of(su3_mul(lds_link(a, lane), X)), full_of(lds_link(b, lane))), q8);
+        else
+            ta_of_product(lds_link(a, lane), mul_nd(X, full_of(lds_link(b, lane))), q8);
         const int p = pair_index(a, b);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            T2<T> v;
+            T2<A> v;
             v.x = q8[2 * e];
             v.y = q8[2 * e + 1];
             tp[p][e][lane] = v;
@@ -773,10 +791,10 @@ __device__ __forceinline__ void ta_force_xrow(const Geo& g, const T* __restrict_
     for (int j = 0; j < 3; j++) {
         const int nu = j + (j >= mu ? 1 : 0);
         const int p = pair_index(mu < nu ? mu : nu, mu < nu ? nu : mu);
-        const T sg = mu < nu ? T(1) : T(-1);
+        const A sg = mu < nu ? A(1) : A(-1);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const T2<T> v = tp[p][e][lane];
+            const T2<A> v = tp[p][e][lane];
             c[2 * e] = fma(sg, v.x, c[2 * e]);
             c[2 * e + 1] = fma(sg, v.y, c[2 * e + 1]);
         }
@@ -862,18 +880,18 @@ __device__ __forceinline__ bool wide_sum(M3<T>& m, int j, T2<T> (*red)[9][64]) {
     return true;
 }
 // TA(U_mu Sigma_mu) in wave 0 (true), each wave's from its own plane's staples
-template <typename T>
+template <typename T, typename A>
 __device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict__ U, const WideIndex& wi,
-                                              R6<T>& own, T2<T> (*tp)[4][64], T c[8]) {
+                                              R6<T>& own, T2<A> (*tp)[4][64], A c[8]) {
     const int lane = (int)(threadIdx.x & 63u);
     int x[4];
     decode(g, wi.s, x);
     const M3<T> sig = staples_of_plane(g, U, (unsigned)g.V, wi.s, x, wi.mu, wi.j + (wi.j >= wi.mu ? 1 : 0), own);
-    ta_coeffs(mul(full_of(own), sig), c);
+    ta_of_product(own, sig, c);
     if (wi.j > 0) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            T2<T> v;
+            T2<A> v;
             v.x = c[2 * e];
             v.y = c[2 * e + 1];
             tp[wi.j - 1][e][lane] = v;
@@ -885,7 +903,7 @@ __device__ __forceinline__ bool ta_force_wide(const Geo& g, const T* __restrict_
     for (int k = 0; k < 2; k++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const T2<T> v = tp[k][e][lane];
+            const T2<A> v = tp[k][e][lane];
             c[2 * e] += v.x;
             c[2 * e + 1] += v.y;
         }
@@ -908,20 +926,20 @@ inline int stencil_form(const Geo& g) {
 constexpr int stencil_threads(int form) { return form == ST_WIDE ? 192 : 256; }
 constexpr int stencil_groups(int form, int groups) { return form == ST_WIDE ? 4 * groups : groups; }
 // links and coefficient pairs a workgroup shares
-template <typename T, int ST>
+template <typename T, int ST, typename A>
 struct ForceShare {
     T2<T> ol[4][6][kXW];
-    T2<T> tp[6][4][64];
+    T2<A> tp[6][4][64];
 };
-template <typename T>
-struct ForceShare<T, ST_WIDE> {
-    T2<T> tp[2][4][64];
+template <typename T, typename A>
+struct ForceShare<T, ST_WIDE, A> {
+    T2<A> tp[2][4][64];
 };
 // The workgroup's waves, with the site and U_mu(x) they work on, and TA(U_mu Sigma_mu) in c; false for the
 // waves and lanes that have nothing to store.
-template <int ST, typename T>
-__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, T c[8]) {
-    __shared__ ForceShare<T, ST> sh;
+template <int ST, typename T, typename A>
+__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, A c[8]) {
+    __shared__ ForceShare<T, ST, A> sh;
     if constexpr (ST == ST_WIDE) {
         const WideIndex wi = wide_index(g);
         s = wi.s;

@@ -1011,8 +1011,8 @@ __device__ __forceinline__ M3<T> round_link(const M3<double>& d) {
 }
 
 // exp(i t sum_a c_a lambda_a / 2) U
-template <typename T>
-__device__ __forceinline__ M3<T> exp_coeffs_times(const T c[8], double t, const M3<T>& u) {
+template <typename T, typename A>
+__device__ __forceinline__ M3<T> exp_coeffs_times(const A c[8], double t, const M3<T>& u) {
     if constexpr (std::is_same<T, float>::value) {
         double cd[8];
 #pragma unroll

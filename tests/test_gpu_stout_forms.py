@@ -1,0 +1,36 @@
+"""The stout kernels in the forms that lattices beyond the smallest take, against the CPU oracle.
+
+Extents: one small lattice (at most 160 groups of 64 sites in FP64, 256 in FP32), whole rows (NX divides 64, V a multiple
+of 64) and rows cut by the groups with idle lanes, above both limits.
+"""
+import numpy as np
+import pytest
+
+import lattice_tools as lt
+
+pytestmark = pytest.mark.gpu
+
+gen = lt.gen
+SMALL, ROWS, CUT = (8, 8, 8, 8), (16, 16, 16, 6), (18, 10, 10, 10)
+
+
+def links(oracle, dims, seed, spread=0.3):
+    U = gen.cold_links(dims)
+    oracle.exp_update(dims, U, gen.algebra_coefficients(dims, spread, seed), 1.0)
+    return U
+
+
+# One FP32 level at rho = 1, where the error of Q outweighs the rounding of the stored link (1e-8): RMS of rows 0 and 1
+# against the FP64 level of the same float links.  A numpy emulation of the kernel's products on such links (float FMAs
+# for the staples, the product with U, the TA projection and the sum in double) gives 5.0e-8, with the products, TA and
+# the sum in float as well 7.7e-8; the bar lies 1.2 above the first.
+@pytest.mark.parametrize("dims", [SMALL, ROWS, CUT])
+def test_fp32_level_forms_q_in_double(gf, oracle, dims):
+    print(f"[stout] FP32 level {dims}", flush=True)
+    with gf.Lattice(dims, precision="f32") as L:
+        L.upload_links(links(oracle, dims, 71))
+        U = L.download_links()
+        L.stout_config(1, 1.0, "store")
+        S = L.stout_smear()
+    d = (S - oracle.stout_smear(dims, U, 1, 1.0)).reshape(4, -1, 3, 3)[..., :2]  # [.., j, i]: column-major
+    assert np.sqrt(np.mean(np.abs(d) ** 2)) < 1.2 * 5.03e-8
