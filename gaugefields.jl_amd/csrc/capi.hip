@@ -46,6 +46,7 @@ struct gf_ctx {
     int smode = GF_STOUT_STORE;
     void* lev[GF_MAX_LEV] = {};  // smeared levels 1..nlev
     void* Qst[GF_MAX_LEV] = {};  // Q coefficients per level (input level index; recompute mode: [0] only)
+    bool q_there = false;        // every level's Q is there and belongs to the levels as they are
     void* G = nullptr;           // Lam of the level being pulled back
     void* Fl = nullptr;          // its derivative without the far plaquette contributions
     void* far = nullptr;         // those (3 momentum fields)
@@ -407,11 +408,13 @@ int stout_forward_all(gf_ctx* c, bool with_q = false) {
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
         const bool stored = c->smode == GF_STOUT_STORE;
+        c->q_there = false;
         for (int l = 0; l < c->nlev; l++)
             HIPCHK(c, launch_stout_forward<T>(c->geo, (const T*)level_in(c, l), (T*)c->lev[l],
                                               with_q && (stored || l == c->nlev - 1) ? (T*)c->Qst[stored ? l : 0]
                                                                                      : nullptr,
                                               c->rho, c->stream));
+        c->q_there = with_q && stored;
         return GF_OK;
     });
 }
@@ -420,10 +423,13 @@ int stout_forward_all(gf_ctx* c, bool with_q = false) {
 int stout_backward_all(gf_ctx* c) {
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        const T* in[GF_MAX_LEV];
-        for (int l = 0; l < c->nlev; l++) in[l] = (const T*)level_in(c, l);
-        HIPCHK(c, launch_stout_backward<T>(c->geo, in, c->nlev, (T*)c->D, (T*)c->D2, (T*)c->G, (T*)c->Fl, c->rho,
-                                           c->stream));
+        const T *in[GF_MAX_LEV], *q[GF_MAX_LEV];
+        for (int l = 0; l < c->nlev; l++) {
+            in[l] = (const T*)level_in(c, l);
+            q[l] = (const T*)c->Qst[l];
+        }
+        HIPCHK(c, launch_stout_backward<T>(c->geo, in, c->q_there ? q : nullptr, c->nlev, (const T*)c->D, (T*)c->D2,
+                                           (T*)c->G, (T*)c->Fl, c->rho, c->stream));
         std::swap(c->D, c->D2);
         return GF_OK;
     });
@@ -1207,6 +1213,7 @@ int gf_stout_config(gf_ctx* c, int nlev, double rho, int mode) {
     c->nlev = nlev;
     c->rho = rho;
     c->smode = mode;
+    c->q_there = false;
     if (nlev > 0) TRY(stout_alloc(c));
     return GF_OK;
 }
@@ -1221,7 +1228,7 @@ int gf_stout_smear(gf_ctx* c, double* ref) {
     CTXCHK(c);
     NOT_S64(c, "calc_smearedU");
     if (c->nlev == 0) return fail(c, GF_ESTATE, "no stout levels configured");
-    TRY(stout_forward_all(c));
+    TRY(stout_forward_all(c, c->smode == GF_STOUT_STORE && stout_backward_reads_q(c->geo, c->prec == GF_F64)));
     if (ref) return download_linkfield(c, c->lev[c->nlev - 1], ref);
     return GF_OK;
 }

@@ -171,10 +171,14 @@ template <typename T>
 hipError_t launch_stout_gather(const Geo& g, const T* far, T* Fl, double rho, const T* Qst, T* Lc, hipStream_t st,
                                int fmode = -1, const T* U = nullptr, T* FP = nullptr, double eps_p = 0.0,
                                T* Unew = nullptr, double eps_u = 0.0, double* U64 = nullptr);
-// explicit backward pass of nlev levels (Uin[l] the input links of level l): D2 = dS/dU_bare from D = dS/dU
-// of the top level (general matrix fields); Lc, Lc2: scratch momentum fields
+// explicit backward pass of nlev levels: D2 = dS/dU_bare from D = dS/dU of the top level (general matrix fields).
+// Uin[l] the input links of level l, Q[l] its Q; Q null: C formed from the staples again (as in any case where
+// stout_backward_reads_q is false); Lc, Lc2: scratch momentum fields
+inline bool stout_backward_reads_q(const Geo& g, bool f64) {
+    return (f64 ? stencil_form<double>(g) : stencil_form<float>(g)) != ST_WIDE;
+}
 template <typename T>
-hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, int nlev, T* D, T* D2, T* Lc, T* Lc2, double rho,
-                                 hipStream_t st);
+hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, const T* const* Q, int nlev, const T* D, T* D2,
+                                 T* Lc, T* Lc2, double rho, hipStream_t st);
 
 }  // namespace gf

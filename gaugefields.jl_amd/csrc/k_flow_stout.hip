@@ -302,8 +302,12 @@ __global__ __launch_bounds__(kBlock) void k_stout_gather(Geo g, const T* __restr
 //   Din_mu = Dout_mu e^{Q_mu} + (Lam_mu C_mu)^dag,   Lam_mu = TA(CdexpQdQ(U_mu Dout_mu, Q_mu))
 // Lam_mu (traceless anti-Hermitian) is stored as its 8 su(3) coefficients; the staple part
 // uses G_mu = U_mu^dag Lam_mu (= dS/dC_mu) without storing it.
-// C_mu is formed from the staples again.  (Used by the explicit backward pass, whose dS/dU_in is wanted
-// as a matrix; the forces take the algebra form above.)
+// (Used by the explicit backward pass, whose dS/dU_in is wanted as a matrix; the forces take the algebra form
+// above.)  Where the smearing has kept Q_mu, it is read (back_local_q), and (Lam C)^dag = -rho Sigma Lam is left to the
+// staple part, which walks the staples of Sigma anyway: a streaming step without a stencil, done by the staple part's
+// kernel of the level above.  Otherwise, and on small lattices, C_mu is formed from the staples again (back_local).
+// Two levels, us, C formed again / Q read: FP64 16^4 197 / 165, 20^3x10 234 / 198, 24^4 888 / 748, 32^4 2953 / 2380; FP32
+// 116 / 96, 133 / 116, 500 / 418, 1555 / 1211.
 // ---------------------------------------------------------------------------
 // A 3x3 field element kept in the wave's own LDS slice between two uses (each lane reads back what
 // it wrote: no barrier), instead of being held in registers or read from memory twice.
@@ -387,7 +391,43 @@ __global__ __launch_bounds__(stencil_threads(ST)) void k_stout_back_local(Geo g,
     back_local<T>(sig, own, [&] { return ldm<T, GF_LD_NT>(Dout, V, mu, s); }, Din, Lc, rho, V, mu, s, lane,
                   dst[ST == ST_WIDE ? 0 : mu]);
 }
-
+// Lam and Din without (Lam C)^dag, from Q, the link and Dout
+template <typename T>
+__device__ __forceinline__ void back_local_q(const T q[8], const M3<T>& u, const M3<T>& dout, T* __restrict__ Din,
+                                             T* __restrict__ Lc, unsigned V, int mu, int s, int lane, MStage<T> dst) {
+    M3<T> E, L;
+    {
+        const Herm<T> h = herm_of_coeffs(q);
+        M3<T> Q;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const cx<T> e = herm_el(h, i, j);
+                Q.m[3 * i + j].r = -e.i;
+                Q.m[3 * i + j].i = e.r;
+            }
+        exp_dexp(Q, mul(u, stage_m3<T>(dst, lane, dout)), E, L);
+    }
+    T c[8];
+    ta_coeffs(L, c);
+    stp<T, GF_ST_NT>(Lc, V, mu, s, c);
+    stm<T, GF_ST_NT>(Din, V, mu, s, mul(staged_m3<T>(dst, lane), E));
+}
+// a thread per link
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_stout_back_local_q(Geo g, const T* __restrict__ U, const T* __restrict__ Qst,
+                                                               const T* __restrict__ Dout, T* __restrict__ Din, T* __restrict__ Lc) {
+    __shared__ T2<T> dst[4][9][64];
+    const SiteMu sm = site_mu_index(g);
+    const int s = sm.s, mu = sm.mu;
+    if (s >= g.V) return;
+    const unsigned V = g.V;
+    T q[8];
+    ldp<T, GF_LD_NT>(Qst, V, mu, s, q);
+    back_local_q<T>(q, ldu<T, GF_LD_NT>(U, V, mu, s), ldm<T, GF_LD_NT>(Dout, V, mu, s), Din, Lc, V, mu, s,
+                    (int)(threadIdx.x & 63u), dst[mu]);
+}
 // ---------------------------------------------------------------------------
 // K6b: stout backward, staple-derivative part (calc_dSdUν_fromdSCμ_add!, stout_fast.jl:712-785):
 // for output direction a at site y and each plane b != a, with G = U^dag Lam,
@@ -460,8 +500,10 @@ __device__ __forceinline__ void acc_hd(M3<T>& c, const Herm<T>& h, const M3<T>& 
 }
 
 // Plane b of K6b added into acc.  SH: U_b(y) and Lam_b(y) come from the workgroup's LDS copies (ul, hl);
-// A0 (a = 0) and B0 (b = 0): the x-neighbour links and Lam at y + 1 and y - 1 (xr) as well.
-template <typename T, bool SH, bool A0, bool B0>
+// A0 (a = 0) and B0 (b = 0): the x-neighbour links and Lam at y + 1 and y - 1 (xr) as well.  SL adds the plane's
+// part of -Sigma_a Lam_a: of the staples S and U_b(y+a-b)^dag U_a(y-b)^dag U_b(y-b) times H_a(y), by H_b(y) - H_a(y) in
+// place of H_b(y) and H_d - U_b(y-b) H_a(y) U_b(y-b)^dag in place of H_d.
+template <typename T, bool SL, bool SH, bool A0, bool B0>
 __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U, const T* __restrict__ Lc, unsigned V,
                                            int y, const int x[4], int a, int b, int ypa, M3<T>& acc, XLinks<T> ul,
                                            XCoefs<T> hl, int lane, const XRow& xr) {
@@ -484,6 +526,12 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
         const M3<T> S = su3_mul_nd(rows_of(X), ub);
         if (SH) get_c8(hl, b, lane, c);  // Lam_b(y)
         else ldp(Lc, V, b, (unsigned)y, c);
+        if (SL) {
+            T own[8];
+            get_c8(hl, a, lane, own);
+#pragma unroll
+            for (int k = 0; k < 8; k++) c[k] -= own[k];
+        }
         acc_i_mh<T, 1>(acc, S, herm_of_coeffs(c));
         if (A0) get_c8(hl, b, xr.p, c);  // Lam_b(y+a)
         else ldp(Lc, V, b, y1, c);
@@ -493,18 +541,37 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
        // H_d = H_a(y-b) - H_b(y-b)
         int ymb = ymb0, ypamb = ypamb0;
         asm volatile("" : "+v"(ymb), "+v"(ypamb));
-        const M3<T> ua = full_of(B0 ? shared_link<T>(ul, a, xr.m) : ldr(U, V, a, ymb));  // U_a(y-b)
-        T ca[8], cb[8];
-        if (B0) {
-            get_c8(hl, a, xr.m, ca);
-            get_c8(hl, 0, xr.m, cb);
-        } else {
-            ldp(Lc, V, a, ymb, ca);
-            ldp(Lc, V, b, ymb, cb);
-        }
+        Herm<T> hd;
+        {
+            T ca[8], cb[8];
+            if (B0) {
+                get_c8(hl, a, xr.m, ca);
+                get_c8(hl, 0, xr.m, cb);
+            } else {
+                ldp(Lc, V, a, ymb, ca);
+                ldp(Lc, V, b, ymb, cb);
+            }
 #pragma unroll
-        for (int k = 0; k < 8; k++) ca[k] -= cb[k];
-        M3<T> A = mul_dh(ua, herm_of_coeffs(ca));
+            for (int k = 0; k < 8; k++) ca[k] -= cb[k];
+            hd = herm_of_coeffs(ca);
+        }
+        if (SL) {
+            T own[8];
+            get_c8(hl, a, lane, own);
+            const Herm<T> t = herm_conj(full_of(B0 ? shared_link<T>(ul, 0, xr.m) : ldr(U, V, b, ymb)), herm_of_coeffs(own));
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                hd.d[k] -= t.d[k];
+                hd.u[k].r -= t.u[k].r;
+                hd.u[k].i -= t.u[k].i;
+            }
+            // formed before the links below are loaded (registers)
+#pragma unroll
+            for (int k = 0; k < 3; k++) asm volatile("" : "+v"(hd.d[k]), "+v"(hd.u[k].r), "+v"(hd.u[k].i));
+            asm volatile("" : "+v"(ymb), "+v"(ypamb));
+        }
+        const M3<T> ua = full_of(B0 ? shared_link<T>(ul, a, xr.m) : ldr(U, V, a, ymb));  // U_a(y-b)
+        M3<T> A = mul_dh(ua, hd);
         acc_hd(A, herm_at(Lc, V, b, ypamb), ua);
         const M3<T> ubm = full_of(B0 ? shared_link<T>(ul, 0, xr.m) : ldr(U, V, b, ymb));  // U_b(y-b)
         acc_mul_dn(acc, ldu(U, V, b, ypamb), times_i(mul(A, ubm)));
@@ -514,7 +581,7 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
 // The staple part of K6b for output direction a at site y (all planes b != a).  U(y) and Lam(y) of
 // the workgroup's sites and of their x-neighbours go through LDS (per wave 12 link and 6 Lam loads
 // fewer than from memory); one workgroup barrier after filling ul/hl.
-template <bool ROWS, typename T>
+template <bool ROWS, bool SL, typename T>
 __device__ __forceinline__ M3<T> back_stencil_acc(const Geo& g, const T* __restrict__ U, const T* __restrict__ Lc,
                                                   int y, const int x[4], int a, int lane, XLinks<T> ul,
                                                   XCoefs<T> hl) {
@@ -536,13 +603,13 @@ __device__ __forceinline__ M3<T> back_stencil_acc(const Geo& g, const T* __restr
     const int ypa = y + dlt(g, x, a, 1);
     if (a == 0) {
 #pragma unroll 1
-        for (int b = 1; b < 4; b++) back_plane<T, true, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
+        for (int b = 1; b < 4; b++) back_plane<T, SL, true, true, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
     } else {
-        back_plane<T, true, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, xr);
+        back_plane<T, SL, true, false, true>(g, U, Lc, V, y, x, a, 0, ypa, acc, ul, hl, lane, xr);
 #pragma unroll 1
         for (int b = 1; b < 4; b++) {
             if (b == a) continue;
-            back_plane<T, true, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
+            back_plane<T, SL, true, false, false>(g, U, Lc, V, y, x, a, b, ypa, acc, ul, hl, lane, xr);
         }
     }
     return acc;
@@ -559,37 +626,50 @@ __device__ __forceinline__ M3<T> back_din(const T* __restrict__ Din, unsigned V,
     }
     return dn;
 }
-// K6b: Din += rho (staple part).  At most 168 VGPRs (FP64), so that three waves fit per SIMD.
-template <typename T, int ST>
-__global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil(
-    Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho) {
+// K6b: Din += rho (staple part; SL: and -Sigma Lam).  LOCAL: followed by K6a of the level below (Uprev its input links,
+// Qprev its Q), whose Dout this Din is: not stored and read back (1152 B a site in FP64).  Lout is another buffer than Lc,
+// whose entries at neighbour sites other workgroups still read.  At most 168 VGPRs (FP64), so that three waves fit per
+// SIMD; with K6a two.
+template <typename T, bool ROWS, bool SL, bool LOCAL>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(LOCAL && sizeof(T) == 8 ? 2 : 3))) void
+k_stout_back_stencil(Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho,
+                     const T* __restrict__ Uprev, const T* __restrict__ Qprev, T* __restrict__ Lout) {
+    // links and Lam of the sites and their x-neighbours; then Dout of the level below
+    __shared__ __align__(16) unsigned char sh[4 * 10 * kXW * sizeof(T2<T>)];
+    XLinks<T> ul = reinterpret_cast<XLinks<T>>(sh);
+    XCoefs<T> hl = reinterpret_cast<XCoefs<T>>(sh + 4 * 6 * kXW * sizeof(T2<T>));
     const unsigned V = g.V;
     const int lane = (int)(threadIdx.x & 63u);
-    int y, a, x[4];
-    M3<T> acc;
-    bool valid;
-    if constexpr (ST == ST_WIDE) {
-        __shared__ T2<T> red[2][9][64];
-        const WideIndex wi = wide_index(g);
-        y = wi.s;
-        a = wi.mu;
-        decode(g, y, x);
-        acc = zero3<T>();
-        back_plane<T, false, false, false>(g, U, Lc, V, y, x, a, wi.j + (wi.j >= a ? 1 : 0), y + dlt(g, x, a, 1), acc,
-                                           nullptr, nullptr, lane, XRow{});
-        valid = wide_sum(acc, wi.j, red) && wi.site < g.V;
+    const SiteMu sm = site_mu_index(g);
+    const int a = sm.mu, y = stencil_site<ROWS>(g, sm);
+    int x[4];
+    decode(g, y, x);
+    const M3<T> acc = back_stencil_acc<ROWS, SL>(g, U, Lc, y, x, a, lane, ul, hl);
+    if constexpr (LOCAL) __syncthreads();  // every wave is done with ul and hl
+    if (!in_lattice<ROWS>(g, sm)) return;
+    const M3<T> dn = back_din(Din, V, a, y, rho, acc);
+    if constexpr (LOCAL) {
+        MStage<T> dst = reinterpret_cast<T2<T>(*)[9][64]>(sh)[a];
+        T q[8];
+        ldp<T, GF_LD_NT>(Qprev, V, a, y, q);
+        back_local_q<T>(q, ldu<T, GF_LD_NT>(Uprev, V, a, y), dn, Din, Lout, V, a, y, lane, dst);
     } else {
-        __shared__ T2<T> ul[4][6][kXW];
-        __shared__ T2<T> hl[4][4][kXW];
-        const SiteMu sm = site_mu_index(g);
-        a = sm.mu;
-        y = stencil_site<ST == ST_ROWS>(g, sm);
-        decode(g, y, x);
-        acc = back_stencil_acc<ST == ST_ROWS, T>(g, U, Lc, y, x, a, lane, ul, hl);
-        valid = in_lattice<ST == ST_ROWS>(g, sm);
+        stm<T, GF_ST_NT>(Din, V, a, y, dn);
     }
-    if (!valid) return;
-    stm<T, GF_ST_NT>(Din, V, a, y, back_din(Din, V, a, y, rho, acc));
+}
+template <typename T>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil_wide(
+    Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho) {
+    __shared__ T2<T> red[2][9][64];
+    const WideIndex wi = wide_index(g);
+    const int y = wi.s, a = wi.mu;
+    int x[4];
+    decode(g, y, x);
+    M3<T> acc = zero3<T>();
+    back_plane<T, false, false, false, false>(g, U, Lc, (unsigned)g.V, y, x, a, wi.j + (wi.j >= a ? 1 : 0), y + dlt(g, x, a, 1),
+                                       acc, nullptr, nullptr, (int)(threadIdx.x & 63u), XRow{});
+    if (!wide_sum(acc, wi.j, red) || wi.site >= g.V) return;
+    stm<T, GF_ST_NT>(Din, (unsigned)g.V, a, y, back_din(Din, (unsigned)g.V, a, y, rho, acc));
 }
 
 // K6b of a level and K6a of the one below (Uprev its input links) in one launch, on small lattices: the
@@ -611,7 +691,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(1))) void k
 #pragma unroll
     for (int e = 0; e < 9; e++) asm volatile("" : "+v"(sig.m[e].r), "+v"(sig.m[e].i));  // one stencil after the other
     M3<T> acc = zero3<T>();
-    back_plane<T, false, false, false>(g, U, Lc, V, wi.s, x, a, b, wi.s + dlt(g, x, a, 1), acc, nullptr, nullptr, lane,
+    back_plane<T, false, false, false, false>(g, U, Lc, V, wi.s, x, a, b, wi.s + dlt(g, x, a, 1), acc, nullptr, nullptr, lane,
                                        XRow{});
     const bool first = wide_sum(sig, wi.j, red[0]);
     wide_sum(acc, wi.j, red[1]);
@@ -697,23 +777,31 @@ hipError_t launch_stout_gather(const Geo& g, const T* far, T* Fl, double rho, co
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, int nlev, T* D, T* D2, T* Lc, T* Lc2, double rho,
-                                 hipStream_t st) {
-    const int groups = grid_sites_mu(g.V);
+hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, const T* const* Q, int nlev, const T* D, T* D2,
+                                 T* Lc, T* Lc2, double rho, hipStream_t st) {
+    const int groups = grid_sites_mu(g.V), top = nlev - 1;
+    T *la = Lc, *lb = Lc2;
     if (stencil_form<T>(g) == ST_WIDE) {
         const int nb = stencil_groups(ST_WIDE, groups), nt = stencil_threads(ST_WIDE);
-        T *la = Lc, *lb = Lc2;
-        k_stout_back_local<T, ST_WIDE><<<nb, nt, 0, st>>>(g, Uin[nlev - 1], D, D2, la, rho);
-        for (int l = nlev - 1; l >= 1; l--, std::swap(la, lb))
+        k_stout_back_local<T, ST_WIDE><<<nb, nt, 0, st>>>(g, Uin[top], D, D2, la, rho);
+        for (int l = top; l >= 1; l--, std::swap(la, lb))
             k_stout_back_chain_wide<T><<<nb, nt, 0, st>>>(g, Uin[l], la, D2, rho, Uin[l - 1], lb);
-        k_stout_back_stencil<T, ST_WIDE><<<nb, nt, 0, st>>>(g, Uin[0], la, D2, rho);
+        k_stout_back_stencil_wide<T><<<nb, nt, 0, st>>>(g, Uin[0], la, D2, rho);
         return hipGetLastError();
     }
     by_rows(g, [&](auto rows) {
-        constexpr int ST = decltype(rows)::value ? ST_ROWS : ST_CUT;
-        for (int l = nlev - 1; l >= 0; l--) {
-            k_stout_back_local<T, ST><<<groups, kBlock, 0, st>>>(g, Uin[l], l == nlev - 1 ? D : D2, D2, Lc, rho);
-            k_stout_back_stencil<T, ST><<<groups, kBlock, 0, st>>>(g, Uin[l], Lc, D2, rho);
+        constexpr bool R = decltype(rows)::value;
+        if (Q) {
+            k_stout_back_local_q<T><<<groups, kBlock, 0, st>>>(g, Uin[top], Q[top], D, D2, la);
+            for (int l = top; l >= 1; l--, std::swap(la, lb))
+                k_stout_back_stencil<T, R, true, true><<<groups, kBlock, 0, st>>>(g, Uin[l], la, D2, rho, Uin[l - 1], Q[l - 1], lb);
+            k_stout_back_stencil<T, R, true, false><<<groups, kBlock, 0, st>>>(g, Uin[0], la, D2, rho, nullptr, nullptr, nullptr);
+            return;
+        }
+        constexpr int ST = R ? ST_ROWS : ST_CUT;
+        for (int l = top; l >= 0; l--) {
+            k_stout_back_local<T, ST><<<groups, kBlock, 0, st>>>(g, Uin[l], l == top ? D : D2, D2, la, rho);
+            k_stout_back_stencil<T, R, false, false><<<groups, kBlock, 0, st>>>(g, Uin[l], la, D2, rho, nullptr, nullptr, nullptr);
         }
     });
     return hipGetLastError();
@@ -726,8 +814,8 @@ hipError_t launch_stout_backward(const Geo& g, const T* const* Uin, int nlev, T*
     template hipError_t launch_stout_pair<T>(const Geo&, const T*, const T*, T*, T*, double, hipStream_t); \
     template hipError_t launch_stout_gather<T>(const Geo&, const T*, T*, double, const T*, T*, hipStream_t, int, \
                                                const T*, T*, double, T*, double, double*);                \
-    template hipError_t launch_stout_backward<T>(const Geo&, const T* const*, int, T*, T*, T*, T*, double,  \
-                                                 hipStream_t);
+    template hipError_t launch_stout_backward<T>(const Geo&, const T* const*, const T* const*, int, const T*, T*,  \
+                                                 T*, T*, double, hipStream_t);
 
 GF_INST2(double)
 GF_INST2(float)

@@ -183,10 +183,12 @@ int gf_flow_measure(gf_ctx *ctx, double eps, int nsteps, int every, double *out)
 
 /* ---- stout smearing ---------------------------------------------------------------- */
 /* nlev stout layers at rho (STOUT_Layer + CovNeuralnet, stout_fast.jl:6-122,
- * Abstractsmearing.jl:61-99); mode GF_STOUT_STORE keeps every level's Q_mu (8 reals a link),
- * GF_STOUT_RECOMPUTE forms it again in the backward pass, GF_STOUT_AUTO stores when the device has
- * room for the nlev momentum-sized fields (plus a 10 % margin) and recomputes otherwise.  The smeared
- * levels themselves are always kept.  nlev = 0 disables smearing. */
+ * Abstractsmearing.jl:61-99); mode GF_STOUT_STORE keeps every level's Q_mu (8 reals a link) for the
+ * forces and for gf_stout_backward, GF_STOUT_RECOMPUTE forms it (gf_stout_backward: C_mu) again in the
+ * backward pass, GF_STOUT_AUTO stores when the device has room for the nlev momentum-sized fields (plus
+ * a 10 % margin) and recomputes otherwise.  gf_stout_backward forms C_mu again in every mode on small
+ * lattices, and when other calls have smeared the links since gf_stout_smear.  The smeared levels
+ * themselves are always kept.  nlev = 0 disables smearing. */
 int gf_stout_config(gf_ctx *ctx, int nlev, double rho, int mode);
 /* the memory mode in effect after gf_stout_config (GF_STOUT_STORE or GF_STOUT_RECOMPUTE) */
 int gf_stout_mode(const gf_ctx *ctx, int *mode);

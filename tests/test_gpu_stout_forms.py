@@ -34,3 +34,34 @@ def test_fp32_level_forms_q_in_double(gf, oracle, dims):
         S = L.stout_smear()
     d = (S - oracle.stout_smear(dims, U, 1, 1.0)).reshape(4, -1, 3, 3)[..., :2]  # [.., j, i]: column-major
     assert np.sqrt(np.mean(np.abs(d) ** 2)) < 1.2 * 5.03e-8
+
+
+def backward(oracle, dims, U, nlev, rho, D):
+    for l in range(nlev, 0, -1):
+        D = oracle.stout_backward(dims, oracle.stout_smear(dims, U, l - 1, rho) if l > 1 else U, rho, D)
+    return D
+
+
+# The explicit backward pass above the small lattices' limits: the top level's site-local step, the staple part with and
+# without the next level's step behind it, and Q kept by the smearing, formed again (recompute), and formed again because
+# the Hamiltonian has smeared the links anew.  FP64: 1e-13 a level, as at 4^4; FP32: 2e-5 of the largest element, the bar of
+# the three-level force.
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("dims", [SMALL, ROWS, CUT, (131, 3, 7, 6)])
+@pytest.mark.parametrize("nlev,rho", [(1, 0.5), (3, 0.12)])
+def test_explicit_backward(gf, oracle, dims, precision, nlev, rho):
+    print(f"[stout] backward {dims} {precision} {nlev}", flush=True)
+    D = gen.hot_start_links(dims, 43)
+    with gf.Lattice(dims, precision=precision) as L:
+        L.upload_links(links(oracle, dims, 42))
+        U = L.download_links()
+        ref = backward(oracle, dims, U, nlev, rho, D)
+        bar = nlev * 1e-13 if precision == "f64" else 2e-5 * np.abs(ref).max()
+        L.stout_config(nlev, rho, "store")
+        L.stout_smear(download=False)
+        assert np.abs(L.stout_backward(D) - ref).max() < bar
+        L.hamiltonian(3.0)
+        assert np.abs(L.stout_backward(D) - ref).max() < bar
+        L.stout_config(nlev, rho, "recompute")
+        L.stout_smear(download=False)
+        assert np.abs(L.stout_backward(D) - ref).max() < bar
