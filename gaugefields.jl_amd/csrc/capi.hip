@@ -49,9 +49,8 @@ struct gf_ctx {
     bool q_there = false;        // every level's Q is there and belongs to the levels as they are
     void* G = nullptr;           // Lam of the level being pulled back
     void* Fl = nullptr;          // its derivative without the far plaquette contributions
-    void* far = nullptr;         // those (3 momentum fields)
-    void* D = nullptr;           // explicit derivative, explicit backward pass (general matrices)
-    void* D2 = nullptr;
+    void* far = nullptr;         // those (3 momentum fields); explicit backward pass: dS/dU as it comes in
+    void* D = nullptr;           // explicit derivative, result of the explicit backward pass (general matrices)
     // FP32 bulk: FP64 copies of the links (and smeared levels, ping-pong) for the Hamiltonian
     void* W64[2] = {nullptr, nullptr};
     // FP32 forces over an FP64 state: the links and momenta as held and updated (U holds the links
@@ -419,7 +418,7 @@ int stout_forward_all(gf_ctx* c, bool with_q = false) {
     });
 }
 
-// explicit backward pass: D (dS/dU of the top level) -> D holds dS/dU_bare
+// explicit backward pass: far (dS/dU of the top level) -> D holds dS/dU_bare
 int stout_backward_all(gf_ctx* c) {
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
@@ -428,9 +427,8 @@ int stout_backward_all(gf_ctx* c) {
             in[l] = (const T*)level_in(c, l);
             q[l] = (const T*)c->Qst[l];
         }
-        HIPCHK(c, launch_stout_backward<T>(c->geo, in, c->q_there ? q : nullptr, c->nlev, (const T*)c->D, (T*)c->D2,
+        HIPCHK(c, launch_stout_backward<T>(c->geo, in, c->q_there ? q : nullptr, c->nlev, (const T*)c->far, (T*)c->D,
                                            (T*)c->G, (T*)c->Fl, c->rho, c->stream));
-        std::swap(c->D, c->D2);
         return GF_OK;
     });
 }
@@ -705,7 +703,7 @@ int gf_destroy(gf_ctx* c) {
     if (!c) return GF_EINVAL;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void** bufs[] = {&c->U,   &c->Ualt, &c->Ubak, &c->P,      &c->F,      &c->A,   &c->D,   &c->D2,
+    void** bufs[] = {&c->U,   &c->Ualt, &c->Ubak, &c->P,      &c->F,      &c->A,   &c->D,
                      &c->G,   &c->Fl,   &c->far, &c->W64[0], &c->W64[1], &c->U64, &c->P64, &c->U64bak};
     for (void** b : bufs)
         if (*b) (void)hipFree(*b);
@@ -1195,7 +1193,8 @@ int gf_stout_config(gf_ctx* c, int nlev, double rho, int mode) {
     if (mode != GF_STOUT_STORE && mode != GF_STOUT_RECOMPUTE && mode != GF_STOUT_AUTO)
         return fail(c, GF_EINVAL, "unknown stout mode %d", mode);
     if (mode == GF_STOUT_AUTO) {
-        // bytes still to allocate for levels, backward buffers and (if stored) Q per level
+        // bytes still to allocate for levels, backward buffers (those of gf_stout_backward too, which come with its
+        // first call) and, if stored, Q per level
         size_t free_b = 0, total_b = 0;
         HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
         size_t need_levels = 0, need_q = 0;
@@ -1203,7 +1202,8 @@ int gf_stout_config(gf_ctx* c, int nlev, double rho, int mode) {
             if (!c->lev[l]) need_levels += link_bytes(c);
             if (!c->Qst[l]) need_q += mom_bytes(c);
         }
-        need_levels += (c->G ? 0 : mom_bytes(c)) + (c->Fl ? 0 : mom_bytes(c)) + (c->far ? 0 : 3 * mom_bytes(c));
+        need_levels += (c->G ? 0 : mom_bytes(c)) + (c->Fl ? 0 : mom_bytes(c)) + (c->far ? 0 : 3 * mom_bytes(c)) +
+                       (c->D ? 0 : mat_bytes(c));
         mode = (double)(need_levels + need_q) * 1.1 <= (double)free_b ? GF_STOUT_STORE : GF_STOUT_RECOMPUTE;
     }
     // release the levels' Q of a previous store-mode configuration if no longer needed
@@ -1239,8 +1239,7 @@ int gf_stout_backward(gf_ctx* c, const double* dout_ref, double* din_ref) {
     if (c->nlev == 0) return fail(c, GF_ESTATE, "no stout levels configured");
     if (!dout_ref || !din_ref) return fail(c, GF_EINVAL, "null derivative buffer");
     TRY(alloc(c, &c->D, mat_bytes(c)));
-    TRY(alloc(c, &c->D2, mat_bytes(c)));
-    TRY(upload_linkfield(c, c->D, dout_ref, true));
+    TRY(upload_linkfield(c, c->far, dout_ref, true));
     TRY(stout_backward_all(c));
     return download_linkfield(c, c->D, din_ref, true);
 }

@@ -3,6 +3,8 @@
 Extents: one small lattice (at most 160 groups of 64 sites in FP64, 256 in FP32), whole rows (NX divides 64, V a multiple
 of 64) and rows cut by the groups with idle lanes, above both limits.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -65,3 +67,22 @@ def test_explicit_backward(gf, oracle, dims, precision, nlev, rho):
         L.stout_config(nlev, rho, "recompute")
         L.stout_smear(download=False)
         assert np.abs(L.stout_backward(D) - ref).max() < bar
+
+
+def test_auto_mode_leaves_room_for_back_prop(gf):
+    """11.5 GB free where three levels with Q and the force's buffers take 10.1 GB, without Q 8.5 GB, and the explicit
+    backward pass 1.8 GB more: auto has to choose recompute, and back_prop to work"""
+    dims = (32, 32, 32, 96)
+    with gf.Lattice(dims) as L:
+        hip = ctypes.CDLL("libamdhip64.so.7")  # the one that the library has loaded
+        free, total, filler = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_void_p()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        assert hip.hipMalloc(ctypes.byref(filler), ctypes.c_size_t(free.value - int(11.5e9))) == 0
+        try:
+            L.stout_config(3, 0.1, "auto")
+            assert L.stout_mode() == "recompute"
+            L.stout_smear(download=False)
+            D = L.stout_backward(np.zeros((4, int(np.prod(dims)), 9), complex))
+        finally:
+            assert hip.hipFree(filler) == 0
+    assert not D.any()
