@@ -106,7 +106,7 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
 // (Replaces a gather that evaluated every plaquette once per link, 3258 instead of 1390 x 6/4 FMAs per
 // link and four times the loads, and carried dS/dU and C.)
 // ---------------------------------------------------------------------------
-// FP32: four waves per SIMD at the price of two spilled registers (force with three levels 32^4 2.34 -> 2.32 ms).
+// FP32: four waves per SIMD (force with three levels 32^4 2.34 -> 2.32 ms).
 template <typename T, int ST>
 __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4))) void k_stout_top(
     Geo g, const T* __restrict__ Utop, double coeff, const T* __restrict__ Qst, T* __restrict__ Lc,
@@ -114,13 +114,28 @@ __global__ __launch_bounds__(stencil_threads(ST)) __attribute__((amdgpu_waves_pe
     int s, mu;
     R6<T> own;
     T c[8];
-    if (!ta_force<ST>(g, Utop, s, mu, own, c)) return;
+    __shared__ ForceShare<T, ST, T> sh;
+    if (!ta_force<ST>(g, Utop, s, mu, own, c, sh)) return;
     const unsigned V = g.V;
     T q[8], lam[8], fl[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) c[k] = scale1(coeff, c[k]);
+    // F' waits for its second use in LDS that only this wave still uses: in registers it would spill some, and the
+    // first launch of a spilling kernel on a stream waits 130 us for its private segment (first force of a context, two
+    // levels, 8^4 203 -> 71 us, 16^4 356 -> 229)
+    int lane = (int)(threadIdx.x & 63u);
+    if constexpr (ST == ST_WIDE)
+        put_c8<T>(sh.tp, 0, lane, c);
+    else
+        put_c8<T>(sh.ol, mu, lane, c);
     ldp<T, GF_LD_NT>(Qst, V, mu, s, q);
-    stout_local(q, c, lam, fl);
+    stout_local(q, c, lam, fl, [&](T f[8]) {
+        asm volatile("" : "+v"(lane));
+        if constexpr (ST == ST_WIDE)
+            get_c8(sh.tp, 0, lane, f);
+        else
+            get_c8(sh.ol, mu, lane, f);
+    });
     stp(Lc, V, mu, s, lam);
     stp(Fl, V, mu, s, fl);
 }
@@ -508,8 +523,6 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
                                            int y, const int x[4], int a, int b, int ypa, M3<T>& acc, XLinks<T> ul,
                                            XCoefs<T> hl, int lane, const XRow& xr) {
     const int ypb0 = y + dlt(g, x, b, 1);
-    const int dmb = dlt(g, x, b, -1);
-    const int ymb0 = y + dmb, ypamb0 = ypa + dmb;
     // each group loads its links through its own opaque index copies, so the compiler
     // issues them group by group instead of hoisting all of them
     {  // upper: i X H_a(y+b) U_b(y)^dag + i [S H_b(y) - H_b(y+a) S],  S = X U_b(y)^dag
@@ -539,7 +552,11 @@ __device__ __forceinline__ void back_plane(const Geo& g, const T* __restrict__ U
     }
     {  // lower: U_b(y+a-b)^dag i [U_a(y-b)^dag H_d + H_b(y+a-b) U_a(y-b)^dag] U_b(y-b),
        // H_d = H_a(y-b) - H_b(y-b)
-        int ymb = ymb0, ypamb = ypamb0;
+        // opaque: the offset is formed here, not kept through the upper staple (registers)
+        int xb = sel4(b, x[0], x[1], x[2], x[3]);
+        asm volatile("" : "+v"(xb));
+        const int dmb = (xb == 0 ? sel4(b, g.n[0], g.n[1], g.n[2], g.n[3]) - 1 : -1) * sel4(b, g.st[0], g.st[1], g.st[2], g.st[3]);
+        int ymb = y + dmb, ypamb = ypa + dmb;
         asm volatile("" : "+v"(ymb), "+v"(ypamb));
         Herm<T> hd;
         {
@@ -658,7 +675,7 @@ k_stout_back_stencil(Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T
     }
 }
 template <typename T>
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_stout_back_stencil_wide(
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(2))) void k_stout_back_stencil_wide(
     Geo g, const T* __restrict__ U, const T* __restrict__ Lc, T* __restrict__ Din, double rho) {
     __shared__ T2<T> red[2][9][64];
     const WideIndex wi = wide_index(g);

@@ -22,8 +22,8 @@
 // contracts the planes.  No step goes along t, so both run over blocks of whole t-slices, which bounds the
 // buffer between them (256 MB: 24^3x48 FP64 clover / improved charge 303 / 901 us; 128 MB 316 / 941, 512 MB
 // 324 / 902).  Against walking every loop from x in one kernel, clover / improved charge with the readback: 32^4
-// FP64 533 / 2030 -> 477 / 1398 us, 24^3x48 334 / 1290 -> 303 / 901, 20^3x10 94 / 238 -> 50 / 113, 8^4 37 / 66
-// -> 24 / 33; FP32 links 32^4 562 / 2047 -> 416 / 1367.  At 32^4 k_loops moves links and fields at 4.4 TB/s, the
+// FP64 533 / 2030 -> 474 / 1294 us, 24^3x48 334 / 1290 -> 303 / 834, 20^3x10 94 / 238 -> 49 / 107, 8^4 37 / 66
+// -> 23 / 30; FP32 links 32^4 562 / 2047 -> 403 / 1286.  At 32^4 k_loops moves links and fields at 4.4 TB/s, the
 // rest of its time is the products.
 // Products are evaluated in double for both storage precisions.
 #include <algorithm>
@@ -108,9 +108,10 @@ __device__ __forceinline__ bool same_wave(int i, int j) { return (i >> 6) == (j 
 // One wave per 64 sites of the block [s0, s0 + n), plane and path type (clover and plaquette; rectangles).  The
 // links of a path are loaded one ahead of their use, as in staple_sigma_pipe.  In the planes (0, b) the far
 // site is mostly one of the wave's own (the sites are consecutive along x): its part is then added to the
-// near one there, through LDS, and only what leaves the wave is stored.
+// near one there, through LDS, and only what leaves the wave is stored.  FP32 links hold whole products (Path): two
+// waves per SIMD without spills instead of three with (32^4 improved charge 1309 -> 1286 us).
 template <typename T, int SETS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && (SETS & 4) ? 2 : 3))) void
 k_loops(Geo g, const T* __restrict__ U, int s0, int n, double2* __restrict__ fields) {
     __shared__ C8Lds<double> sh[kBlock / 64], park[(SETS & 4) ? kBlock / 64 : 1];
     constexpr int NT = ((SETS & 3) ? 1 : 0) + ((SETS & 4) ? 1 : 0), FIRST = (SETS & 3) ? 0 : 1;
@@ -125,7 +126,7 @@ k_loops(Geo g, const T* __restrict__ U, int s0, int n, double2* __restrict__ fie
     const unsigned V = g.V;
     int a, b;
     plane_dirs(pl, a, b);
-    const int xa = sel4(a, x[0], x[1], x[2], x[3]), xb = sel4(b, x[0], x[1], x[2], x[3]);
+    int xa = sel4(a, x[0], x[1], x[2], x[3]), xb = sel4(b, x[0], x[1], x[2], x[3]);
     // offset of d steps along a direction (periodic; extents may be smaller than d)
     auto off = [&](int dir, int xd, int d) {
         const int e = g.n[dir];
@@ -216,11 +217,15 @@ k_loops(Geo g, const T* __restrict__ U, int s0, int n, double2* __restrict__ fie
         minus(p.get());
         {
             const M3<double> u = full_of(r6_f64(cur));
-            cur = ld(b, 2, 0);
             ta_coeffs(mul(u, K), near_);
             far_part(mul(K, u), 1, kRect<SETS> + 1);
             put_c8(&park[w], lane, near_);
         }
+        // the second kind's first link and site offsets are not formed before this (spills: 32^4 1375 -> 1294 us, and the
+        // first launch of a spilling kernel on a stream waits 130 us for its private segment)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(xa), "+v"(xb));
+        cur = ld(b, 2, 0);
         GF_STEP(start, ld(a, 1, 1))
         GF_STEP(mul_dag, ld(a, 0, 1))
         GF_STEP(mul_dag, ld(b, 0, 0))

@@ -938,8 +938,8 @@ struct ForceShare<T, ST_WIDE, A> {
 // The workgroup's waves, with the site and U_mu(x) they work on, and TA(U_mu Sigma_mu) in c; false for the
 // waves and lanes that have nothing to store.
 template <int ST, typename T, typename A>
-__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, A c[8]) {
-    __shared__ ForceShare<T, ST, A> sh;
+__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, A c[8],
+                                         ForceShare<T, ST, A>& sh) {
     if constexpr (ST == ST_WIDE) {
         const WideIndex wi = wide_index(g);
         s = wi.s;
@@ -954,6 +954,11 @@ __device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, 
         ta_force_xrow<ST == ST_ROWS>(g, U, (unsigned)g.V, s, x, mu, own, sh.ol, sh.tp, c);
         return in_lattice<ST == ST_ROWS>(g, sm);
     }
+}
+template <int ST, typename T, typename A>
+__device__ __forceinline__ bool ta_force(const Geo& g, const T* __restrict__ U, int& s, int& mu, R6<T>& own, A c[8]) {
+    __shared__ ForceShare<T, ST, A> sh;
+    return ta_force<ST>(g, U, s, mu, own, c, sh);
 }
 
 // block sum of a double into partial[blockIdx.x] (fixed order: deterministic)

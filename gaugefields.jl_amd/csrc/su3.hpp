@@ -906,8 +906,9 @@ __device__ __forceinline__ void exp_dexp(const M3<T>& Q, const M3<T>& X, M3<T>& 
 // a_k = sum_j b_kj tr(X H^j); H commutes with e^-Q, so f1 X + f2 (HX + XH) = i e^-Q (f1 Hf + f2 (H Hf + Hf H)),
 // and the traces follow from tr(H^n Hf), n = 1, 2, by H^3 = c1 H + c0.
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void stout_local(const T q[8], const T f[8], T lam[8], T floc[8]) {
+// f_again(x): f once more, for a caller that keeps it elsewhere than in registers meanwhile
+template <typename T, typename Again>
+__device__ __forceinline__ void stout_local(const T q[8], const T f[8], T lam[8], T floc[8], Again&& f_again) {
     const Herm<T> H = herm_of_coeffs(q), F = herm_of_coeffs(f);
     M3<T> Hm;
 #pragma unroll
@@ -990,8 +991,17 @@ __device__ __forceinline__ void stout_local(const T q[8], const T f[8], T lam[8]
             for (int j = 0; j < 3; j++) Lm.m[3 * i + j] = herm_el(Hl, i, j);
         ta_coeffs(mul_hm(H, Lm), m);
     }
+    T g[8];
+    f_again(g);
 #pragma unroll
-    for (int k = 0; k < 8; k++) floc[k] = fma(T(2), m[k], f[k]);
+    for (int k = 0; k < 8; k++) floc[k] = fma(T(2), m[k], g[k]);
+}
+template <typename T>
+__device__ __forceinline__ void stout_local(const T q[8], const T f[8], T lam[8], T floc[8]) {
+    stout_local(q, f, lam, floc, [&](T g[8]) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) g[k] = f[k];
+    });
 }
 
 // ---------------------------------------------------------------------------
