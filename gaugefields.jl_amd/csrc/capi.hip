@@ -326,27 +326,32 @@ int fstrength_queue(gf_ctx* c, int sets, double* at, double* dens, int dens_meth
     // density: where it has room for most of the usual block (FP64 from 5e5 sites, FP32 from 1e6), the first
     // measurement of a context then allocates nothing (24^3x48 density and energy, first pass 2470 -> 2110 us).  Else
     // they get a buffer of their own (12^4: five blocks in the partner's room would take longer on each call), of
-    // smaller blocks where the device has no room for the usual ones.
+    // smaller blocks where the device has no room for the usual ones, and where it has none the partner's room after all.
     const size_t behind = dens ? ((size_t)c->V + 1) / 2 * 16 : 0;
     void* fields = (char*)c->Ualt + behind;
     size_t room = link_bytes(c) - behind;
     size_t need = field_strength_bytes(c->geo, sets, SIZE_MAX);
     const size_t least = field_strength_bytes(c->geo, sets, 1);
     if (room < std::max(need / 4 * 3, least)) {
-        if (need > c->loops_bytes && !(c->loops_short && c->loops_bytes >= least)) {
+        if (need > c->loops_bytes && !(c->loops_short && std::max(room, c->loops_bytes) >= least)) {
             HIPCHK(c, hipStreamSynchronize(c->stream));
             release(c, &c->loops, c->loops_bytes);
             c->loops_bytes = 0;
             int r;
-            while ((r = alloc(c, &c->loops, need)) != GF_OK && need > least) {
-                need = field_strength_bytes(c->geo, sets, need / 2);
+            while ((r = alloc(c, &c->loops, need)) != GF_OK) {
                 c->loops_short = true;
+                if (need <= least) break;
+                need = field_strength_bytes(c->geo, sets, need / 2);
             }
-            TRY(r);
-            c->loops_bytes = need;
+            if (r == GF_OK)
+                c->loops_bytes = need;
+            else if (room < least)
+                return r;
         }
-        fields = c->loops;
-        room = c->loops_bytes;
+        if (c->loops_bytes > room) {
+            fields = c->loops;
+            room = c->loops_bytes;
+        }
     }
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
