@@ -220,14 +220,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
             // the contribution to the lane of x + 1, through this wave's place in LDS (its lanes in step)
             const int from = s + dlt(g, x, 0, -1);
             put_c8(&near_[2 * p + 1], lane, t);
-            __builtin_amdgcn_wave_barrier();
+            wave_exchange();
             if (ROWS || same_group(from, s)) {
                 T n[8];
                 get_c8(&near_[2 * p + 1], from & 63, n);
 #pragma unroll
                 for (int k = 0; k < 8; k++) c[k] += n[k];
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_exchange();
             store = !ROWS && store && !same_group(fw[0], s);
         }
         if (store) stp<T, GF_ST_NT>(far + (size_t)a * 32 * V, V, b, (unsigned)s, t);

@@ -169,14 +169,14 @@ k_loops(Geo g, const T* __restrict__ U, int s0, int n, double2* __restrict__ fie
         if (a == 0) {
             const int to = i + off(0, xa, d), from = i + off(0, xa, -d);
             put_c8(&sh[w], lane, c);
-            __builtin_amdgcn_wave_barrier();
+            wave_exchange();
             if (same_wave(i, from)) {
                 double t[8];
                 get_c8(&sh[w], from & 63, t);
 #pragma unroll
                 for (int e = 0; e < 8; e++) near_[e] += t[e];
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_exchange();
             store = !same_wave(i, to);
         }
         if (store) st_coeffs(field(k), n, i, c);

@@ -305,11 +305,11 @@ __device__ __forceinline__ void words_in(const double* __restrict__ at, dvec2* s
         const int i = 64 * k + lane;
         if (i < n) sh[i / WORDS * PITCH + i % WORDS] = __builtin_nontemporal_load(p + i);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_exchange();
 }
 template <int WORDS, int PITCH>
 __device__ __forceinline__ void words_out(double* __restrict__ at, const dvec2* sh, int lane, int n) {
-    __builtin_amdgcn_wave_barrier();
+    wave_exchange();
     dvec2* const p = (dvec2*)at;
 #pragma unroll
     for (int k = 0; k < WORDS; k++) {

@@ -421,6 +421,14 @@ __device__ __forceinline__ void ldp(const T* __restrict__ p, unsigned V, int mu,
     }
 }
 
+// Between a wave's own writes to LDS and its reads of what other lanes wrote (or the other way round): the hardware keeps
+// a wave's LDS accesses in order, this keeps the compiler from moving them.
+__device__ __forceinline__ void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The coefficients of a link per lane in LDS as memory holds them: planes of 16 bytes per lane (FP64
 // four pairs, FP32 two quads).  ldp_lds loads them there from memory without passing registers; the
 // wave has to wait_lds_loads() before it reads the place (the compiler does not see the dependence),
