@@ -86,3 +86,39 @@ def test_auto_mode_leaves_room_for_back_prop(gf):
         finally:
             assert hip.hipFree(filler) == 0
     assert not D.any()
+
+
+# Above 512 groups the pair kernel runs with four waves and the gather with whole workgroups: whole rows (640 groups) and
+# rows cut by the groups with idle lanes (552).  The force, and the fused kick and link update of the force's last kernel.
+# FP64: 1e-12; float forces: 2e-6 (plain) and 2e-5 (two levels) of the largest, as on the smaller lattices.  In the
+# FP32-force form the links and momenta are FP64: the update agrees with the oracle's from the same momenta to 1e-13.
+@pytest.mark.parametrize("precision", ["f64", "f32", "f32force"])
+@pytest.mark.parametrize("dims", [(16, 16, 16, 10), (18, 14, 14, 10)])
+@pytest.mark.parametrize("nlev", [0, 2])
+def test_updates_of_larger_lattices(gf, oracle, dims, precision, nlev):
+    print(f"[stout] updates {dims} {precision} {nlev}", flush=True)
+    coeff, rho = 3.0, 0.1
+    bar = 1e-12 if precision == "f64" else (2e-5 if nlev else 2e-6)
+    P = gen.gaussian_momenta(dims, 72)
+    with gf.Lattice(dims, precision=precision) as L:
+        L.upload_links(links(oracle, dims, 71))
+        L.upload_momenta(P)
+        U, P = L.download_links(), L.download_momenta()
+        F = oracle.stout_force(dims, U, nlev, rho, coeff) if nlev else oracle.force(dims, U, coeff)
+        top = np.abs(F).max()
+        for mode in ("store", "recompute") if nlev else ("store",):
+            L.stout_config(nlev, rho, mode)
+            L.upload_links(U)
+            L.upload_momenta(P)
+            L.force(coeff)
+            assert np.abs(L.download_force() - F).max() < bar * top
+            L.force_kick(coeff, 0.02)
+            P1 = P + 0.02 * F
+            assert np.abs(L.download_momenta() - P1).max() < bar * np.abs(P1).max()
+            L.md_update(coeff, 0.03, 0.04)
+            P1 += 0.03 * F
+            got = L.download_momenta()
+            assert np.abs(got - P1).max() < bar * np.abs(P1).max()
+            U1 = U.copy()
+            oracle.exp_update(dims, U1, got, 0.04)
+            assert np.abs(L.download_links() - U1).max() < (2e-6 if precision == "f32" else 1e-13)
