@@ -122,8 +122,6 @@ template <typename T>
 hipError_t launch_set_identity(T* U, int V, hipStream_t st);
 template <typename T>
 hipError_t launch_fill(T* p, size_t n, T v, hipStream_t st);
-template <typename T>
-hipError_t launch_axpby(T* y, const T* x, double a, double b, size_t n, hipStream_t st);
 
 // ---- k_fstrength.hip ----
 // Field strengths of the loop sets in `sets` (bit 0 plaquette, 1 clover, 2 rectangle); out4 =

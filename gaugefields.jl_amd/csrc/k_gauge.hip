@@ -408,11 +408,6 @@ __global__ __launch_bounds__(kBlock) void k_fill(T* __restrict__ p, size_t n, T 
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
 }
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_axpby(T* __restrict__ y, const T* __restrict__ x, T a, T b, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = a * x[i] + b * y[i];
-}
 // The FP32-bulk storage rounding applied to FP64 fields (precision study): rows 0 and 1 of every
 // link, after the double-precision SU(3) projection the FP32 link updates apply when PROJECT,
 // rounded to the nearest float in place; momenta: every coefficient.
@@ -492,10 +487,12 @@ hipError_t launch_plaquette(const Geo& g, const T* U, double* partial, double* o
     const int nb = grid_sites_mu(g.V);
     // the shared form for whole rows in FP64 only: with rows cut by the groups it was slower (24^4: 57 -> 60
     // us), and in FP32 it spilled 16 B at 168 VGPRs (32^4: 0.156 -> 0.171 ms)
-    if (sizeof(T) == 8 && rows_whole(g))
-        k_plaquette_xrow<T><<<nb, kBlock, 0, st>>>(g, U, partial);
-    else
-        k_plaquette<T><<<nb, kBlock, 0, st>>>(g, U, partial);
+    bool shared = false;
+    if constexpr (sizeof(T) == 8) {
+        shared = rows_whole(g);
+        if (shared) k_plaquette_xrow<T><<<nb, kBlock, 0, st>>>(g, U, partial);
+    }
+    if (!shared) k_plaquette<T><<<nb, kBlock, 0, st>>>(g, U, partial);
     return out ? launch_sum_partials(partial, nb, 1, out, st) : hipGetLastError();
 }
 template <typename T>
@@ -591,12 +588,6 @@ hipError_t launch_fill(T* p, size_t n, T v, hipStream_t st) {
     k_fill<T><<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, st>>>(p, n, v);
     return hipGetLastError();
 }
-template <typename T>
-hipError_t launch_axpby(T* y, const T* x, double a, double b, size_t n, hipStream_t st) {
-    if (n == 0) return hipSuccess;
-    k_axpby<T><<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, st>>>(y, x, (T)a, (T)b, n);
-    return hipGetLastError();
-}
 
 #define GF_INST(T)                                                                                       \
     template hipError_t launch_plaquette<T>(const Geo&, const T*, double*, double*, hipStream_t);        \
@@ -611,8 +602,7 @@ hipError_t launch_axpby(T* y, const T* x, double a, double b, size_t n, hipStrea
     template hipError_t launch_momenta_from_ref<T>(const double*, T*, int, int, int, hipStream_t);       \
     template hipError_t launch_momenta_to_ref<T>(const T*, double*, int, int, int, hipStream_t);         \
     template hipError_t launch_set_identity<T>(T*, int, hipStream_t);                                    \
-    template hipError_t launch_fill<T>(T*, size_t, T, hipStream_t);                                      \
-    template hipError_t launch_axpby<T>(T*, const T*, double, double, size_t, hipStream_t);
+    template hipError_t launch_fill<T>(T*, size_t, T, hipStream_t);
 
 GF_INST(double)
 GF_INST(float)
