@@ -747,6 +747,9 @@ hipError_t launch_stout_top(const Geo& g, const T* Utop, double coeff, const T* 
     });
     return hipGetLastError();
 }
+// Six waves a group, one pair each, up to 256 groups, a workgroup per CU; four above.  Kernel, six / four waves, us: FP64 64
+// groups 10.9 / 12.6, 256 12.8 / 13.8, 282 19.9 / 18.6, 384 21.5 / 19.8, 1024 48.0 / 37.0; FP32 64 8.1 / 10.4, 256 9.7 / 12.2,
+// 384 13.5 / 13.6, 512 13.8 / 14.4, 648 16.3 / 16.0, 1024 27.6 / 21.3.
 template <typename T>
 hipError_t launch_stout_pair(const Geo& g, const T* U, const T* Lc, T* Fl, T* far, double rho, hipStream_t st) {
     const int groups = grid_sites_mu(g.V);
@@ -758,6 +761,9 @@ hipError_t launch_stout_pair(const Geo& g, const T* U, const T* Lc, T* Fl, T* fa
     });
     return hipGetLastError();
 }
+// Workgroups of one wave up to 512 groups, of four above.  Kernel, one / four waves, us: FP64 64 groups 4.8 / 5.3, 256 8.5 /
+// 7.8, 384 11.3 / 11.0, 512 11.6 / 12.8, 768 17.8 / 18.2, 1250 25.7 / 26.2; FP32 64 4.8 / 5.2, 256 5.5 / 5.5, 512 10.4 / 9.5, 648
+// 10.8 / 10.8, 1024 14.9 / 16.8, 1250 17.6 / 16.9: it matters below 100 groups only.
 template <typename T>
 hipError_t launch_stout_gather(const Geo& g, const T* far, T* Fl, double rho, const T* Qst, T* Lc, hipStream_t st,
                                int fmode, const T* U, T* FP, double eps_p, T* Unew, double eps_u, double* U64) {
