@@ -24,6 +24,7 @@ namespace gf {
 // Pieces 0 .. total of one call's work; those below `limit` may be claimed, in order, by whoever is running.
 struct Job {
     long total = 0, next = 0, limit = 0, active = 0;
+    bool offered = false;  // to the helpers
     virtual void run(long i) = 0;       // outside the lock
     virtual void ran(long) {}           // inside it
     virtual ~Job() = default;
@@ -79,6 +80,7 @@ class Helpers {
             for (One& o : one_) o.work.notify_one();
         }
         for (; n_ > 0; n_--) pthread_join(one_[n_ - 1].thread, nullptr);
+        std::lock_guard<std::mutex> lk(m_);
         for (One& o : one_) o.called = 0;
         idle_ = 0;
         calling_ = stop_ = false;
@@ -90,6 +92,7 @@ class Helpers {
         for (Job*& p : jobs_)
             if (!p) {
                 p = &j;
+                j.offered = true;
                 break;
             }
         call(j);
@@ -137,7 +140,7 @@ class Helpers {
     static bool claimable(const Job& j) { return j.next < std::min(j.limit, j.total); }
     // a helper, if there is a piece for it and none is on its way
     void call(const Job& j) {
-        if (!claimable(j) || calling_ || idle_ == 0) return;
+        if (!j.offered || !claimable(j) || calling_ || idle_ == 0) return;
         One& o = *idle_at_[--idle_];
         o.called = now();
         calling_ = true;

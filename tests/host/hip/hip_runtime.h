@@ -16,7 +16,7 @@ constexpr unsigned hipHostMallocDefault = 0x0, hipHostMallocCoherent = 0x4000000
 struct Fake {
     std::atomic<long> records{0};
     long fail_wait_of = -1;  // the wait for this record fails
-    unsigned host_flags = ~0u, host_allocs = 0;  // flags that all host allocations had
+    std::atomic<unsigned> host_flags{~0u}, host_allocs{0};  // flags that all host allocations had
 };
 inline Fake fake;
 

@@ -15,9 +15,10 @@
 
 // the clock of all threads but the main one may be made to run ahead
 static const std::thread::id main_thread = std::this_thread::get_id();
-static std::atomic<long> ahead_ns{0};
+static std::atomic<long> ahead_ns{0}, calls{0};  // calls: times read, one for each helper that is called
 static int skewed_clock(clockid_t id, timespec* t) {
     const int r = clock_gettime(id, t);
+    calls++;
     if (std::this_thread::get_id() == main_thread) return r;
     t->tv_nsec += ahead_ns;
     t->tv_sec += t->tv_nsec / 1000000000;
@@ -74,7 +75,7 @@ int coherent() {
     if (wrong_bytes(r, 64, e) || e != hipSuccess) return 1;
     r.free();
     if (fake.host_allocs > 0 && (fake.host_flags & hipHostMallocCoherent)) return 0;
-    return printf("flags %#x\n", fake.host_flags), 1;
+    return printf("flags %#x\n", fake.host_flags.load()), 1;
 }
 
 // pieces of 1 ms that helpers took
@@ -100,6 +101,50 @@ int late_helper() {
     return late == 0 && in_time > 0 ? 0 : (printf("pieces taken late %d, in time %d\n", late, in_time), 1);
 }
 
+// a transfer too small to share calls no helper, also where another context has some waiting
+int small_transfer() {
+    HostRing helped, r;
+    helped.shape(96 * kUnit, 0);
+    r.shape(96 * kUnit, 0);
+    (void)by_helpers(helped);
+    usleep(20000);
+    calls = 0;
+    hipError_t e;
+    const long wrong = wrong_bytes(r, 2, e);
+    r.free();
+    helped.free();
+    return wrong == 0 && calls == 0 ? 0 : (printf("wrong %ld, helpers called %ld\n", wrong, calls.load()), 1);
+}
+// contexts on several threads, helpers started and ended all the while
+int several_threads() {
+    std::atomic<long> wrong{0};
+    std::vector<std::thread> threads;
+    for (int id = 0; id < 4; id++)
+        threads.emplace_back([&wrong, id] {
+            for (int rep = 0; rep < 40; rep++) {
+                HostRing r;
+                r.shape(96 * kUnit * (1 + rep % 3), 0);
+                const long units = (long)(r.slot / kUnit) * (2 + (rep * 7 + id) % 40);
+                std::vector<char> dev(units * kUnit), host(dev.size()), back(dev.size());
+                for (size_t k = 0; k < dev.size(); k += 61) dev[k] = (char)(k * 31 + id + rep);
+                auto off = [](long q) { return (size_t)q * kUnit; };
+                hipError_t e = r.pull(host.data(), units, kUnit, off, [&](long q, long n, char* p) {
+                    return memcpy(p, &dev[q * kUnit], n * kUnit), hipSuccess;
+                }, nullptr);
+                wrong += e != hipSuccess || host != dev;
+                e = r.push(host.data(), units, kUnit, off, [&](long q, long n, const char* p) {
+                    return memcpy(&back[q * kUnit], p, n * kUnit), hipSuccess;
+                }, nullptr);
+                wrong += e != hipSuccess || back != dev;
+                std::vector<int> seen(50, 0);
+                gf::in_parts(r, 50, [&](long k) { seen[k]++; });
+                for (const int n : seen) wrong += n != 1;
+                r.free();
+            }
+        });
+    for (std::thread& t : threads) t.join();
+    return wrong ? printf("%ld wrong\n", wrong.load()), 1 : 0;
+}
 // a signal to the process that the program has blocked stays pending: no helper takes it
 int blocked_signal() {
     HostRing r;
@@ -123,5 +168,7 @@ int main(int argc, char** argv) {
     if (what == "coherent") return coherent();
     if (what == "late_helper") return late_helper();
     if (what == "blocked_signal") return blocked_signal();
+    if (what == "small_transfer") return small_transfer();
+    if (what == "several_threads") return several_threads();
     return printf("no scenario %s\n", what.c_str()), 2;
 }

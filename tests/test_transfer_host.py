@@ -16,7 +16,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["failed_wait", "coherent", "late_helper", "blocked_signal"])
+@pytest.mark.parametrize("scenario", ["failed_wait", "coherent", "late_helper", "blocked_signal",
+                                      "small_transfer", "several_threads"])
 def test_transfer(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
