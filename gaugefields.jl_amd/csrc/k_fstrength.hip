@@ -20,11 +20,11 @@
 // instead of 20, 2a x b rectangles (the double link D = U_a(x) U_a(x+a) in place of U_a, far site x + 2a) 9
 // instead of 20.  k_loops stores near and far coefficients, k_charge adds near(x) and far(x - a) and
 // contracts the planes.  No step goes along t, so both run over blocks of whole t-slices, which bounds the
-// buffer between them (256 MB: 24^3x48 FP64 clover / improved charge 303 / 901 us; 128 MB 316 / 941, 512 MB
-// 324 / 902).  Against walking every loop from x in one kernel, clover / improved charge with the readback: 32^4
+// buffer between them (256 MB: 24^3x48 FP64 clover / improved charge 296 / 821 us; 128 MB 312 / 876, 512 MB
+// 324 / 830; 32^4 475 / 1283, 493 / 1327, 495 / 1286).  Against walking every loop from x in one kernel, clover / improved charge with the readback: 32^4
 // FP64 533 / 2030 -> 474 / 1294 us, 24^3x48 334 / 1290 -> 303 / 834, 20^3x10 94 / 238 -> 49 / 107, 8^4 37 / 66
-// -> 23 / 30; FP32 links 32^4 562 / 2047 -> 403 / 1286.  At 32^4 k_loops moves links and fields at 4.4 TB/s, the
-// rest of its time is the products.
+// -> 23 / 30; FP32 links 32^4 562 / 2047 -> 403 / 1286.  k_loops is bound by the L2 reads of links up to two steps
+// away and by the products.
 // Products are evaluated in double for both storage precisions.
 #include <algorithm>
 

@@ -122,7 +122,7 @@ def test_trajectory_against_fp64_oracle(Lat, oracle, integ, fused):
     assert maxdiff(L.download_links(), Uo) < 1e-5 and maxdiff(L.download_momenta(), Po) < 1e-4
 
 
-# the plain force in its other two stencil forms (LDS-shared pairs, per-thread staples), with the
+# the plain force where NX does not divide 64 and where V is not a multiple of 64, with the
 # FP64 kick and link update of the streaming state kernel
 @pytest.mark.parametrize("dims", [(12, 4, 4, 4), (2, 4, 2, 6)])
 def test_trajectory_other_stencil_forms(Lat, oracle, dims):
@@ -140,8 +140,8 @@ def test_trajectory_other_stencil_forms(Lat, oracle, dims):
     assert maxdiff(L.download_links(), Uo) < 1e-5 and maxdiff(L.download_momenta(), Po) < 1e-4
 
 
-# the three stencil forms of the fused stout epilogue: whole x-rows (4^4), LDS-shared pairs
-# (12,4,4,4), per-thread staples (2,4,2,6: V not a multiple of 64)
+# the stout epilogue with NX that divides 64 (4^4), NX that does not (12,4,4,4), V not a multiple of
+# 64 (2,4,2,6)
 @pytest.mark.parametrize("dims", [D4, (12, 4, 4, 4), (2, 4, 2, 6)])
 def test_stout_trajectory_and_reversibility(Lat, oracle, dims):
     print(f"[f32force] stout trajectory {dims}", flush=True)

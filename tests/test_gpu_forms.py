@@ -31,7 +31,7 @@ def maxdiff(a, b):
 
 
 # FP64: the bar of the other parity tests, relative 1e-12.  FP32: the float forces of float-rounded
-# links, 2e-6 (plain) and 2e-5 (three stout levels) of the largest, as in the FP32 parity tests.
+# links, 2e-6 (plain) and 2e-5 (stout, two levels here) of the largest, as in the FP32 parity tests.
 @pytest.mark.parametrize("precision", ["f64", "f32"])
 @pytest.mark.parametrize("dims", DIMS)
 def test_force_flow_and_stout_forms(gf, oracle, dims, precision):

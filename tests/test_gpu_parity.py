@@ -138,8 +138,8 @@ def test_dsdu_parity(Lat, oracle, dims):
     assert maxdiff(L.dsdu(COEFF), oracle.dsdu(dims, U, COEFF)) < 1e-13 * COEFF * 6
 
 
-# stencil forms: per-thread staples (2,4,2,6: V not a multiple of 64), shared plaquettes
-# (12,4,4,4: NX does not divide 64), x-rows from LDS (the rest; 64,2,2,2: one row per workgroup)
+# lattices of few groups, the planes of a link on the waves of a group: V not a multiple of 64 (2,4,2,6), NX
+# that does not divide 64 (12,4,4,4), whole rows (the rest; 64,2,2,2: one row per group)
 @pytest.mark.parametrize("dims", [D4, (2, 4, 2, 6), (8, 8, 8, 8), (16, 8, 4, 8), (12, 4, 4, 4), (64, 2, 2, 2)])
 def test_force_parity(Lat, oracle, dims):
     L = Lat(dims)
@@ -263,8 +263,8 @@ def test_stout_smear_and_force_parity(Lat, oracle, mode):
     assert rel(H, oracle.stout_potential(D4, U, 3, 0.1, COEFF)) < 1e-12  # momenta are zero
 
 
-# stencil forms of the backward stencil: x-rows from LDS (4^4), the site's own U and Lam from LDS
-# (12,4,4,4: NX does not divide 64), every load from memory (2,4,2,6: V not a multiple of 64)
+# the backward stencil on lattices of few groups, where each site's terms are spread over the waves of a
+# group: NX that divides 64 (4^4), NX that does not (12,4,4,4), V not a multiple of 64 (2,4,2,6)
 # rho 0.12 keeps every exponent's spectral radius below 1 (the series coefficients), rho 0.5 takes
 # part of the links past c1 = 3/4 (the closed form) within the same waves
 @pytest.mark.parametrize("rho", [0.12, 0.5])
@@ -279,8 +279,8 @@ def test_stout_backward_level_parity(Lat, oracle, dims, rho):
     assert maxdiff(L.stout_backward(D), oracle.stout_backward(dims, U, rho, D)) < 1e-13
 
 
-# the fused 2MN sequence: the thin-link backward stencil forms the force and the link update, in
-# the x-row (4^4) and shared (12,4,4,4) stencil forms
+# the 2MN sequence: the thin-link backward stencil forms the force and the link update, with NX that
+# divides 64 (4^4) and that does not (12,4,4,4)
 @pytest.mark.parametrize("dims", [D4, (12, 4, 4, 4)])
 def test_stout_md_parity(Lat, oracle, dims):
     L = Lat(dims)
@@ -313,8 +313,8 @@ def test_fp32_bulk_against_fp64_oracle(Lat, oracle):
     assert abs(H[2] - Href[2]) < 1e-3
 
 
-# FP32 bulk (quad-plane storage) in the three stencil forms: 3-level stout force and stout force
-# + kick + link update (the fused 2MN sequence) against the FP64 oracle on the same float-rounded
+# FP32 bulk (quad-plane storage), NX that divides 64, that does not, and V not a multiple of 64: 3-level
+# stout force and stout force + kick + link update (the 2MN sequence) against the FP64 oracle on the same float-rounded
 # links.  Measured: force 4.7e-6 ... 6.1e-6 of its maximum, dH within 7e-7 ... 3.8e-5; bars 2e-5
 # and 1e-4.
 @pytest.mark.parametrize("dims", [D4, (12, 4, 4, 4), (2, 4, 2, 6)])
