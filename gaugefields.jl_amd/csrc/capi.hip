@@ -46,7 +46,7 @@ struct gf_ctx {
     int smode = GF_STOUT_STORE;
     void* lev[GF_MAX_LEV] = {};  // smeared levels 1..nlev
     void* Qst[GF_MAX_LEV] = {};  // Q coefficients per level (input level index; recompute mode: [0] only)
-    bool q_there = false;        // every level's Q is there and belongs to the levels as they are
+    bool q_there = false;        // every level's Q is there and belongs to the links and levels as they are
     void* G = nullptr;           // Lam of the level being pulled back
     void* Fl = nullptr;          // its derivative without the far plaquette contributions
     void* far = nullptr;         // those (3 momentum fields); explicit backward pass: dS/dU as it comes in
@@ -313,7 +313,16 @@ int plaq_queue(gf_ctx* c, const void* U, double* at) {
     });
 }
 
-void swap_links(gf_ctx* c) { std::swap(c->U, c->Ualt); }
+void swap_links(gf_ctx* c) {
+    std::swap(c->U, c->Ualt);
+    c->q_there = false;
+}
+// the links, to be changed in place
+template <typename T>
+T* links_out(gf_ctx* c) {
+    c->q_there = false;
+    return (T*)c->U;
+}
 
 // field-strength observables of the current links: out = {clover energy sum, Q plaquette,
 // Q clover, Q rectangle}; dens (V doubles, at Ualt) receives the density of dens_method if non-null
@@ -514,7 +523,7 @@ int expupd(gf_ctx* c, double eps) {
     if (c->s64) return state64_step(c, 1, eps);
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_exp_update<T>(c->geo, (const T*)c->U, (T*)c->U, (const T*)c->P, eps, c->stream));
+        HIPCHK(c, launch_exp_update<T>(c->geo, (const T*)c->U, links_out<T>(c), (const T*)c->P, eps, c->stream));
         return GF_OK;
     });
 }
@@ -748,7 +757,7 @@ int gf_set_cold(gf_ctx* c) {
     if (c->s64) HIPCHK(c, launch_set_identity<double>((double*)c->U64, c->V, c->stream));
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_set_identity<T>((T*)c->U, c->V, c->stream));
+        HIPCHK(c, launch_set_identity<T>(links_out<T>(c), c->V, c->stream));
         return GF_OK;
     });
 }
@@ -840,7 +849,7 @@ int gf_upload_links(gf_ctx* c, const double* ref) {
                         "links must be SU(3): at direction %d, site %zu %s by %g (limit %g)",
                         (int)(chk.link / (size_t)c->V) + 1, chk.link % (size_t)c->V, chk.what, chk.worst, kSu3Tol);
     }
-    if (!c->s64) return upload_linkfield(c, c->U, ref);
+    if (!c->s64) return upload_linkfield(c, links_out<void>(c), ref);
     TRY(upload_links_as<double>(c, (double*)c->U64, ref, false));
     TRY(state64_step(c, 3, 0.0));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -913,7 +922,7 @@ int gf_restore_links(gf_ctx* c) {
         return state64_step(c, 3, 0.0);
     }
     if (!c->Ubak) return fail(c, GF_ESTATE, "gf_restore_links before gf_save_links");
-    HIPCHK(c, hipMemcpyAsync(c->U, c->Ubak, link_bytes(c), hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(links_out<void>(c), c->Ubak, link_bytes(c), hipMemcpyDeviceToDevice, c->stream));
     return GF_OK;
 }
 
@@ -1064,7 +1073,7 @@ int gf_hot_start(gf_ctx* c, unsigned long long seed) {
     }
     return dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_hot_links<T>(c->geo, (T*)c->U, seed, c->stream));
+        HIPCHK(c, launch_hot_links<T>(c->geo, links_out<T>(c), seed, c->stream));
         return GF_OK;
     });
 }
@@ -1083,7 +1092,7 @@ static int heatbath_sweep(gf_ctx* c, int mode, double beta, unsigned long long s
     if (mode == 0 && !(beta > 0.0 && std::isfinite(beta))) return fail(c, GF_EINVAL, "beta must be positive; got %g", beta);
     TRY(dispatch(c, [&](auto* tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
-        HIPCHK(c, launch_heatbath<T>(c->geo, (T*)c->U, mode, beta, seed, sweep, itmax, c->partial, c->hres, c->stream));
+        HIPCHK(c, launch_heatbath<T>(c->geo, links_out<T>(c), mode, beta, seed, sweep, itmax, c->partial, c->hres, c->stream));
         return GF_OK;
     }));
     if (mode != 0) return GF_OK;  // overrelaxation always succeeds: nothing to read back
@@ -1175,7 +1184,7 @@ int gf_flow(gf_ctx* c, double eps, int nsteps, int every, double* E_out) {
         TRY(dispatch(c, [&](auto* tag) -> int {
             using T = std::remove_pointer_t<decltype(tag)>;
             HIPCHK(c, launch_flow_stage<T>(c->geo, (const T*)c->U, (T*)c->Ualt, (T*)c->A, -eps / 4.0, 0.0, c->stream));
-            HIPCHK(c, launch_flow_stage<T>(c->geo, (const T*)c->Ualt, (T*)c->U, (T*)c->A, -8.0 * eps / 9.0, -17.0 / 9.0,
+            HIPCHK(c, launch_flow_stage<T>(c->geo, (const T*)c->Ualt, links_out<T>(c), (T*)c->A, -8.0 * eps / 9.0, -17.0 / 9.0,
                                            c->stream));
             HIPCHK(c, launch_flow_stage<T>(c->geo, (const T*)c->U, (T*)c->Ualt, (T*)c->A, -3.0 * eps / 4.0, -1.0,
                                            c->stream));
@@ -1275,7 +1284,7 @@ int gf_round_to_float(gf_ctx* c, int fields) {
     if (c->prec != GF_F64) return fail(c, GF_ESTATE, "rounding to float applies to an FP64 context");
     if (fields & ~(GF_ROUND_LINKS | GF_ROUND_PROJECT | GF_ROUND_MOMENTA))
         return fail(c, GF_EINVAL, "unknown rounding flags 0x%x", fields);
-    HIPCHK(c, launch_round_f32((double*)c->U, (double*)c->P, c->V, (fields & GF_ROUND_LINKS) != 0,
+    HIPCHK(c, launch_round_f32(links_out<double>(c), (double*)c->P, c->V, (fields & GF_ROUND_LINKS) != 0,
                                (fields & GF_ROUND_PROJECT) != 0, (fields & GF_ROUND_MOMENTA) != 0, c->stream));
     return GF_OK;
 }

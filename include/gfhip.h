@@ -187,7 +187,7 @@ int gf_flow_measure(gf_ctx *ctx, double eps, int nsteps, int every, double *out)
  * forces and for gf_stout_backward, GF_STOUT_RECOMPUTE forms it (gf_stout_backward: C_mu) again in the
  * backward pass, GF_STOUT_AUTO stores when the device has room for the nlev momentum-sized fields (plus
  * a 10 % margin) and recomputes otherwise.  gf_stout_backward forms C_mu again in every mode on small
- * lattices, and when other calls have smeared the links since gf_stout_smear.  The smeared levels
+ * lattices, and when other calls have changed or smeared the links since gf_stout_smear.  The smeared levels
  * themselves are always kept.  nlev = 0 disables smearing. */
 int gf_stout_config(gf_ctx *ctx, int nlev, double rho, int mode);
 /* the memory mode in effect after gf_stout_config (GF_STOUT_STORE or GF_STOUT_RECOMPUTE) */

@@ -69,6 +69,47 @@ def test_explicit_backward(gf, oracle, dims, precision, nlev, rho):
         assert np.abs(L.stout_backward(D) - ref).max() < bar
 
 
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_backward_pass_of_links_changed_since_the_smearing(gf, oracle, precision):
+    """One level needs nothing of the smearing but the links it started from: back_prop then belongs to the links as they
+    are, also where Q has been kept from earlier ones"""
+    print(f"[stout] backward of changed links {precision}", flush=True)
+    dims, rho = ROWS, 0.2
+    D = gen.hot_start_links(dims, 43)
+    with gf.Lattice(dims, precision=precision) as L:
+        A, B = links(oracle, dims, 42), links(oracle, dims, 44)
+        L.upload_links(A)
+        L.gaussian_momenta(5)
+        L.save_links()
+        L.stout_config(1, rho, "store")
+        changes = {
+            "upload": lambda: L.upload_links(B),
+            "cold": L.set_cold,
+            "hot": lambda: L.hot_start(3),
+            "links from algebra": lambda: L.links_from_algebra(gen.algebra_coefficients(dims, 0.3, 46)),
+            "exp update": lambda: L.exp_update(0.1),
+            "md update": lambda: L.md_update(3.0, 0.1, 0.1),
+            "trajectory": lambda: L.md_trajectory(3.0, 2, 0.1),
+            "restore": L.restore_links,
+            "heatbath": lambda: L.heatbath(5.5, 1, 2),
+            "overrelaxation": lambda: L.overrelaxation(1, 2),
+            "flow": lambda: L.flow(0.02, 1),
+        }
+        for name, change in changes.items():
+            L.stout_smear(download=False)
+            change()
+            U = L.download_links()
+            ref = oracle.stout_backward(dims, U, rho, D)
+            bar = 1e-13 if precision == "f64" else 2e-5 * np.abs(ref).max()
+            assert np.abs(L.stout_backward(D) - ref).max() < bar, name
+        if precision == "f64":  # links that are SU(3) to float rounding only: as recompute mode does it, which keeps no Q
+            L.stout_smear(download=False)
+            L.round_to_float(links=True)
+            din = L.stout_backward(D)
+            L.stout_config(1, rho, "recompute")
+            assert np.array_equal(din, L.stout_backward(D))
+
+
 def test_auto_mode_leaves_room_for_back_prop(gf):
     """11.5 GB free where three levels with Q and the force's buffers take 10.1 GB, without Q 8.5 GB, and the explicit
     backward pass 1.8 GB more: auto has to choose recompute, and back_prop to work"""
