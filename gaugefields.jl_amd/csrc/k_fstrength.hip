@@ -21,10 +21,10 @@
 // instead of 20.  k_loops stores near and far coefficients, k_charge adds near(x) and far(x - a) and
 // contracts the planes.  No step goes along t, so both run over blocks of whole t-slices, which bounds the
 // buffer between them (256 MB: 24^3x48 FP64 clover / improved charge 296 / 821 us; 128 MB 312 / 876, 512 MB
-// 324 / 830; 32^4 475 / 1283, 493 / 1327, 495 / 1286).  Against walking every loop from x in one kernel, clover / improved charge with the readback: 32^4
-// FP64 533 / 2030 -> 474 / 1294 us, 24^3x48 334 / 1290 -> 303 / 834, 20^3x10 94 / 238 -> 49 / 107, 8^4 37 / 66
-// -> 23 / 30; FP32 links 32^4 562 / 2047 -> 403 / 1286.  k_loops is bound by the L2 reads of links up to two steps
-// away and by the products.
+// 324 / 830; 32^4 475 / 1283, 493 / 1327, 495 / 1286).  Against walking every loop from x in one kernel, clover /
+// improved charge with the readback: 32^4 FP64 533 / 2030 -> 475 / 1283 us, 24^3x48 334 / 1290 -> 296 / 821, 20^3x10
+// 94 / 238 -> 49 / 107, 8^4 37 / 66 -> 23 / 30; FP32 links 32^4 562 / 2047 -> 403 / 1286.  k_loops is bound by the L2
+// reads of links up to two steps away and by the products.
 // Products are evaluated in double for both storage precisions.
 #include <algorithm>
 
